@@ -49,6 +49,7 @@ struct LloydWorkspace {
   bool store_flush = false;
   int mixed_terms = 0;     // BF16 split terms (1 or 3) or 8 (FP8) of the mixed path, 0: FP32
   bool tiled = false;      // tiled path: centroids streamed, separate update
+  bool wide = false;       // features streamed, separate update (d > 128)
   int blocks_b = 0;        // partial slots of the FP32 re-score (mixed path)
   // LDS-resident mixed path: the re-score restricted to candidate tiles,
   // from the sample-major copy xr, and the queue's separate exact update
@@ -325,15 +326,21 @@ static std::unique_ptr<LloydWorkspace<T, I>> make_workspace(int64_t n,
     return ws;
   }
   FusedPlan p = plan_generic_fused<T>(n, d, k);
-  if (p.priv)
+  // features streamed through the matrix core: the same sums into the same
+  // copies as the generic kernel's atomics
+  const bool wide = std::is_same<T, float>::value && wide_supported(n, d, k) &&
+                    label_sums_supported(k);
+  if (p.priv && !wide)
     return std::make_unique<LloydWorkspace<T, I>>(
         n, d, k, p.blocks, false, true, p, sizeof(T) * (size_t)p.blocks * d * k,
         sizeof(T) * (size_t)p.blocks * k, s);
-  // sums too large for LDS: global atomics into a few zeroed copies
+  // sums too large for LDS: atomics into a few zeroed copies
   const int copies = 8;
-  return std::make_unique<LloydWorkspace<T, I>>(
+  auto ws = std::make_unique<LloydWorkspace<T, I>>(
       n, d, k, copies, false, false, p, sizeof(T) * (size_t)copies * d * k,
       sizeof(T) * (size_t)copies * k, s);
+  ws->wide = wide;
+  return ws;
 }
 
 // Optional timing of the fused-step kernel with HIP events on the driver's
@@ -564,7 +571,17 @@ static void lloyd_front(LloydWorkspace<T, I> &ws, const T *X, const T *w,
   }
   if (n > 0) {
     timer.begin(s);
-    launch_fused_generic<T, I>(n, d, k, ws.blocks, ws.plan, ws.store_flush, X,
+    if constexpr (std::is_same<T, float>::value) {
+      if (ws.wide) {
+        launch_wide_assign<I>(n, d, k, X, cur, ws.hn.template as<const T>(), labels, s,
+                              skip);
+        launch_label_sums<I>(n, d, k, ws.blocks, X, w, cur, labels,
+                             ws.copies.template as<T>(),
+                             ws.sizes_copies.template as<T>(), s, skip);
+      }
+    }
+    if (!ws.wide)
+      launch_fused_generic<T, I>(n, d, k, ws.blocks, ws.plan, ws.store_flush, X,
                                w, cur, ws.hn.template as<const T>(), labels,
                                ws.copies.template as<T>(),
                                ws.sizes_copies.template as<T>(), s);

@@ -90,4 +90,48 @@ __device__ inline void fixed_point_scales_from_bits(
   flag[0] = bad ? 1 : (coarse ? 2 : 0);
 }
 
+// Exact binade-window sums (for the steps that run no pass over X for
+// scales).  A finite FP32 value v = m 2^(e - 150) (m the
+// 24-bit significand, e the biased exponent) whose binade e lies in
+// [lo, lo + W] is the integer m << (e - lo) in units of 2^(lo - 150), with
+// no rounding: those values go into the block's int64 LDS sums exactly
+// (|m << W| < 2^(24 + W) leaves 2^(39 - W) additions of headroom).  Values
+// outside the window (zeros aside), infinities and NaNs are added straight
+// into the caller's copy with an FP32 atomic, as the reference adds every
+// value.  lo is set per feature so that the window ends kWinMargin binades
+// above the largest centroid coordinate of that feature: samples lie near
+// their centroids, so nearly every value falls inside.
+constexpr int kWinMargin = 4;
+constexpr int kWinTopW = 20;   // weights: window up to 2^20
+
+__device__ inline void window_add(unsigned long long *sum, float *fallback, int64_t off,
+                                  float v, int lo, int W) {
+  const unsigned b = __float_as_uint(v);
+  const int sh = (int)((b >> 23) & 0xffu) - lo;
+  if ((unsigned)sh <= (unsigned)W) {
+    const unsigned long long m =
+        (unsigned long long)((b & 0x7fffffu) | 0x800000u) << sh;
+    atomicAdd(sum + off, (b >> 31) ? 0ull - m : m);
+  } else if (v != 0.f) {
+    atomicAdd(fallback + off, v);
+  }
+}
+
+// Width W of the window when one block adds at most `count` values into one
+// sum: 2^(24 + W) count < 2^63.
+inline int window_width(int64_t count) {
+  int bits = 0;
+  while (bits < 40 && (int64_t(1) << bits) < count) ++bits;
+  const int w = 38 - bits;
+  return w < 1 ? 1 : w > 30 ? 30 : w;
+}
+
+// Lowest binade of the window whose largest value's binade is `e` (a
+// centroid coordinate's, for a feature) and whose margin is `margin`.
+__device__ inline int window_low(int e, int margin, int W) {
+  const int top = e + margin;
+  const int lo = top > W + 1 ? top : W + 1;
+  return (lo < 254 ? lo : 254) - W;
+}
+
 }  // namespace kmd

@@ -215,7 +215,18 @@ void launch_fused_step_copies(int64_t n, int64_t d, int64_t k,
     // tiles streamed through LDS, then the update from those labels
     if (tiled_supported(d, k)) {
       launch_tiled_assign<I>(n, d, k, X, C, hn, labels, s, nullptr, scratch);
-      launch_label_update<I>(n, d, k, n_copies, X, w, labels, copies, sizes_copies, s);
+      // the exact window sums where one row of them fits LDS
+      if (label_sums_supported(k))
+        launch_label_sums<I>(n, d, k, n_copies, X, w, C, labels, copies, sizes_copies, s);
+      else
+        launch_label_update<I>(n, d, k, n_copies, X, w, labels, copies, sizes_copies, s);
+      return;
+    }
+    // more than 128 features: the labels with the features streamed (no
+    // scratch), the same sums
+    if (wide_supported(n, d, k) && label_sums_supported(k)) {
+      launch_wide_assign<I>(n, d, k, X, C, hn, labels, s);
+      launch_label_sums<I>(n, d, k, n_copies, X, w, C, labels, copies, sizes_copies, s);
       return;
     }
   }
@@ -237,6 +248,10 @@ void launch_assignment(int64_t n, int64_t d, int64_t k, int64_t h,
   if constexpr (std::is_same<T, float>::value) {
     if (tiled_supported(d, k)) {
       launch_tiled_assign<I>(n, d, k, X, C, hn, labels, s);
+      return;
+    }
+    if (wide_supported(n, d, k)) {
+      launch_wide_assign<I>(n, d, k, X, C, hn, labels, s);
       return;
     }
   } else {

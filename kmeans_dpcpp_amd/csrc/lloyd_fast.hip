@@ -99,33 +99,6 @@ __device__ inline void load_x(const float *__restrict__ X, int64_t n, int d,
   }
 }
 
-// Exact binade-window sums (the reference-API fused step, which runs no
-// pass over X for scales).  A finite FP32 value v = m 2^(e - 150) (m the
-// 24-bit significand, e the biased exponent) whose binade e lies in
-// [lo, lo + W] is the integer m << (e - lo) in units of 2^(lo - 150), with
-// no rounding: those values go into the block's int64 LDS sums exactly
-// (|m << W| < 2^(24 + W) leaves 2^(39 - W) additions of headroom).  Values
-// outside the window (zeros aside), infinities and NaNs are added straight
-// into the caller's copy with an FP32 atomic, as the reference adds every
-// value.  lo is set per feature so that the window ends kWinMargin binades
-// above the largest centroid coordinate of that feature: samples lie near
-// their centroids, so nearly every value falls inside.
-constexpr int kWinMargin = 4;
-constexpr int kWinTopW = 20;   // weights: window up to 2^20
-
-__device__ inline void window_add(u64 *sum, float *fallback, int64_t off,
-                                  float v, int lo, int W) {
-  const unsigned b = __float_as_uint(v);
-  const int sh = (int)((b >> 23) & 0xffu) - lo;
-  if ((unsigned)sh <= (unsigned)W) {
-    const u64 m = (u64)((b & 0x7fffffu) | 0x800000u) << sh;
-    atomicAdd(sum + off, (b >> 31) ? (u64)0 - m : m);
-  } else if (v != 0.f) {
-    atomic_add(fallback + off, v);
-  }
-}
-
-
 // Launch parameters shared by the kernel variants.
 struct FastArgs {
   int64_t n;
@@ -236,8 +209,8 @@ __global__ void __launch_bounds__(NT) mfma_lloyd_krn(FastArgs a) {
     }
     __syncthreads();
     for (int f = tid; f <= d; f += NT) {
-      const int top = f < d ? Ew[f] + kWinMargin : 127 + kWinTopW;
-      Ew[f] = min(max(top, a.window + 1), 254) - a.window;
+      Ew[f] = f < d ? window_low(Ew[f], kWinMargin, a.window)
+                    : window_low(127, kWinTopW, a.window);
     }
     __syncthreads();
   }
@@ -678,8 +651,7 @@ __global__ void __launch_bounds__((smallk_threads<DB, G>()))
     }
     __syncthreads();
     for (int f = tid; f <= DB; f += NT) {
-      const int top = f < d ? Ew[f] + kWinMargin : 127 + kWinTopW;
-      Ew[f] = min(max(top, W + 1), 254) - W;
+      Ew[f] = f < d ? window_low(Ew[f], kWinMargin, W) : window_low(127, kWinTopW, W);
     }
     __syncthreads();
   }
@@ -1293,8 +1265,7 @@ void launch_fast_fused(int64_t n, int64_t d, int64_t k, int64_t n_copies,
     a.vec = vec_ok(X, n, L.s) ? 1 : 0;
     a.scale = nullptr;
     a.nonfinite = nullptr;
-    // window width from the most samples one block adds into one sum:
-    // 2^(24 + W) * count < 2^63
+    // window width from the most samples one block adds into one sum
     int64_t per_block =
         ceil_div<int64_t>(ceil_div<int64_t>(n, 32 * L.s), L.blocks) * 32 * L.s;
     if (L.smallk) {
@@ -1303,9 +1274,7 @@ void launch_fast_fused(int64_t n, int64_t d, int64_t k, int64_t n_copies,
       per_block = ceil_div<int64_t>(ceil_div<int64_t>(n, kWave), L.blocks * waves) *
                   waves * kWave;
     }
-    int bits = 0;
-    while (bits < 40 && (int64_t(1) << bits) < per_block) ++bits;
-    a.window = std::max(1, std::min(30, 38 - bits));
+    a.window = window_width(per_block);
     a.copies = copies;
     a.sizes_copies = sizes_copies;
     a.n_copies = n_copies;

@@ -259,6 +259,23 @@ void launch_tiled_update(int64_t n, int64_t d, int64_t k, const float *X_r,
                          void *scratch, void *sums, hipStream_t s,
                          const int *skip = nullptr);
 
+// ---- float32 beyond the tiled kernels (lloyd_wide.hip) ----------------------
+// Labels with the features streamed (any d and k; no working memory).
+bool wide_supported(int64_t n, int64_t d, int64_t k);
+template <typename I>
+void launch_wide_assign(int64_t n, int64_t d, int64_t k, const float *X_t,
+                        const float *C, const float *hn, I *labels,
+                        hipStream_t s, const int *skip = nullptr);
+// The fused step's accumulate-into update from given labels: exact window
+// sums per block (windows set from the centroids C), the blocks' totals added
+// into the copies with FP32 atomics.
+bool label_sums_supported(int64_t k);
+template <typename I>
+void launch_label_sums(int64_t n, int64_t d, int64_t k, int64_t n_copies,
+                       const float *X_t, const float *w, const float *C,
+                       const I *labels, float *copies, float *sizes_copies,
+                       hipStream_t s, const int *skip = nullptr);
+
 // ---- batched fits (batched.hip) -------------------------------------------
 struct BatchedFit {
   int64_t n, d, k;
