@@ -45,6 +45,26 @@ void allow_full_lds(const void *kernel) {
   done.push_back(kernel);
 }
 
+int blocks_per_cu(const void *kernel, int threads, size_t lds_bytes) {
+  struct Known {
+    const void *kernel;
+    size_t lds;
+    int device, threads, blocks;
+  };
+  static thread_local std::vector<Known> known;
+  int dev = 0;
+  KMD_HIP_CHECK(hipGetDevice(&dev));
+  for (const Known &q : known)
+    if (q.kernel == kernel && q.lds == lds_bytes && q.threads == threads && q.device == dev)
+      return q.blocks;
+  int blocks = 0;
+  KMD_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, threads,
+                                                             lds_bytes));
+  if (known.size() >= 256) known.clear();
+  known.push_back(Known{kernel, lds_bytes, dev, threads, blocks});
+  return blocks;
+}
+
 int64_t device_l2_bytes(int device) {
   int bytes = 0;
   KMD_HIP_CHECK(

@@ -75,6 +75,11 @@ inline int apply_blocks_cap(int per_cu) {
   return (cap > 0 && per_cu > cap) ? cap : per_cu;
 }
 
+// Blocks of `kernel` that one CU holds with this block size and dynamic LDS
+// (hipOccupancyMaxActiveBlocksPerMultiprocessor, asked once per thread,
+// device and launch shape: it costs microseconds, as much as a launch).
+int blocks_per_cu(const void *kernel, int threads, size_t lds_bytes);
+
 // Stream-ordered temporary device buffer (hipMallocAsync / hipFreeAsync).
 // Freed in stream order when the object is destroyed, so work enqueued on the
 // same stream before destruction may still use it.
@@ -165,25 +170,67 @@ template <typename T, typename I>
 void launch_reduce_centroids(int64_t n_copies, int64_t d, int64_t k,
                              const T *sizes_copies, const T *cent_copies,
                              T *out_sizes, T *out_cent, I *empty_list,
-                             I *n_empty, int64_t list_len, hipStream_t s,
-                             bool from_zero = false);
+                             I *n_empty, int64_t list_len, hipStream_t s);
+// The same sums without the list (skip as in the step kernels).
+template <typename T>
+void launch_sum_copies(int64_t n_copies, int64_t d, int64_t k, const T *sizes_copies,
+                       const T *cent_copies, T *out_sizes, T *out_cent, hipStream_t s,
+                       const int *skip);
 template <typename T>
 void launch_centroid_shifts(int64_t d, int64_t k, const T *old_c,
                             const T *new_c, T *out, hipStream_t s);
 template <typename T, typename I>
 void launch_inertia(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
                     const T *C, const I *labels, T *out, hipStream_t s);
-// End of a Lloyd iteration in one launch: next /= sizes (per column), shifts
-// against cur, FP64 sum of the shifts into out_sum[0], half squared norms of
-// the new centroids into hn_next (when not null); skipped entirely while
-// gate[0] != 0 (gate may be null).  partials: finalize_step_blocks(k) doubles;
-// ticket: one zero-initialised counter (left at zero).
-int finalize_step_blocks(int64_t k);
+// State of a fit's loop, on the device and (published at the end of every
+// iteration) in pinned host memory.  The kernels of an iteration return at
+// once while stop != 0, so iterations can be enqueued ahead of the host's
+// knowledge of how the one before ended.
+constexpr int kLoopConverged = 1, kLoopEmpty = 2;
+struct LoopState {
+  int stop;            // 0, kLoopConverged or kLoopEmpty
+  int pad;
+  long long done;      // iterations finished
+  long long n_empty;   // kLoopEmpty: clusters to relocate
+  double shift;        // sum of the squared shifts of the last iteration
+  long long rescored;  // samples re-scored so far (mixed precision)
+};
+struct LoopHost {
+  unsigned long long word;   // done * 4 + stop
+  long long n_empty;         // valid when the word says kLoopEmpty
+};
+
+// Writes the state to host memory, the word after the rest (which only a loop
+// with clusters to relocate has).
+__device__ inline void publish(LoopHost *h, const LoopState &st) {
+  if (st.stop == kLoopEmpty) {
+    h->n_empty = st.n_empty;
+    __threadfence_system();
+  }
+  __hip_atomic_store(&h->word, (unsigned long long)st.done * 4 + st.stop, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// End of a Lloyd iteration in one launch (util.hip): the empty-cluster list,
+// or the new centroids, their shifts and half norms, the loop's state.
 template <typename T, typename I>
-void launch_finalize_step(int64_t d, int64_t k, const I *gate, const T *sizes,
-                          const T *cur, T *next, T *shifts, T *hn_next,
-                          double *partials, unsigned *ticket, double *out_sum,
-                          hipStream_t s);
+struct StepTail {
+  int64_t d, k;
+  const T *sums, *sizes, *cur;   // undivided sums (d, k), sizes (k), old centroids
+  T *next, *shifts, *hn;
+  I *list;                       // k + 1 entries
+  LoopState *state;
+  LoopHost *host;
+  const int *rescored;           // this iteration's re-scored samples, or null
+  T tol;
+  int relocated;                 // the sums after a relocation: no list, not
+                                 // counted as another iteration
+  double *partials;              // step_tail_partials(k) doubles
+  unsigned *ticket;              // one zero counter (left at zero)
+};
+int64_t step_tail_partials(int64_t k);
+template <typename T, typename I>
+void launch_step_tail(const StepTail<T, I> &a, hipStream_t s);
 template <typename T>
 void launch_reduce_sum(int64_t n, const T *data, double *dev_result,
                        hipStream_t s);

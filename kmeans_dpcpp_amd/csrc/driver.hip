@@ -11,28 +11,30 @@
 // and is overwritten.
 //
 // Differences (all on the host side, none in results):
-//  * the host is off the GPU's critical path: the division, shifts and
-//    shift sum run in one kernel that skips itself when the iteration found
-//    empty clusters, so a whole iteration is enqueued without a host
-//    decision, and iteration i + 1 is enqueued before iteration i's scalars
-//    {shift sum, empty count} are read back (one wait per iteration, on an
-//    event, while the GPU runs the next iteration).  The work enqueued ahead
-//    is discarded when the fit stops, or redone after a relocation; the
-//    centroid buffers rotate over three (init, res, a scratch one) so it
-//    never overwrites centroids still needed;
+//  * the host is off the GPU's critical path: an iteration is three launches
+//    (step, reduction, tail), enqueued without a host decision.  The tail
+//    kernel keeps the loop's state on the device (finished iterations, and
+//    whether the loop converged or found empty clusters) and publishes it in
+//    pinned host memory; the kernels of an iteration return at once when the
+//    loop has stopped, so a few iterations are enqueued ahead and cost next
+//    to nothing when they were not needed.  The host reads the state from
+//    memory between launches; it relocates empty clusters and enqueues the
+//    iterations after that again;
 //  * private copies are one per block of the persistent fused kernel and are
 //    written with plain stores, so the sums are deterministic;
-//  * the relocation path reuses the labels of the fused step (kept per
-//    iteration parity) instead of recomputing them from the same centroids
-//    and half-norms (src/kmeans_lloyd_driver.hpp:226-250);
+//  * the relocation path reuses the labels of the fused step instead of
+//    recomputing them from the same centroids and half-norms
+//    (src/kmeans_lloyd_driver.hpp:226-250);
 //  * the verbose line reports the inertia of the centroids that produced the
 //    labels (the reference evaluates it against the undivided sums).
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <sstream>
+#include <thread>
 #include <tuple>
 #include <vector>
 
@@ -65,34 +67,36 @@ struct LloydWorkspace {
   TempBuffer qmask{0, nullptr}, cand{0, nullptr};  // tiled BF16: candidate tiles
   TempBuffer xb{0, nullptr}, xnb{0, nullptr};  // tiled BF16 (T = 1): BF16 samples
   int64_t seg_cap = 0;     // capacity of each block's re-score queue segment
-  // Two iterations can be in flight (the next one is enqueued before this
-  // one's scalars are read back): cluster sizes, the empty list and the
-  // scalars {shift sum @0, n_empty @8, re-scored count @16} have one slot per
-  // iteration parity `par`.  cbuf: the third centroid buffer of the rotation.
-  int par = 0;
-  TempBuffer cbuf, fin_part, fin_ticket;
+  // `sums`: the undivided sums of the iteration (kept until the next one's
+  // reduction, for the relocation of empty clusters); `scalars`: the loop's
+  // state @0, an iteration's re-scored count @48, the epilogue's sum @56
+  TempBuffer sums, tail_part, tail_ticket;
   // copies_bytes / sizes_bytes: private copies of the generic kernel, or the
   // fast path's per-block partials (in `copies`, sizes_bytes = 0)
   LloydWorkspace(int64_t n_, int64_t d_, int64_t k_, int blocks_, bool fast_,
                  bool store_, const FusedPlan &plan_, size_t copies_bytes,
                  size_t sizes_bytes, hipStream_t s)
       : n(n_), d(d_), k(k_), blocks(blocks_), fast(fast_), store_flush(store_),
-        plan(plan_), hn(sizeof(T) * k_, s), sizes(2 * sizeof(T) * k_, s),
+        plan(plan_), hn(sizeof(T) * k_, s), sizes(sizeof(T) * k_, s),
         shifts(sizeof(T) * k_, s), per_sample(sizeof(T) * (n_ > 0 ? n_ : 1), s),
         copies(copies_bytes, s), sizes_copies(sizes_bytes, s),
-        list(2 * sizeof(I) * (k_ + 1), s), scalars(64, s),
+        list(sizeof(I) * (k_ + 1), s), scalars(64, s),
         scales(fast_ ? sizeof(float) * (d_ + 1) + 16 : 0, s),
-        cbuf(sizeof(T) * d_ * k_, s),
-        fin_part(sizeof(double) * finalize_step_blocks(k_), s),
-        fin_ticket(sizeof(unsigned), s) {
-    KMD_HIP_CHECK(hipMemsetAsync(fin_ticket.as<unsigned>(), 0, sizeof(unsigned), s));
+        sums(sizeof(T) * d_ * k_, s),
+        tail_part(sizeof(double) * step_tail_partials(k_), s),
+        tail_ticket(sizeof(unsigned), s) {
+    KMD_HIP_CHECK(hipMemsetAsync(tail_ticket.as<unsigned>(), 0, sizeof(unsigned), s));
+    KMD_HIP_CHECK(hipMemsetAsync(scalars.as<char>(), 0, scalars.bytes(), s));
   }
-  T *sizes_p() const { return sizes.as<T>() + par * k; }
-  I *list_p() const { return list.as<I>() + par * (k + 1); }
-  char *scalars_p() const { return scalars.as<char>() + 32 * par; }
-  I *n_empty() const { return reinterpret_cast<I *>(scalars_p() + 8); }
-  int *queue_count() const { return reinterpret_cast<int *>(scalars_p() + 16); }
-  double *shift_sum() const { return reinterpret_cast<double *>(scalars_p()); }
+  LoopState *state() const { return scalars.as<LoopState>(); }
+  const int *stop() const { return &state()->stop; }
+  int *queue_count() const {
+    static_assert(sizeof(LoopState) <= 48, "layout of scalars");
+    return reinterpret_cast<int *>(scalars.as<char>() + 48);
+  }
+  double *epilogue_sum() const {
+    return reinterpret_cast<double *>(scalars.as<char>() + 56);
+  }
   float *scale() const { return scales.as<float>(); }
   int *nonfinite() const {
     return reinterpret_cast<int *>(scales.as<char>() + sizeof(float) * (d + 1));
@@ -343,26 +347,30 @@ static std::unique_ptr<LloydWorkspace<T, I>> make_workspace(int64_t n,
   return ws;
 }
 
+// Iterations enqueued ahead of the last one known to have finished.  Enough
+// to cover the launches of the next ones on the smallest shapes, few enough
+// that what is left to skip when the loop stops costs little.
+constexpr int kAhead = 3;
+
 // Optional timing of the fused-step kernel with HIP events on the driver's
-// stream: one event pair per iteration parity (two iterations can be in
-// flight), read back once that iteration is known to have finished.
+// stream: one event pair per iteration that can be in flight, read back once
+// that iteration is known to have finished.
 struct FusedTimer {
   bool on = false;
-  hipEvent_t start[2] = {nullptr, nullptr}, stop[2] = {nullptr, nullptr};
-  bool pending[2] = {false, false};
+  hipEvent_t start[kAhead + 1] = {}, stop[kAhead + 1] = {};
   int slot = 0;
   double total_ms = 0.0;
   int64_t launches = 0;
   explicit FusedTimer(bool enable) : on(enable) {
     if (on) {
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i <= kAhead; ++i) {
         KMD_HIP_CHECK(hipEventCreate(&start[i]));
         KMD_HIP_CHECK(hipEventCreate(&stop[i]));
       }
     }
   }
   ~FusedTimer() {
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i <= kAhead; ++i) {
       if (start[i]) (void)hipEventDestroy(start[i]);
       if (stop[i]) (void)hipEventDestroy(stop[i]);
     }
@@ -371,30 +379,22 @@ struct FusedTimer {
     if (on) KMD_HIP_CHECK(hipEventRecord(start[slot], s));
   }
   void end(hipStream_t s) {
-    if (!on) return;
-    KMD_HIP_CHECK(hipEventRecord(stop[slot], s));
-    pending[slot] = true;
+    if (on) KMD_HIP_CHECK(hipEventRecord(stop[slot], s));
   }
-  // call once the work timed in slot i has finished
+  // the launch timed in slot i has finished
   void collect(int i) {
-    if (!on || !pending[i]) return;
+    if (!on) return;
     float ms = 0.f;
+    KMD_HIP_CHECK(hipEventSynchronize(stop[i]));
     KMD_HIP_CHECK(hipEventElapsedTime(&ms, start[i], stop[i]));
     total_ms += ms;
     ++launches;
-    pending[i] = false;
   }
-  void collect_all() {
-    collect(0);
-    collect(1);
-  }
-  void discard(int i) { pending[i] = false; }
 };
 
-// Pinned host slots for the per-iteration scalars (32 bytes per parity), so
-// their device-to-host copies are asynchronous.  Pinning and unpinning cost
-// hundreds of microseconds, so the 64-byte blocks are kept in a process-wide
-// free list and reused (one per driver call running at a time).
+// Pinned host memory for the loop's published state (LoopHost).  Pinning and
+// unpinning cost hundreds of microseconds, so the 64-byte blocks are kept in
+// a process-wide free list and reused (one per driver call running at a time).
 std::mutex g_pinned_mu;
 std::vector<char *> g_pinned_free;
 
@@ -419,22 +419,45 @@ struct PinnedScalars {
   }
   PinnedScalars(const PinnedScalars &) = delete;
   PinnedScalars &operator=(const PinnedScalars &) = delete;
-  char *slot(int i) const { return p + 32 * i; }
+  LoopHost *host() const { return reinterpret_cast<LoopHost *>(p); }
+};
+static_assert(sizeof(LoopHost) <= 64, "one pinned block holds the state");
+
+// Leaves no kernel behind that may still write the pinned block when the
+// driver is left by an exception.
+struct DrainOnThrow {
+  hipStream_t s;
+  int entered = std::uncaught_exceptions();
+  ~DrainOnThrow() {
+    if (std::uncaught_exceptions() > entered) (void)hipStreamSynchronize(s);
+  }
 };
 
-struct IterEvents {
-  hipEvent_t e[2] = {nullptr, nullptr};
-  IterEvents() {
-    for (int i = 0; i < 2; ++i)
-      KMD_HIP_CHECK(hipEventCreateWithFlags(&e[i], hipEventDisableTiming));
+// Waits until `host` shows more than `done` finished iterations or a stopped
+// loop; its word.  A device error ends the wait.
+inline unsigned long long wait_loop(const LoopHost *host, long long done, hipStream_t s) {
+  auto word = [&] { return __atomic_load_n(&host->word, __ATOMIC_ACQUIRE); };
+  auto ended = [&](unsigned long long w) {
+    return (long long)(w >> 2) > done || (w & 3) != 0;
+  };
+  for (int spins = 1;; ++spins) {
+    unsigned long long w = word();
+    if (ended(w)) return w;
+    if (spins % 4096 == 0) {
+      const hipError_t e = hipStreamQuery(s);
+      if (e == hipSuccess) {   // all done: the word must be there
+        w = word();
+        if (ended(w)) return w;
+        throw RuntimeError("Lloyd loop: an iteration left no state");
+      }
+      if (e != hipErrorNotReady) KMD_HIP_CHECK(e);
+      (void)hipGetLastError();   // "not ready" is no error of a later launch
+      std::this_thread::yield();
+    } else {
+      __builtin_ia32_pause();
+    }
   }
-  ~IterEvents() {
-    for (int i = 0; i < 2; ++i)
-      if (e[i]) (void)hipEventDestroy(e[i]);
-  }
-  IterEvents(const IterEvents &) = delete;
-  IterEvents &operator=(const IterEvents &) = delete;
-};
+}
 
 // LDS-resident mixed path: BF16 step (operands already prepared for `cur`)
 // and the re-score of its undecided samples, in the workspace's form:
@@ -465,7 +488,7 @@ static void mixed_labels_and_partials(LloydWorkspace<T, I> &ws, const T *X,
           labels, ws.queue.template as<const int>(),
           ws.queue_counts.template as<const int>(),
           ws.qmask.template as<const unsigned>(), ws.blocks, ws.seg_cap,
-          ws.cand.template as<void>(), ws.queue_count(), s);
+          ws.cand.template as<void>(), ws.queue_count(), s, skip);
       launch_queue_update<I>(d, k, ws.blocks_b, ws.blocks, ws.seg_cap,
                              ws.queue.template as<const int>(),
                              ws.queue_counts.template as<const int>(),
@@ -478,7 +501,7 @@ static void mixed_labels_and_partials(LloydWorkspace<T, I> &ws, const T *X,
                              ws.copies.template as<void>(), ws.blocks,
                              ws.queue.template as<const int>(),
                              ws.queue_counts.template as<const int>(),
-                             ws.blocks, ws.seg_cap, ws.queue_count(), s);
+                             ws.blocks, ws.seg_cap, ws.queue_count(), s, skip);
     }
   } else {
     (void)ws, (void)X, (void)w, (void)cur, (void)labels, (void)s, (void)skip;
@@ -486,15 +509,19 @@ static void mixed_labels_and_partials(LloydWorkspace<T, I> &ws, const T *X,
   }
 }
 
-// hn (unless the previous iteration's finalize computed it), fused step and
-// reduction for centroids `cur`, sums into `next`; the empty count is
-// written, not accumulated.
+// Fused step and reduction for centroids `cur` (half norms in ws.hn):
+// undivided sums into ws.sums, cluster sizes into ws.sizes.
 template <typename T, typename I>
 static void lloyd_front(LloydWorkspace<T, I> &ws, const T *X, const T *w,
-                        const T *cur, T *next, I *labels, hipStream_t s,
-                        FusedTimer &timer, bool hn_ready, const int *skip) {
+                        const T *cur, I *labels, hipStream_t s, FusedTimer &timer) {
   const int64_t n = ws.n, d = ws.d, k = ws.k;
-  if (!hn_ready) launch_half_l2_norm<T>(d, k, cur, ws.hn.template as<T>(), s);
+  const int *skip = ws.stop();
+  T *sums = ws.sums.template as<T>();
+  T *sizes = ws.sizes.template as<T>();
+  auto reduce_fixed = [&](int64_t slots) {
+    launch_sum_fixed_partials<T>(slots, d, k, ws.copies.template as<const void>(),
+                                 ws.scale(), ws.nonfinite(), sizes, sums, s, skip);
+  };
   if constexpr (std::is_same<T, float>::value) {
     if (ws.tiled) {
       const float *xr = ws.xr.template as<const float>();
@@ -519,12 +546,12 @@ static void lloyd_front(LloydWorkspace<T, I> &ws, const T *X, const T *w,
               ws.queue.template as<const int>(),
               ws.queue_counts.template as<const int>(),
               ws.qmask.template as<const unsigned>(), ws.blocks_b, ws.seg_cap,
-              ws.cand.template as<void>(), ws.queue_count(), s);
+              ws.cand.template as<void>(), ws.queue_count(), s, skip);
         else
           launch_tiled_rescore<I>(n, d, k, xr, cur, ws.hn.template as<const T>(),
                                   labels, ws.queue.template as<const int>(),
                                   ws.queue_counts.template as<const int>(),
-                                  ws.blocks_b, ws.seg_cap, ws.queue_count(), s);
+                                  ws.blocks_b, ws.seg_cap, ws.queue_count(), s, skip);
       } else {
         launch_tiled_assign<I>(n, d, k, X, cur, ws.hn.template as<const T>(),
                                labels, s, skip);
@@ -533,9 +560,7 @@ static void lloyd_front(LloydWorkspace<T, I> &ws, const T *X, const T *w,
                              ws.upd.template as<void>(),
                              ws.copies.template as<void>(), s, skip);
       timer.end(s);
-      launch_reduce_fixed_partials<T, I>(
-          1, d, k, ws.copies.template as<const void>(), ws.scale(),
-          ws.nonfinite(), ws.sizes_p(), next, ws.list_p(), ws.n_empty(), k, s, true);
+      reduce_fixed(1);
       return;
     }
     if (ws.mixed_terms > 0) {
@@ -545,9 +570,7 @@ static void lloyd_front(LloydWorkspace<T, I> &ws, const T *X, const T *w,
       timer.begin(s);
       mixed_labels_and_partials(ws, X, w, cur, labels, s, skip);
       timer.end(s);
-      launch_reduce_fixed_partials<T, I>(
-          ws.blocks + ws.blocks_b, d, k, ws.copies.template as<const void>(),
-          ws.scale(), ws.nonfinite(), ws.sizes_p(), next, ws.list_p(), ws.n_empty(), k, s, true);
+      reduce_fixed(ws.blocks + ws.blocks_b);
       return;
     }
   }
@@ -558,9 +581,7 @@ static void lloyd_front(LloydWorkspace<T, I> &ws, const T *X, const T *w,
                                   ws.scale(), ws.nonfinite(),
                                   ws.copies.template as<void>(), ws.blocks, s, skip);
     timer.end(s);
-    launch_reduce_fixed_partials<T, I>(
-        ws.blocks, d, k, ws.copies.template as<const void>(), ws.scale(),
-        ws.nonfinite(), ws.sizes_p(), next, ws.list_p(), ws.n_empty(), k, s, true);
+    reduce_fixed(ws.blocks);
     return;
   }
   if (!ws.store_flush || n == 0) {
@@ -569,29 +590,24 @@ static void lloyd_front(LloydWorkspace<T, I> &ws, const T *X, const T *w,
     KMD_HIP_CHECK(hipMemsetAsync(ws.sizes_copies.template as<T>(), 0,
                                  ws.sizes_copies.bytes(), s));
   }
-  if (n > 0) {
-    timer.begin(s);
-    if constexpr (std::is_same<T, float>::value) {
-      if (ws.wide) {
-        launch_wide_assign<I>(n, d, k, X, cur, ws.hn.template as<const T>(), labels, s,
-                              skip);
-        launch_label_sums<I>(n, d, k, ws.blocks, X, w, cur, labels,
-                             ws.copies.template as<T>(),
-                             ws.sizes_copies.template as<T>(), s, skip);
-      }
+  timer.begin(s);
+  if constexpr (std::is_same<T, float>::value) {
+    if (ws.wide) {
+      launch_wide_assign<I>(n, d, k, X, cur, ws.hn.template as<const T>(), labels, s,
+                            skip);
+      launch_label_sums<I>(n, d, k, ws.blocks, X, w, cur, labels,
+                           ws.copies.template as<T>(),
+                           ws.sizes_copies.template as<T>(), s, skip);
     }
-    if (!ws.wide)
-      launch_fused_generic<T, I>(n, d, k, ws.blocks, ws.plan, ws.store_flush, X,
+  }
+  if (!ws.wide)
+    launch_fused_generic<T, I>(n, d, k, ws.blocks, ws.plan, ws.store_flush, X,
                                w, cur, ws.hn.template as<const T>(), labels,
                                ws.copies.template as<T>(),
-                               ws.sizes_copies.template as<T>(), s);
-    timer.end(s);
-  }
-  launch_reduce_centroids<T, I>(ws.blocks, d, k,
-                                ws.sizes_copies.template as<const T>(),
-                                ws.copies.template as<const T>(),
-                                ws.sizes_p(), next, ws.list_p(), ws.n_empty(),
-                                k, s, true);
+                               ws.sizes_copies.template as<T>(), s, skip);
+  timer.end(s);
+  launch_sum_copies<T>(ws.blocks, d, k, ws.sizes_copies.template as<const T>(),
+                       ws.copies.template as<const T>(), sizes, sums, s, skip);
 }
 
 template <typename T, typename I>
@@ -686,79 +702,54 @@ static void driver_impl(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
   auto ws_ptr = make_workspace<T, I>(n, d, k, X, w, precision, s);
   FusedTimer timer(stats != nullptr);
   auto &ws = *ws_ptr;
-  // centroid buffers rotate init -> res -> cbuf: iteration i reads
-  // bufs[i % 3] and writes bufs[(i + 1) % 3], so an iteration enqueued ahead
-  // never writes the centroids the one before it read
-  T *bufs[3] = {init, res, ws.cbuf.template as<T>()};
+  // centroid buffers: iteration i reads bufs[i % 2] and writes the other one
+  // (when it finds empty clusters: only ws.sums)
+  T *bufs[2] = {init, res};
   const T tol_t = static_cast<T>(tol);
-  int64_t it = 0;
-  T shift = std::numeric_limits<T>::infinity();
-  int64_t rescored = 0;
-  PinnedScalars host;
-  IterEvents ev;
-  // labels of odd iterations go to a second buffer, so the relocation of
-  // iteration i still has its labels when iteration i + 1 was enqueued ahead
-  // (the epilogue writes the caller's labels)
-  TempBuffer lab2(sizeof(I) * (size_t)(n > 0 ? n : 1), s);
-  // valid (zero) labels from the start: kernels of an iteration whose main
-  // kernel skipped itself may still read them as cluster indices
-  KMD_HIP_CHECK(hipMemsetAsync(lab2.as<I>(), 0, lab2.bytes(), s));
-  I *labs[2] = {labels, lab2.as<I>()};
-  // one iteration: front half, then (unless it found empty clusters) the
-  // division, shifts, their sum and the next half-norms; its scalars go to
-  // host slot `par`
-  auto enqueue_iter = [&](int64_t i) {
-    ws.par = (int)(i & 1);
-    timer.slot = ws.par;
-    T *cur = bufs[i % 3];
-    T *next = bufs[(i + 1) % 3];
-    // the previous iteration's empty count: when it found empty clusters,
-    // this iteration's main kernel returns at once (it will be redone)
-    const int *skip =
-        i > 0 ? reinterpret_cast<const int *>(ws.scalars.template as<char>() +
-                                              32 * (ws.par ^ 1) + 8)
-              : nullptr;
-    lloyd_front<T, I>(ws, X, w, cur, next, labs[ws.par], s, timer, i > 0, skip);
-    launch_finalize_step<T, I>(d, k, ws.n_empty(), ws.sizes_p(), cur, next,
-                               ws.shifts.template as<T>(),
-                               ws.hn.template as<T>(),
-                               ws.fin_part.template as<double>(),
-                               ws.fin_ticket.template as<unsigned>(),
-                               ws.shift_sum(), s);
-    KMD_HIP_CHECK(hipMemcpyAsync(host.slot(ws.par), ws.scalars_p(), 32,
-                                 hipMemcpyDeviceToHost, s));
-    KMD_HIP_CHECK(hipEventRecord(ev.e[ws.par], s));
+  int64_t it = 0;         // iterations known to have finished
+  int64_t queued = 0;     // iterations enqueued
+  PinnedScalars pinned;
+  DrainOnThrow drain{s};
+  LoopHost *host = pinned.host();
+  // no iteration at all where the sum of shifts could not exceed tol
+  if (!(std::numeric_limits<T>::infinity() > tol_t)) max_iter = 0;
+  StepTail<T, I> tail{};
+  tail.d = d;
+  tail.k = k;
+  tail.sums = ws.sums.template as<const T>();
+  tail.sizes = ws.sizes.template as<const T>();
+  tail.shifts = ws.shifts.template as<T>();
+  tail.hn = ws.hn.template as<T>();
+  tail.list = ws.list.template as<I>();
+  tail.state = ws.state();
+  tail.host = host;
+  tail.rescored = ws.mixed_terms > 0 ? ws.queue_count() : nullptr;
+  tail.tol = tol_t;
+  tail.partials = ws.tail_part.template as<double>();
+  tail.ticket = ws.tail_ticket.template as<unsigned>();
+  auto enqueue_tail = [&](int64_t i, bool relocated) {
+    tail.cur = bufs[i % 2];
+    tail.next = bufs[(i + 1) % 2];
+    tail.relocated = relocated ? 1 : 0;
+    launch_step_tail<T, I>(tail, s);
   };
-
-  // Iteration it + 1 is enqueued before iteration it's scalars are read
-  // (not in verbose mode, which prints between iterations).  It is discarded
-  // when the fit stops after iteration it (it wrote only the rotation's third
-  // buffer, labels and scratch, all rewritten before use), or when iteration
-  // it found empty clusters (then it is enqueued again after the relocation).
-  const bool ahead = !verbose;
-  if (max_iter > 0) enqueue_iter(0);
-  while (it < max_iter && shift > tol_t) {
-    bool next_queued = false;
-    if (ahead && it + 1 < max_iter) {
-      enqueue_iter(it + 1);
-      next_queued = true;
+  launch_half_l2_norm<T>(d, k, init, ws.hn.template as<T>(), s);
+  // verbose mode prints between iterations: nothing is enqueued ahead there
+  const int ahead = verbose ? 0 : kAhead;
+  while (it < max_iter) {
+    while (queued < max_iter && queued <= it + ahead) {
+      timer.slot = (int)(queued % (kAhead + 1));
+      lloyd_front<T, I>(ws, X, w, bufs[queued % 2], labels, s, timer);
+      enqueue_tail(queued, false);
+      ++queued;
     }
-    const int p = (int)(it & 1);
-    KMD_HIP_CHECK(hipEventSynchronize(ev.e[p]));
-    timer.collect(p);
-    I ne;
-    std::memcpy(&ne, host.slot(p) + 8, sizeof(I));
-    const int64_t n_empty = (int64_t)ne;
-    if (ws.mixed_terms > 0) {
-      int qc;
-      std::memcpy(&qc, host.slot(p) + 16, sizeof(int));
-      rescored += qc;
-    }
-    T *cur = bufs[it % 3];
-    T *next = bufs[(it + 1) % 3];
-    I *lab = labs[p];
+    const unsigned long long word = wait_loop(host, it, s);
+    const int64_t done = (int64_t)(word >> 2);
+    int stop = (int)(word & 3);
+    for (; it < done; ++it) timer.collect((int)(it % (kAhead + 1)));
+    T *cur = bufs[(it + 1) % 2];   // of iteration it - 1, the last finished
     if (verbose) {
-      launch_inertia<T, I>(n, d, k, X, w, cur, lab,
+      launch_inertia<T, I>(n, d, k, X, w, cur, labels,
                            ws.per_sample.template as<T>(), s);
       double tot = 0.0;
       TempBuffer dres(sizeof(double), s);
@@ -768,57 +759,34 @@ static void driver_impl(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
                                    hipMemcpyDeviceToHost, s));
       KMD_HIP_CHECK(hipStreamSynchronize(s));
       std::ostringstream ss;
-      ss << "Iteration: " << it << " Inertia: " << static_cast<T>(tot);
+      ss << "Iteration: " << it - 1 << " Inertia: " << static_cast<T>(tot);
       if (print_fn) print_fn(ss.str().c_str(), print_user);
     }
-    if (n_empty > 0) {
-      // the division was skipped; the iteration enqueued ahead (if any) ran
-      // on undivided sums and is redone below
-      KMD_HIP_CHECK(hipStreamSynchronize(s));
-      timer.discard(p ^ 1);  // a skipped launch, when one was enqueued
-      ws.par = p;
+    if (stop == kLoopEmpty) {
       // squared distance to the nearest centroid (unit weights), then move
-      // the farthest samples into the empty clusters
-      launch_inertia<T, I>(n, d, k, X, nullptr, cur, lab,
+      // the farthest samples into the empty clusters, on the undivided sums;
+      // the iterations enqueued ahead skip themselves
+      launch_inertia<T, I>(n, d, k, X, nullptr, cur, labels,
                            ws.per_sample.template as<T>(), s);
-      launch_relocate<T, I>(n, d, k, n_empty, X, w, lab, ws.list_p(),
-                            ws.per_sample.template as<const T>(), next,
-                            ws.sizes_p(), ws.per_sample.template as<T>(), s);
-      // the redone next iteration must not take itself for one to skip
-      KMD_HIP_CHECK(hipMemsetAsync(ws.n_empty(), 0, sizeof(I), s));
-      launch_finalize_step<T, I>(d, k, static_cast<const I *>(nullptr),
-                                 ws.sizes_p(), cur, next,
-                                 ws.shifts.template as<T>(),
-                                 ws.hn.template as<T>(),
-                                 ws.fin_part.template as<double>(),
-                                 ws.fin_ticket.template as<unsigned>(),
-                                 ws.shift_sum(), s);
-      KMD_HIP_CHECK(hipMemcpyAsync(host.slot(p), ws.scalars_p(), 32,
-                                   hipMemcpyDeviceToHost, s));
-      KMD_HIP_CHECK(hipEventRecord(ev.e[p], s));
-      KMD_HIP_CHECK(hipEventSynchronize(ev.e[p]));
-      next_queued = false;
+      launch_relocate<T, I>(n, d, k, host->n_empty, X, w, labels,
+                            ws.list.template as<const I>(),
+                            ws.per_sample.template as<const T>(),
+                            ws.sums.template as<T>(), ws.sizes.template as<T>(),
+                            ws.per_sample.template as<T>(), s);
+      enqueue_tail(it - 1, true);
+      KMD_HIP_CHECK(hipStreamSynchronize(s));
+      queued = it;
+      stop = (int)(host->word & 3);
     }
-    double sh;
-    std::memcpy(&sh, host.slot(p), sizeof(double));
-    shift = static_cast<T>(sh);
-    ++it;
-    if (it < max_iter && shift > tol_t && !next_queued) enqueue_iter(it);
+    if (stop == kLoopConverged) break;
   }
-  T *cur = bufs[it % 3];
-  ws.par = 0;
-  auto read_sum = [&]() -> double {
-    double v = 0.0;
-    KMD_HIP_CHECK(hipMemcpyAsync(&v, ws.shift_sum(), sizeof(double),
-                                 hipMemcpyDeviceToHost, s));
-    KMD_HIP_CHECK(hipStreamSynchronize(s));
-    return v;
-  };
+  // ws.hn holds the half norms of the final centroids: the last tail's, or
+  // (no iteration) those of init
+  T *cur = bufs[it % 2];
 
   // epilogue: labels and weighted inertia of the final centroids (on the
   // tiled mixed path with its BF16 kernel and exact re-score: the FP32
   // labels)
-  launch_half_l2_norm<T>(d, k, cur, ws.hn.template as<T>(), s);
   bool labelled = false;
   if constexpr (std::is_same<T, float>::value) {
     if (ws.tiled && ws.mixed_terms > 0 && n > 0) {
@@ -867,9 +835,16 @@ static void driver_impl(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
     KMD_HIP_CHECK(hipMemcpyAsync(res, cur, sizeof(T) * d * k,
                                  hipMemcpyDeviceToDevice, s));
   launch_reduce_sum<T>(n, ws.per_sample.template as<const T>(),
-                       ws.shift_sum(), s);
-  *inertia_out = static_cast<double>(static_cast<T>(read_sum()));
-  timer.collect_all();
+                       ws.epilogue_sum(), s);
+  char end[64];   // the loop's state and the epilogue's sum
+  KMD_HIP_CHECK(hipMemcpyAsync(end, ws.scalars.template as<char>(), sizeof(end),
+                               hipMemcpyDeviceToHost, s));
+  KMD_HIP_CHECK(hipStreamSynchronize(s));
+  LoopState final_state;
+  std::memcpy(&final_state, end, sizeof(final_state));
+  double total;
+  std::memcpy(&total, end + 56, sizeof(total));
+  *inertia_out = static_cast<double>(static_cast<T>(total));
   *n_iters_out = it;
   if (stats) {
     stats->fused_kernel_ms = timer.total_ms;
@@ -879,7 +854,7 @@ static void driver_impl(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
     if (ws.tiled) path += 3;  // 4 tiled FP32, 5 tiled BF16, 6 tiled BF16x3
     if (ws.tiled && ws.mixed_terms == 8) path = 7;  // tiled FP8
     stats->fused_path = path;
-    stats->n_rescored = rescored;
+    stats->n_rescored = final_state.rescored;
   }
 }
 

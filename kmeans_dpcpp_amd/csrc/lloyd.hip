@@ -38,7 +38,9 @@ __global__ void __launch_bounds__(kBlock)
                    const T *__restrict__ hn, I *__restrict__ labels,
                    T *__restrict__ copies, T *__restrict__ sizes_copies,
                    int64_t n_copies, int priv, int store_flush,
-                   T *__restrict__ D) {
+                   T *__restrict__ D, const int *skip = nullptr) {
+  // an iteration enqueued ahead of the loop's end: nothing to compute
+  if (skip != nullptr && *skip != 0) return;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *cwin = reinterpret_cast<T *>(smem_raw);  // [kH][kKW]
   T *hnw = cwin + kH * kKW;                   // [kKW]
@@ -173,19 +175,20 @@ template <typename T, typename I>
 void launch_fused_generic(int64_t n, int64_t d, int64_t k, int64_t n_copies,
                           const FusedPlan &p, bool store_flush, const T *X,
                           const T *w, const T *C, const T *hn, I *labels,
-                          T *copies, T *sizes_copies, hipStream_t s) {
+                          T *copies, T *sizes_copies, hipStream_t s,
+                          const int *skip) {
   if (n == 0) return;
   if constexpr (std::is_same<T, double>::value) {
     if (fast64_supported(d, k, true)) {
       launch_fast64_fused<I>(n, d, k, n_copies, p, store_flush, X, w, C, hn, labels,
-                             copies, sizes_copies, s);
+                             copies, sizes_copies, s, skip);
       return;
     }
   }
   hipLaunchKernelGGL((lloyd_tile_krn<T, I, MODE_FUSED>), dim3(p.blocks),
                      dim3(kBlock), p.lds_bytes, s, n, (int)d, (int)k, X, w, C,
                      hn, labels, copies, sizes_copies, n_copies, (int)p.priv,
-                     (int)store_flush, (T *)nullptr);
+                     (int)store_flush, (T *)nullptr, skip);
   KMD_LAUNCH_CHECK();
 }
 
@@ -264,7 +267,7 @@ void launch_assignment(int64_t n, int64_t d, int64_t k, int64_t h,
   hipLaunchKernelGGL((lloyd_tile_krn<T, I, MODE_ASSIGN>), dim3(blocks),
                      dim3(kBlock), window_lds_bytes<T>(), s, n, (int)d, (int)k,
                      X, (const T *)nullptr, C, hn, labels, (T *)nullptr,
-                     (T *)nullptr, (int64_t)1, 0, 0, (T *)nullptr);
+                     (T *)nullptr, (int64_t)1, 0, 0, (T *)nullptr, (const int *)nullptr);
   KMD_LAUNCH_CHECK();
 }
 
@@ -278,14 +281,15 @@ void launch_distances(int64_t n, int64_t d, int64_t k, int64_t h, const T *X,
                      dim3(kBlock), window_lds_bytes<T>(), s, n, (int)d, (int)k,
                      X, (const T *)nullptr, C, (const T *)nullptr,
                      (int32_t *)nullptr, (T *)nullptr, (T *)nullptr,
-                     (int64_t)1, 0, 0, D);
+                     (int64_t)1, 0, 0, D, (const int *)nullptr);
   KMD_LAUNCH_CHECK();
 }
 
 #define KMD_INST_LLOYD(T, I)                                                   \
   template void launch_fused_generic<T, I>(                                    \
       int64_t, int64_t, int64_t, int64_t, const FusedPlan &, bool, const T *,  \
-      const T *, const T *, const T *, I *, T *, T *, hipStream_t);            \
+      const T *, const T *, const T *, I *, T *, T *, hipStream_t,             \
+      const int *);                                                            \
   template void launch_fused_step_copies<T, I>(                                \
       int64_t, int64_t, int64_t, int64_t, int64_t, const T *, const T *,       \
       const T *, const T *, I *, T *, T *, hipStream_t, void *);               \

@@ -54,6 +54,7 @@ struct F64Args {
   double *sizes;              // [n_copies][k]
   int64_t n_copies;
   int store_flush;            // 1: write slot blockIdx.x; 0: atomics into copies
+  const int *skip;            // when non-null and *skip != 0 the launch does nothing
 };
 
 size_t lds64_bytes(int ks4, int64_t d, int64_t k, bool update) {
@@ -64,6 +65,8 @@ size_t lds64_bytes(int ks4, int64_t d, int64_t k, bool update) {
 
 template <int KS4, typename I, bool UPDATE>
 __global__ void __launch_bounds__(kNT64) mfma64_lloyd_krn(F64Args a) {
+  // an iteration enqueued ahead of the loop's end: nothing to compute
+  if (a.skip != nullptr && *a.skip != 0) return;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   constexpr int kWaves = kNT64 / 64;
   const int d = a.d, k = a.k, kpad = a.kpad;
@@ -224,7 +227,7 @@ template <typename I, bool UPDATE>
 void launch64(int64_t n, int64_t d, int64_t k, int blocks, const double *X,
               const double *w, const double *C, const double *hn, I *labels,
               double *copies, double *sizes, int64_t n_copies, bool store_flush,
-              hipStream_t s) {
+              hipStream_t s, const int *skip = nullptr) {
   const int ks4 = ks4_bucket(d);
   F64Args a{};
   a.n = n;
@@ -240,6 +243,7 @@ void launch64(int64_t n, int64_t d, int64_t k, int blocks, const double *X,
   a.sizes = sizes;
   a.n_copies = std::max<int64_t>(1, n_copies);
   a.store_flush = store_flush ? 1 : 0;
+  a.skip = skip;
   Kern64 fn = pick64<I, UPDATE>(ks4);
   hipLaunchKernelGGL(fn, dim3(blocks), dim3(kNT64), lds64_bytes(ks4, d, k, UPDATE), s,
                      a);
@@ -267,10 +271,10 @@ void launch_fast64_fused(int64_t n, int64_t d, int64_t k, int64_t n_copies,
                          const FusedPlan &p, bool store_flush, const double *X,
                          const double *w, const double *C, const double *hn,
                          I *labels, double *copies, double *sizes_copies,
-                         hipStream_t s) {
+                         hipStream_t s, const int *skip) {
   if (n <= 0) return;
   launch64<I, true>(n, d, k, p.blocks, X, w, C, hn, labels, copies, sizes_copies,
-                    n_copies, store_flush, s);
+                    n_copies, store_flush, s, skip);
 }
 
 template <typename I>
@@ -287,12 +291,12 @@ template void launch_fast64_fused<int32_t>(int64_t, int64_t, int64_t, int64_t,
                                            const FusedPlan &, bool, const double *,
                                            const double *, const double *,
                                            const double *, int32_t *, double *,
-                                           double *, hipStream_t);
+                                           double *, hipStream_t, const int *);
 template void launch_fast64_fused<int64_t>(int64_t, int64_t, int64_t, int64_t,
                                            const FusedPlan &, bool, const double *,
                                            const double *, const double *,
                                            const double *, int64_t *, double *,
-                                           double *, hipStream_t);
+                                           double *, hipStream_t, const int *);
 template void launch_fast64_assign<int32_t>(int64_t, int64_t, int64_t, const double *,
                                             const double *, const double *, int32_t *,
                                             hipStream_t);

@@ -926,11 +926,17 @@ inline size_t lds_bytes(int64_t d, int64_t k, bool update, int copies = 1) {
   return b;
 }
 
-// Copies of the LDS sums the fused step keeps (up to 8, as LDS allows: the
-// kernel runs one block per CU).
-inline int sum_copies(int64_t d, int64_t k) {
+// Copies of the LDS sums the fused step keeps: up to 8, as LDS allows (the
+// kernel runs one block per CU), and one per 256 samples of a block.  Every
+// copy is cleared and added up once per block, which pays only where enough
+// samples meet in it (n = 50,000, d = 14, k = 127, 512 samples per block:
+// 11.3 us with 8 copies, 10.7 us with 2).
+inline int sum_copies(int64_t n, int64_t d, int64_t k) {
+  const int64_t per_block =
+      ceil_div<int64_t>(n, std::min<int64_t>(device_cu_count(), ceil_div<int64_t>(n, 512)));
   int r = 1;
-  while (r < 8 && lds_bytes(d, k, true, 2 * r) <= kLdsPerCu) r *= 2;
+  while (r < 8 && 2 * r * 256 <= per_block && lds_bytes(d, k, true, 2 * r) <= kLdsPerCu)
+    r *= 2;
   return r;
 }
 
@@ -1071,10 +1077,8 @@ MfmaLaunch plan_smallk(int64_t n, int64_t d, int64_t k) {
   L.fn = pick_smallk<I, UPDATE, WINDOW>(d, k);
   if (L.fn == nullptr) return L;
   allow_full_lds(reinterpret_cast<const void *>(L.fn));
-  int per_cu = 0;
-  KMD_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &per_cu, reinterpret_cast<const void *>(L.fn), L.threads, L.lds));
-  per_cu = apply_blocks_cap(per_cu);
+  const int per_cu = apply_blocks_cap(
+      blocks_per_cu(reinterpret_cast<const void *>(L.fn), L.threads, L.lds));
   if (per_cu < 1) {
     L.fn = nullptr;
     return L;
@@ -1098,7 +1102,7 @@ MfmaLaunch plan_launch(int64_t n, int64_t d, int64_t k) {
     if (L.fn != nullptr) return L;
     L = MfmaLaunch{};
   }
-  L.copies = UPDATE ? sum_copies(d, k) : 1;
+  L.copies = UPDATE ? sum_copies(n > 0 ? n : 1, d, k) : 1;
   L.lds = lds_bytes(d, k, UPDATE, L.copies);
   if (L.lds > kLdsPerCu) return L;
   int shape = (UPDATE && STORE) ? tuned_shape() : 0;
@@ -1120,10 +1124,8 @@ MfmaLaunch plan_launch(int64_t n, int64_t d, int64_t k) {
         break;
       }
   }
-  int per_cu = 0;
-  KMD_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &per_cu, reinterpret_cast<const void *>(L.fn), L.threads, L.lds));
-  per_cu = apply_blocks_cap(per_cu);
+  const int per_cu = apply_blocks_cap(
+      blocks_per_cu(reinterpret_cast<const void *>(L.fn), L.threads, L.lds));
   if (per_cu < 1) {
     L.fn = nullptr;
     return L;
@@ -1334,10 +1336,8 @@ MfmaLaunch plan_rescore(int64_t d, int64_t k) {
   L.fn = pick_rescore<I>(d);
   if (L.fn == nullptr) return L;
   allow_full_lds(reinterpret_cast<const void *>(L.fn));
-  int per_cu = 0;
-  KMD_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &per_cu, reinterpret_cast<const void *>(L.fn), L.threads, L.lds));
-  per_cu = apply_blocks_cap(per_cu);
+  const int per_cu = apply_blocks_cap(
+      blocks_per_cu(reinterpret_cast<const void *>(L.fn), L.threads, L.lds));
   if (per_cu < 1) {
     L.fn = nullptr;
     return L;
@@ -1360,7 +1360,8 @@ void launch_fast_rescore(int64_t n, int64_t d, int64_t k, const float *X,
                          I *labels, const float *scale, const int *nonfinite,
                          void *partials, int64_t slot0, const int *queue,
                          const int *queue_counts, int n_segments,
-                         int64_t seg_cap, int *n_rescored, hipStream_t s) {
+                         int64_t seg_cap, int *n_rescored, hipStream_t s,
+                         const int *skip) {
   const MfmaLaunch L = plan_rescore<I>(d, k);
   if (L.fn == nullptr) throw RuntimeError("FP32 re-score: no launch plan");
   if (n_segments < 1 || n_segments > kMaxSegments)
@@ -1377,6 +1378,7 @@ void launch_fast_rescore(int64_t n, int64_t d, int64_t k, const float *X,
   a.n_segments = n_segments;
   a.seg_cap = seg_cap;
   a.n_rescored = n_rescored;
+  a.skip = skip;
   run(L, a, s);
 }
 
@@ -1388,14 +1390,16 @@ template void launch_fast_rescore<int32_t>(int64_t, int64_t, int64_t,
                                            int32_t *, const float *,
                                            const int *, void *, int64_t,
                                            const int *, const int *, int,
-                                           int64_t, int *, hipStream_t);
+                                           int64_t, int *, hipStream_t,
+                                           const int *);
 template void launch_fast_rescore<int64_t>(int64_t, int64_t, int64_t,
                                            const float *, const float *,
                                            const float *, const float *,
                                            int64_t *, const float *,
                                            const int *, void *, int64_t,
                                            const int *, const int *, int,
-                                           int64_t, int *, hipStream_t);
+                                           int64_t, int *, hipStream_t,
+                                           const int *);
 template int fast_fused_blocks<int32_t>(int64_t, int64_t, int64_t);
 template int fast_fused_blocks<int64_t>(int64_t, int64_t, int64_t);
 template bool fast_fused_supported<float>(int64_t, int64_t);

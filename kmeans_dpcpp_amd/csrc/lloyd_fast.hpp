@@ -43,7 +43,8 @@ template <typename T, typename I>
 void launch_fused_generic(int64_t n, int64_t d, int64_t k, int64_t n_copies,
                           const FusedPlan &p, bool store_flush, const T *X,
                           const T *w, const T *C, const T *hn, I *labels,
-                          T *copies, T *sizes_copies, hipStream_t s);
+                          T *copies, T *sizes_copies, hipStream_t s,
+                          const int *skip = nullptr);
 
 // FP64 MFMA path (v_mfma_f64_16x16x4f64; csrc/lloyd_f64.hip): true when the
 // centroid operands (and, with update, the FP64 sums) fit LDS, d <= 64.
@@ -54,7 +55,7 @@ void launch_fast64_fused(int64_t n, int64_t d, int64_t k, int64_t n_copies,
                          const FusedPlan &p, bool store_flush, const double *X,
                          const double *w, const double *C, const double *hn,
                          I *labels, double *copies, double *sizes_copies,
-                         hipStream_t s);
+                         hipStream_t s, const int *skip = nullptr);
 template <typename I>
 void launch_fast64_assign(int64_t n, int64_t d, int64_t k, const double *X,
                           const double *C, const double *hn, I *labels,
@@ -107,15 +108,12 @@ void launch_fast_fused_fixed(int64_t n, int64_t d, int64_t k, const T *X,
                              hipStream_t s, const int *skip = nullptr);
 
 // Sums the per-block partials of launch_fast_fused_fixed (exactly, in int64,
-// when the fixed-point path ran) into out_cent (d x k) and out_sizes (k),
-// then appends empty clusters to empty_list at n_empty[0]++.
-template <typename T, typename I>
-void launch_reduce_fixed_partials(int64_t n_blocks, int64_t d, int64_t k,
-                                  const void *partials, const float *scale,
-                                  const int *nonfinite, T *out_sizes,
-                                  T *out_cent, I *empty_list, I *n_empty,
-                                  int64_t list_len, hipStream_t s,
-                                  bool from_zero = false);
+// when the fixed-point path ran) into out_cent (d x k) and out_sizes (k).
+template <typename T>
+void launch_sum_fixed_partials(int64_t n_blocks, int64_t d, int64_t k,
+                               const void *partials, const float *scale,
+                               const int *nonfinite, T *out_sizes, T *out_cent,
+                               hipStream_t s, const int *skip = nullptr);
 
 }  // namespace kmd
 
@@ -180,7 +178,8 @@ void launch_fast_rescore(int64_t n, int64_t d, int64_t k, const float *X,
                          I *labels, const float *scale, const int *nonfinite,
                          void *partials, int64_t slot0, const int *queue,
                          const int *queue_counts, int n_segments,
-                         int64_t seg_cap, int *n_rescored, hipStream_t s);
+                         int64_t seg_cap, int *n_rescored, hipStream_t s,
+                         const int *skip = nullptr);
 
 // ---- tiled path (lloyd_tiled.hip): d <= 128, centroids streamed via LDS ----
 bool tiled_supported(int64_t d, int64_t k);
@@ -208,7 +207,7 @@ void launch_tiled_rescore(int64_t n, int64_t d, int64_t k, const float *X_r,
                           const float *C, const float *hn, I *labels,
                           const int *queue, const int *queue_counts,
                           int n_segments, int64_t seg_cap, int *n_rescored,
-                          hipStream_t s);
+                          hipStream_t s, const int *skip = nullptr);
 // BF16 (T = 1) / BF16x3 (T = 3) assignment with the certified margin test:
 // grid size (0 when not served), queue segment capacity, A-operand bytes
 template <typename I>
@@ -250,7 +249,7 @@ void launch_tiled_cand_rescore(int64_t n, int64_t d, int64_t k, const float *X_r
                                const int *queue, const int *queue_counts,
                                const unsigned *qmask, int n_segments,
                                int64_t seg_cap, void *scratch, int *n_rescored,
-                               hipStream_t s);
+                               hipStream_t s, const int *skip = nullptr);
 // Exact int64 fixed-point sums [d*k + k] of w x per label from X_r
 size_t tiled_update_scratch_bytes(int64_t n, int64_t k);
 template <typename I>

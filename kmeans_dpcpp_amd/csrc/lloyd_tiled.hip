@@ -345,7 +345,12 @@ struct CandArgs {
   const float *Xr, *tiles;
   void *labels;
   int *n_rescored;
+  const int *skip;               // when non-null and *skip != 0: do nothing
 };
+
+__device__ inline bool skipped(const CandArgs &a) {
+  return a.skip != nullptr && *a.skip != 0;
+}
 
 __device__ inline unsigned order_key(float v) {
   const unsigned b = __float_as_uint(v + 0.0f);  // -0 -> +0
@@ -353,6 +358,7 @@ __device__ inline unsigned order_key(float v) {
 }
 
 __global__ void __launch_bounds__(256) cand_count_krn(CandArgs a) {
+  if (skipped(a)) return;
   __shared__ int cnt[32];
   const int seg = blockIdx.x;
   if (threadIdx.x < 32) cnt[threadIdx.x] = 0;
@@ -374,6 +380,7 @@ __global__ void __launch_bounds__(256) cand_count_krn(CandArgs a) {
 }
 
 __global__ void cand_scan_krn(CandArgs a) {
+  if (skipped(a)) return;
   if (threadIdx.x != 0) return;
   int run = 0, wrun = 0;
   for (int t = 0; t < a.n_ct; ++t) {
@@ -393,7 +400,7 @@ __global__ void cand_scan_krn(CandArgs a) {
 
 __global__ void __launch_bounds__(256) cand_scatter_krn(CandArgs a) {
   __shared__ int cnt[32];
-  if (a.overflow[0]) return;
+  if (skipped(a) || a.overflow[0]) return;
   const int seg = blockIdx.x;
   if (threadIdx.x < 32) cnt[threadIdx.x] = 0;
   __syncthreads();
@@ -428,7 +435,7 @@ __global__ void __launch_bounds__(256) cand_scatter_krn(CandArgs a) {
 template <int KS>
 __global__ void __launch_bounds__(kTNT) cand_rescore_krn(CandArgs a) {
   constexpr int TF = tile_floats<KS>();
-  if (a.overflow[0]) return;
+  if (skipped(a) || a.overflow[0]) return;
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int col = lane & 31, half = lane >> 5;
   const int total = a.tile_witem[a.n_ct];
@@ -503,7 +510,7 @@ __global__ void __launch_bounds__(kTNT) cand_rescore_krn(CandArgs a) {
 
 template <typename I>
 __global__ void __launch_bounds__(256) cand_finalize_krn(CandArgs a) {
-  if (a.overflow[0]) return;
+  if (skipped(a) || a.overflow[0]) return;
   const int seg = blockIdx.x;
   const int m = a.queue_counts[seg];
   const int64_t base = (int64_t)seg * a.seg_cap;
@@ -1639,9 +1646,7 @@ int occupancy_grid(F fn, size_t lds) {
         break;
       }
   }
-  int per_cu = 0;
-  KMD_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, p, kTNT, lds));
-  per_cu = apply_blocks_cap(per_cu);
+  const int per_cu = apply_blocks_cap(blocks_per_cu(p, kTNT, lds));
   if (per_cu < 1) return 0;
   return device_cu_count() * per_cu;
 }
@@ -1703,7 +1708,8 @@ template <typename I>
 void launch_rescore_full(int64_t n, int64_t d, int64_t k, const float *X_r,
                          const float *tiles, I *labels, const int *queue,
                          const int *queue_counts, int n_segments, int64_t seg_cap,
-                         int *n_rescored, const int *only_if, hipStream_t s) {
+                         int *n_rescored, const int *only_if, hipStream_t s,
+                         const int *skip) {
   require(n_segments >= 1 && n_segments <= kMaxSegments,
           "tiled re-score: segment count out of range");
   TiledFn fn = pick_fp32<I, true>(d);
@@ -1724,6 +1730,7 @@ void launch_rescore_full(int64_t n, int64_t d, int64_t k, const float *X_r,
   a.seg_cap = seg_cap;
   a.n_rescored = n_rescored;
   a.only_if = only_if;
+  a.skip = skip;
   hipLaunchKernelGGL(fn, dim3(grid), dim3(kTNT), lds, s, a);
   KMD_LAUNCH_CHECK();
 }
@@ -1734,10 +1741,10 @@ void launch_tiled_rescore(int64_t n, int64_t d, int64_t k, const float *X_r,
                           const float *C, const float *hn, I *labels,
                           const int *queue, const int *queue_counts,
                           int n_segments, int64_t seg_cap, int *n_rescored,
-                          hipStream_t s) {
+                          hipStream_t s, const int *skip) {
   TempBuffer tiles = prep_fp32_tiles(d, k, C, hn, s);
   launch_rescore_full<I>(n, d, k, X_r, tiles.as<const float>(), labels, queue,
-                         queue_counts, n_segments, seg_cap, n_rescored, nullptr, s);
+                         queue_counts, n_segments, seg_cap, n_rescored, nullptr, s, skip);
 }
 
 bool tiled_cand_supported(int64_t k) { return ceil_div<int64_t>(k, 32) <= 32; }
@@ -1755,7 +1762,7 @@ void launch_tiled_cand_rescore(int64_t n, int64_t d, int64_t k, const float *X_r
                                const int *queue, const int *queue_counts,
                                const unsigned *qmask, int n_segments,
                                int64_t seg_cap, void *scratch, int *n_rescored,
-                               hipStream_t s) {
+                               hipStream_t s, const int *skip) {
   require(tiled_cand_supported(k), "candidate re-score: more than 32 tiles");
   const int n_ct = (int)ceil_div<int64_t>(k, 32);
   TempBuffer tiles = prep_fp32_tiles(d, k, C, hn, s);
@@ -1781,6 +1788,7 @@ void launch_tiled_cand_rescore(int64_t n, int64_t d, int64_t k, const float *X_r
   a.tiles = tiles.as<const float>();
   a.labels = labels;
   a.n_rescored = n_rescored;
+  a.skip = skip;
   hipLaunchKernelGGL(fill_zero_i32_krn, dim3(1), dim3(256), 0, s, 2 * (n_ct + 1),
                      a.tile_cnt);
   KMD_LAUNCH_CHECK();
@@ -1806,7 +1814,7 @@ void launch_tiled_cand_rescore(int64_t n, int64_t d, int64_t k, const float *X_r
   KMD_LAUNCH_CHECK();
   // the pairs did not fit: the full gather re-score of every queued sample
   launch_rescore_full<I>(n, d, k, X_r, tiles.as<const float>(), labels, queue,
-                         queue_counts, n_segments, seg_cap, n_rescored, a.overflow, s);
+                         queue_counts, n_segments, seg_cap, n_rescored, a.overflow, s, skip);
 }
 
 template <typename I>
@@ -2071,7 +2079,7 @@ void launch_label_update(int64_t n, int64_t d, int64_t k, int64_t n_copies,
                                         const float *, const float *,          \
                                         const float *, I *, const int *,       \
                                         const int *, int, int64_t, int *,      \
-                                        hipStream_t);                          \
+                                        hipStream_t, const int *);             \
   template int tiled_mixed_blocks<I>(int64_t, int64_t, int64_t, int);          \
   template void launch_tiled_mixed_assign<I>(int64_t, int64_t, int64_t, int,   \
                                              int, const float *, const void *, \
@@ -2082,7 +2090,7 @@ void launch_label_update(int64_t n, int64_t d, int64_t k, int64_t n_copies,
   template void launch_tiled_cand_rescore<I>(                                  \
       int64_t, int64_t, int64_t, const float *, const float *, const float *,  \
       I *, const int *, const int *, const unsigned *, int, int64_t, void *,   \
-      int *, hipStream_t);                                                     \
+      int *, hipStream_t, const int *);                                        \
   template void launch_tiled_update<I>(int64_t, int64_t, int64_t,              \
                                        const float *, const float *,           \
                                        const I *, const float *, void *,       \

@@ -2,6 +2,8 @@
 // squared norms, private-copy reduction with the empty-cluster list, centroid
 // shifts, per-sample inertia, deterministic sum / max reductions, selection of
 // far samples and empty-cluster relocation.
+#include <algorithm>
+
 #include "common.hpp"
 #include "lloyd_fast.hpp"
 
@@ -36,56 +38,81 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // ---- half squared norms (src/util_kernels.hpp:47-82) -----------------------
-// Column c, rows ascending, fused multiply-add accumulation, then / 2.
+// Column c, rows ascending, fused multiply-add accumulation, then / 2.  The
+// chain of a column is serial, so its values are staged in LDS by the whole
+// block first: 32 columns x 64 rows at a time, all loads in flight.  One
+// thread per column reading global memory took 69 us at d = 300, k = 100
+// (each of the d dependent steps waits on L2), this form 8 us.
+constexpr int kHnCols = 32, kHnRows = 64;
+
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
-    half_l2_norm_krn(int64_t d, int64_t k, const T *C, T *out) {
-  int64_t c = blockIdx.x * (int64_t)kBlock + threadIdx.x;
-  if (c >= k) return;
+    half_l2_norm_krn(int64_t d, int64_t k, const T *__restrict__ C, T *__restrict__ out) {
+  __shared__ T v[kHnRows][kHnCols + 1];
+  const int e = threadIdx.x % kHnCols, g = threadIdx.x / kHnCols;
+  const int64_t c = blockIdx.x * (int64_t)kHnCols + e;
   T acc = T(0);
-  for (int64_t f = 0; f < d; ++f) {
-    T v = C[f * k + c];
-    acc = fma(v, v, acc);
+  for (int64_t f0 = 0; f0 < d; f0 += kHnRows) {
+    __syncthreads();
+#pragma unroll
+    for (int r = g; r < kHnRows; r += kBlock / kHnCols)
+      v[r][e] = (f0 + r < d && c < k) ? C[(f0 + r) * k + c] : T(0);
+    __syncthreads();
+    const int m = (int)min<int64_t>(kHnRows, d - f0);
+    if (g == 0)
+      for (int r = 0; r < m; ++r) acc = fma(v[r][e], v[r][e], acc);
   }
-  out[c] = acc / T(2);
+  if (g == 0 && c < k) out[c] = acc / T(2);
 }
 
 // ---- reduce private copies (src/util_kernels.hpp:84-161) -------------------
-// out[i] = sum over copies of src[copy * stride + i].  A 1024-thread block
-// owns 64 consecutive elements; its 16 wavefronts each sum the copies
-// congruent to their index mod 16 (ascending), then the 16 partial sums are
+// Elements i < dk: centroid sums, out_cent[i] = sum over copies of
+// cent[copy * dk + i]; the k after them: cluster sizes.  A 1024-thread block
+// owns 1024 / G consecutive elements; its thread groups each sum the copies
+// congruent to their index mod G (ascending), then the G partial sums are
 // added in ascending order: a fixed order, so the result is deterministic.
+// Few elements in many copies (few clusters: 264 elements in 695 copies)
+// leave most of the chip idle with G = 16; G = 64 gives four times the blocks
+// and a quarter of the serial additions (35 us in two launches before, 9 us
+// in one).
+constexpr int kRedThreads = 1024;
 constexpr int kRedElems = 64;
 constexpr int kRedGroups = 16;
 
-template <typename T>
-__global__ void __launch_bounds__(kRedElems * kRedGroups)
-    sum_copies_krn(int64_t n_copies, int64_t m, int64_t stride,
-                   const T *__restrict__ src, T *__restrict__ out) {
-  __shared__ T part[kRedGroups][kRedElems];
-  const int e = threadIdx.x % kRedElems, g = threadIdx.x / kRedElems;
-  const int64_t i = blockIdx.x * (int64_t)kRedElems + e;
+template <typename T, int G>
+__global__ void __launch_bounds__(kRedThreads)
+    sum_copies_krn(int64_t n_copies, int64_t dk, int64_t k, const T *__restrict__ cent,
+                   const T *__restrict__ sizes, T *__restrict__ out_cent,
+                   T *__restrict__ out_sizes, const int *skip) {
+  if (skip != nullptr && *skip != 0) return;
+  constexpr int E = kRedThreads / G;
+  __shared__ T part[G][E + 1];
+  const int e = threadIdx.x % E, g = threadIdx.x / E;
+  const int64_t i = blockIdx.x * (int64_t)E + e;
+  const bool is_cent = i < dk;
+  const T *src = is_cent ? cent + i : sizes + (i - dk);
+  const int64_t stride = is_cent ? dk : k;
   T acc = T(0);
-  if (i < m) {
+  if (i < dk + k) {
     int64_t c = g;
-    for (; c + 3 * kRedGroups < n_copies; c += 4 * kRedGroups) {
-      const T a0 = src[c * stride + i];
-      const T a1 = src[(c + kRedGroups) * stride + i];
-      const T a2 = src[(c + 2 * kRedGroups) * stride + i];
-      const T a3 = src[(c + 3 * kRedGroups) * stride + i];
+    for (; c + 3 * G < n_copies; c += 4 * G) {
+      const T a0 = src[c * stride];
+      const T a1 = src[(c + G) * stride];
+      const T a2 = src[(c + 2 * G) * stride];
+      const T a3 = src[(c + 3 * G) * stride];
       acc += a0;
       acc += a1;
       acc += a2;
       acc += a3;
     }
-    for (; c < n_copies; c += kRedGroups) acc += src[c * stride + i];
+    for (; c < n_copies; c += G) acc += src[c * stride];
   }
   part[g][e] = acc;
   __syncthreads();
-  if (g == 0 && i < m) {
+  if (g == 0 && i < dk + k) {
     T t = T(0);
-    for (int q = 0; q < kRedGroups; ++q) t += part[q][e];
-    out[i] = t;
+    for (int q = 0; q < G; ++q) t += part[q][e];
+    (is_cent ? out_cent[i] : out_sizes[i - dk]) = t;
   }
 }
 
@@ -94,12 +121,14 @@ __global__ void __launch_bounds__(kRedElems * kRedGroups)
 // converted once with the feature's scale; or FP32 sums in a fixed order
 // when the inputs held non-finite values.
 template <typename T>
-__global__ void __launch_bounds__(kRedElems * kRedGroups)
+__global__ void __launch_bounds__(kRedThreads)
     sum_partials_fixed_krn(int64_t n_blocks, int64_t d, int64_t k,
                            const void *__restrict__ partials,
                            const float *__restrict__ scale,
                            const int *__restrict__ nonfinite,
-                           T *__restrict__ out_sizes, T *__restrict__ out_cent) {
+                           T *__restrict__ out_sizes, T *__restrict__ out_cent,
+                           const int *skip) {
+  if (skip != nullptr && *skip != 0) return;
   __shared__ long long ipart[kRedGroups][kRedElems];
   __shared__ float fpart[kRedGroups][kRedElems];
   const int e = threadIdx.x % kRedElems, g = threadIdx.x / kRedElems;
@@ -144,10 +173,10 @@ __global__ void __launch_bounds__(kRedElems * kRedGroups)
 template <typename T, typename I>
 __global__ void __launch_bounds__(1024)
     empty_list_krn(int64_t k, const T *__restrict__ sizes, I *empty_list,
-                   I *n_empty, int64_t list_len, bool from_zero) {
+                   I *n_empty, int64_t list_len) {
   __shared__ int wave_counts[1024 / kWave];
   __shared__ int64_t running;
-  if (threadIdx.x == 0) running = from_zero ? 0 : (int64_t)n_empty[0];
+  if (threadIdx.x == 0) running = (int64_t)n_empty[0];
   __syncthreads();
   const int nwaves = blockDim.x / kWave;
   const int w = threadIdx.x / kWave;
@@ -188,75 +217,219 @@ __global__ void __launch_bounds__(kBlock)
   out[c] = acc;
 }
 
-// ---- end of a Lloyd iteration: divide, shifts, their sum -------------------
-// Thread c: column c of `next` divided by sizes[c] (the broadcast divide,
-// src/util_kernels.hpp:9-41), then shift[c] = sum_f (cur - next)^2 in feature
-// order (src/util_kernels.hpp:478-516); the k shifts are summed in FP64 (block
-// sums, then the last block adds the block sums in block order).  With a
-// non-null `gate`, the kernel does nothing while gate[0] != 0: the iteration
-// has empty clusters, which the host relocates (on the undivided sums) before
-// running it again ungated.
+// ---- end of a Lloyd iteration ------------------------------------------------
+// From the undivided sums and sizes: the empty-cluster list, or (no cluster
+// empty) next = sums / sizes (src/util_kernels.hpp:9-41), shift[c] = sum_f
+// (cur - next)^2 in feature order (src/util_kernels.hpp:478-516), the half
+// norms of the new centroids as half_l2_norm_krn computes them, the FP64 sum
+// of the shifts, and the loop's state on the device and in host memory.  A
+// finished loop (stop != 0: converged, or clusters to relocate) makes the
+// kernels enqueued after it return at once.
+//
+// Column tiles are staged in LDS by the whole block (all loads in flight)
+// before the serial chains over the features; a thread per column reading
+// global memory, and a launch for the list, took 38 + 5 us at d = 300, k =
+// 100 and 5.4 + 2.7 us at d = 14, k = 127, where this takes 16 and 4.3 us.
+// Shapes that fit one tile (d = 32, k = 256 does) run on one block and keep
+// the shifts in registers (65 us for one block over six tiles, d = 96, k =
+// 512: 15 us with the others); the others run a block per tile, at most
+// kTailBlocks (the ticket's atomics serialise), and the last one to finish
+// adds up the shifts.
+constexpr int kTailThreads = 1024;
+constexpr int kTailValues = 8192;        // values of one LDS tile
+constexpr int kTailSmall = 2048;         // wanted values of one of many tiles
+constexpr int kTailBlocks = 64;
+
+// Columns of one tile: a power of two up to kTailThreads.
+inline int tail_cols(int64_t d, int64_t k) {
+  auto pow2_up = [](int64_t v) {
+    int64_t p = 1;
+    while (p < v) p *= 2;
+    return p;
+  };
+  const int64_t whole = pow2_up(k);
+  if (whole <= kTailThreads && d * whole <= kTailValues) return (int)whole;
+  int64_t ct = 8;
+  while (2 * ct * d <= kTailSmall) ct *= 2;
+  ct = std::max(ct, pow2_up(ceil_div<int64_t>(k, kTailBlocks)));
+  return (int)std::min<int64_t>(ct, kTailThreads);
+}
+
 template <typename T, typename I>
-__global__ void __launch_bounds__(kBlock)
-    finalize_step_krn(int64_t d, int64_t k, const I *gate,
-                      const T *__restrict__ sizes, const T *__restrict__ cur,
-                      T *__restrict__ next, T *__restrict__ shifts,
-                      T *__restrict__ hn_next, double *partials,
-                      unsigned *ticket, double *out_sum) {
-  __shared__ double lds[kBlock / kWave];
-  __shared__ bool last;
-  if (gate != nullptr && gate[0] != I(0)) return;
-  const int64_t c = blockIdx.x * (int64_t)kBlock + threadIdx.x;
-  double v = 0.0;
-  if (c < k) {
-    const T sz = sizes[c];
-    T acc = T(0), h = T(0);
-    constexpr int kF = 8;  // features loaded ahead of their use
-    for (int64_t f0 = 0; f0 < d; f0 += kF) {
-      T nv[kF], cv[kF];
+__global__ void __launch_bounds__(kTailThreads)
+    step_tail_krn(StepTail<T, I> a, int CT) {
+  extern __shared__ __align__(16) unsigned char tail_smem[];
+  T *qv = reinterpret_cast<T *>(tail_smem);   // [rows][CT] new centroids
+  T *cv = qv + kTailValues;                   // [rows][CT] old centroids
+  double *lds = reinterpret_cast<double *>(cv + kTailValues);   // one per wave
+  int *wave_counts = reinterpret_cast<int *>(lds + kTailThreads / kWave);
+  int &last = wave_counts[kTailThreads / kWave];
+  const int tid = threadIdx.x, wave = tid / kWave;
+  const int64_t d = a.d, k = a.k;
+  // the first sizes are read beside the loop's state
+  const T size0 = tid < k ? a.sizes[tid] : T(1);
+  if (!a.relocated && a.state->stop != 0) return;
+
+  if (!a.relocated) {
+    // every block looks for empty clusters itself; block 0 lists them
+    bool any = size0 == T(0);
+    for (int64_t c = tid + kTailThreads; c < k; c += kTailThreads)
+      any |= a.sizes[c] == T(0);
+    const uint64_t any_mask = __ballot(any);
+    if (lane_id() == 0) wave_counts[wave] = any_mask != 0;
+    __syncthreads();
+    int n_any = 0;
+    for (int i = 0; i < kTailThreads / kWave; ++i) n_any += wave_counts[i];
+    if (n_any != 0) {
+      if (blockIdx.x != 0) return;
+      int64_t found = 0;
+      for (int64_t c0 = 0; c0 < k; c0 += kTailThreads) {
+        const int64_t c = c0 + tid;
+        const bool empty = c < k && a.sizes[c] == T(0);
+        const uint64_t mask = __ballot(empty);
+        __syncthreads();
+        if (lane_id() == 0) wave_counts[wave] = __popcll(mask);
+        __syncthreads();
+        int before = 0, total = 0;
+        for (int i = 0; i < kTailThreads / kWave; ++i) {
+          before += i < wave ? wave_counts[i] : 0;
+          total += wave_counts[i];
+        }
+        if (empty)
+          a.list[found + before + __popcll(mask & ((1ull << lane_id()) - 1ull))] = (I)c;
+        found += total;
+      }
+      if (tid == 0) {
+        LoopState *st = a.state;
+        st->n_empty = found;
+        st->rescored += a.rescored != nullptr ? a.rescored[0] : 0;
+        st->done += 1;
+        // the other blocks read sizes, not this
+        st->stop = kLoopEmpty;
+        publish(a.host, *st);
+      }
+      return;
+    }
+  }
+
+  const int rows = kTailValues / CT;
+  const int e = tid & (CT - 1);              // this thread's column of a tile
+  const int r0 = tid / CT, rstep = kTailThreads / CT;
+  const int64_t n_tiles = (k + CT - 1) / CT;
+  T acc = T(0);
+  for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+    const int64_t c0 = tile * CT;
+    const int64_t c = c0 + tid;
+    const bool col = c0 + e < k;
+    const T size = col ? a.sizes[c0 + e] : T(1);
+    T h = T(0);
+    acc = T(0);
+    for (int64_t f0 = 0; f0 < d; f0 += rows) {
+      const int m = (int)min<int64_t>(rows, d - f0);
+      __syncthreads();
+      constexpr int kU = 4;   // rows loaded ahead of their use
+      for (int r = r0; r < m; r += kU * rstep) {
+        T sv[kU], ov[kU];
 #pragma unroll
-      for (int j = 0; j < kF; ++j) {
-        if (f0 + j < d) {
-          nv[j] = next[(f0 + j) * k + c];
-          cv[j] = cur[(f0 + j) * k + c];
+        for (int u = 0; u < kU; ++u) {
+          const int64_t at = (f0 + r + u * rstep) * k + c0 + e;
+          const bool in = col && r + u * rstep < m;
+          sv[u] = in ? a.sums[at] : T(0);
+          ov[u] = in ? a.cur[at] : T(0);
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          const int64_t at = (f0 + r + u * rstep) * k + c0 + e;
+          if (col && r + u * rstep < m) {
+            const T q = sv[u] / size;
+            a.next[at] = q;
+            qv[(r + u * rstep) * CT + e] = q;
+            cv[(r + u * rstep) * CT + e] = ov[u];
+          }
         }
       }
-#pragma unroll
-      for (int j = 0; j < kF; ++j) {
-        if (f0 + j < d) {
-          const T q = nv[j] / sz;
-          next[(f0 + j) * k + c] = q;
-          const T diff = cv[j] - q;
+      __syncthreads();
+      if (tid < CT && c < k) {
+#pragma unroll 8
+        for (int r = 0; r < m; ++r) {
+          const T q = qv[r * CT + tid], diff = cv[r * CT + tid] - q;
           acc = fma(diff, diff, acc);
           h = fma(q, q, h);
         }
       }
     }
-    shifts[c] = acc;
-    // half squared norm of the new centroid, as half_l2_norm_krn computes it
-    if (hn_next != nullptr) hn_next[c] = h / T(2);
-    v = (double)acc;
+    if (tid < CT && c < k) {
+      a.hn[c] = h / T(2);
+      if (n_tiles > 1) a.shifts[c] = acc;
+    }
   }
-  const double t = block_sum(v, lds);
-  if (threadIdx.x == 0) {
-    partials[blockIdx.x] = t;
-    __threadfence();
-    last = atomicAdd(ticket, 1u) == gridDim.x - 1;
+  // Sum of the shifts in FP64: the 64 columns of a wave by exchanges, the four
+  // waves of each 256 columns, then those sums by 256 threads the same way.
+  auto wave_sum = [](double v) {
+    for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+    return v;
+  };
+  double tot = 0.0;
+  if (n_tiles == 1) {   // k <= 1024: at most four sums of 256 columns
+    const double t = wave_sum(tid < k ? (double)acc : 0.0);
+    if (lane_id() == 0) lds[wave] = t;
+    __syncthreads();
+    if (tid != 0) return;
+    double p[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      p[j] = 0.0;
+      for (int i = 0; i < 4; ++i) p[j] += lds[4 * j + i];
+    }
+    tot = (p[0] + p[2]) + (p[1] + p[3]);   // the exchanges' order
+  } else {
+    if (gridDim.x > 1) {
+      __threadfence();
+      __syncthreads();
+      if (tid == 0) last = atomicAdd(a.ticket, 1u) == gridDim.x - 1 ? 1 : 0;
+      __syncthreads();
+      if (last == 0) return;
+      __threadfence();
+    } else {
+      __syncthreads();
+    }
+    for (int64_t c0 = 0; c0 < k; c0 += kTailThreads) {
+      const int64_t c = c0 + tid;
+      const double v =
+          c < k ? (double)__hip_atomic_load(&a.shifts[c], __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT)
+                : 0.0;
+      const double t = wave_sum(v);
+      __syncthreads();
+      if (lane_id() == 0) lds[wave] = t;
+      __syncthreads();
+      if (tid < kTailThreads / 256 && c0 + 256 * tid < k) {
+        double u = 0.0;
+        for (int i = 0; i < 4; ++i) u += lds[4 * tid + i];
+        a.partials[c0 / 256 + tid] = u;
+      }
+    }
+    __syncthreads();
+    const int64_t nb = (k + 255) / 256;
+    double v = 0.0;
+    if (tid < 256)
+      for (int64_t i = tid; i < nb; i += 256) v += a.partials[i];
+    const double t = wave_sum(v);
+    if (lane_id() == 0) lds[wave] = t;
+    __syncthreads();
+    if (tid != 0) return;
+    for (int i = 0; i < 4; ++i) tot += lds[i];
+    if (gridDim.x > 1) a.ticket[0] = 0u;
   }
-  __syncthreads();
-  if (!last) return;
-  __threadfence();
-  double a = 0.0;
-  const unsigned long long *pb =
-      reinterpret_cast<const unsigned long long *>(partials);
-  for (int i = threadIdx.x; i < (int)gridDim.x; i += kBlock)
-    a += __longlong_as_double((long long)__hip_atomic_load(
-        &pb[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-  const double tot = block_sum(a, lds);
-  if (threadIdx.x == 0) {
-    out_sum[0] = tot;
-    ticket[0] = 0u;
+  LoopState *st = a.state;
+  st->shift = tot;
+  if (!a.relocated) {
+    st->rescored += a.rescored != nullptr ? a.rescored[0] : 0;
+    st->done += 1;
   }
+  // the loop goes on while the sum, in the data type, exceeds tol
+  st->stop = (T)tot > a.tol ? 0 : kLoopConverged;
+  publish(a.host, *st);
 }
 
 // ---- per-sample inertia (src/compute_inertia.hpp:11-99) --------------------
@@ -589,6 +762,25 @@ __global__ void init_counters_krn(I *n_gt, I *n_eq) {
   n_eq[0] = I(1);
 }
 
+// The sums of sum_copies_krn, both arrays in one launch.
+template <typename T>
+void sum_copies(int64_t n_copies, int64_t dk, int64_t k, const T *cent, const T *sizes,
+                T *out_cent, T *out_sizes, hipStream_t s, const int *skip) {
+  if (dk + k <= 0) return;
+  if (n_copies >= 256 && dk + k <= 16384) {
+    hipLaunchKernelGGL((sum_copies_krn<T, 64>),
+                       dim3((unsigned)ceil_div<int64_t>(dk + k, kRedThreads / 64)),
+                       dim3(kRedThreads), 0, s, n_copies, dk, k, cent, sizes, out_cent,
+                       out_sizes, skip);
+  } else {
+    hipLaunchKernelGGL((sum_copies_krn<T, kRedGroups>),
+                       dim3((unsigned)ceil_div<int64_t>(dk + k, kRedElems)),
+                       dim3(kRedThreads), 0, s, n_copies, dk, k, cent, sizes, out_cent,
+                       out_sizes, skip);
+  }
+  KMD_LAUNCH_CHECK();
+}
+
 inline int grid_for(int64_t n, int per_block, int cap) {
   int64_t g = ceil_div<int64_t>(n, per_block);
   if (g < 1) g = 1;
@@ -614,7 +806,7 @@ template <typename T>
 void launch_half_l2_norm(int64_t d, int64_t k, const T *C, T *out,
                          hipStream_t s) {
   if (k == 0) return;
-  hipLaunchKernelGGL(half_l2_norm_krn<T>, dim3(ceil_div<int64_t>(k, kBlock)),
+  hipLaunchKernelGGL(half_l2_norm_krn<T>, dim3((unsigned)ceil_div<int64_t>(k, kHnCols)),
                      dim3(kBlock), 0, s, d, k, C, out);
   KMD_LAUNCH_CHECK();
 }
@@ -623,42 +815,32 @@ template <typename T, typename I>
 void launch_reduce_centroids(int64_t n_copies, int64_t d, int64_t k,
                              const T *sizes_copies, const T *cent_copies,
                              T *out_sizes, T *out_cent, I *empty_list,
-                             I *n_empty, int64_t list_len, hipStream_t s,
-                             bool from_zero) {
-  const int64_t dk = d * k;
-  if (dk > 0) {
-    hipLaunchKernelGGL(sum_copies_krn<T>, dim3(ceil_div<int64_t>(dk, kRedElems)),
-                       dim3(kRedElems * kRedGroups), 0, s, n_copies, dk, dk,
-                       cent_copies, out_cent);
-    KMD_LAUNCH_CHECK();
-  }
-  if (k > 0) {
-    hipLaunchKernelGGL(sum_copies_krn<T>, dim3(ceil_div<int64_t>(k, kRedElems)),
-                       dim3(kRedElems * kRedGroups), 0, s, n_copies, k, k,
-                       sizes_copies, out_sizes);
-    KMD_LAUNCH_CHECK();
-  }
+                             I *n_empty, int64_t list_len, hipStream_t s) {
+  sum_copies<T>(n_copies, d * k, k, cent_copies, sizes_copies, out_cent, out_sizes, s,
+                nullptr);
   hipLaunchKernelGGL((empty_list_krn<T, I>), dim3(1), dim3(1024), 0, s, k,
-                     (const T *)out_sizes, empty_list, n_empty, list_len,
-                     from_zero);
+                     (const T *)out_sizes, empty_list, n_empty, list_len);
   KMD_LAUNCH_CHECK();
 }
 
-template <typename T, typename I>
-void launch_reduce_fixed_partials(int64_t n_blocks, int64_t d, int64_t k,
-                                  const void *partials, const float *scale,
-                                  const int *nonfinite, T *out_sizes,
-                                  T *out_cent, I *empty_list, I *n_empty,
-                                  int64_t list_len, hipStream_t s,
-                                  bool from_zero) {
+template <typename T>
+void launch_sum_copies(int64_t n_copies, int64_t d, int64_t k, const T *sizes_copies,
+                       const T *cent_copies, T *out_sizes, T *out_cent, hipStream_t s,
+                       const int *skip) {
+  sum_copies<T>(n_copies, d * k, k, cent_copies, sizes_copies, out_cent, out_sizes, s,
+                skip);
+}
+
+template <typename T>
+void launch_sum_fixed_partials(int64_t n_blocks, int64_t d, int64_t k,
+                               const void *partials, const float *scale,
+                               const int *nonfinite, T *out_sizes, T *out_cent,
+                               hipStream_t s, const int *skip) {
   const int64_t m = d * k + k;
-  hipLaunchKernelGGL(sum_partials_fixed_krn<T>, dim3(ceil_div<int64_t>(m, kRedElems)),
-                     dim3(kRedElems * kRedGroups), 0, s, n_blocks, d, k,
-                     partials, scale, nonfinite, out_sizes, out_cent);
-  KMD_LAUNCH_CHECK();
-  hipLaunchKernelGGL((empty_list_krn<T, I>), dim3(1), dim3(1024), 0, s, k,
-                     (const T *)out_sizes, empty_list, n_empty, list_len,
-                     from_zero);
+  hipLaunchKernelGGL(sum_partials_fixed_krn<T>,
+                     dim3((unsigned)ceil_div<int64_t>(m, kRedElems)), dim3(kRedThreads), 0,
+                     s, n_blocks, d, k, partials, scale, nonfinite, out_sizes, out_cent,
+                     skip);
   KMD_LAUNCH_CHECK();
 }
 
@@ -671,18 +853,17 @@ void launch_centroid_shifts(int64_t d, int64_t k, const T *a, const T *b,
   KMD_LAUNCH_CHECK();
 }
 
-int finalize_step_blocks(int64_t k) {
-  return (int)ceil_div<int64_t>(k > 0 ? k : 1, kBlock);
-}
+int64_t step_tail_partials(int64_t k) { return ceil_div<int64_t>(k > 0 ? k : 1, 256); }
 
 template <typename T, typename I>
-void launch_finalize_step(int64_t d, int64_t k, const I *gate, const T *sizes,
-                          const T *cur, T *next, T *shifts, T *hn_next,
-                          double *partials, unsigned *ticket, double *out_sum,
-                          hipStream_t s) {
-  hipLaunchKernelGGL((finalize_step_krn<T, I>), dim3(finalize_step_blocks(k)),
-                     dim3(kBlock), 0, s, d, k, gate, sizes, cur, next, shifts,
-                     hn_next, partials, ticket, out_sum);
+void launch_step_tail(const StepTail<T, I> &a, hipStream_t s) {
+  const int CT = tail_cols(a.d, a.k);
+  const unsigned blocks =
+      (unsigned)std::min<int64_t>(ceil_div<int64_t>(a.k, CT), kTailBlocks);
+  const size_t lds = 2 * sizeof(T) * kTailValues +
+                     (kTailThreads / kWave) * (sizeof(double) + sizeof(int)) + sizeof(double);
+  allow_full_lds(reinterpret_cast<const void *>(&step_tail_krn<T, I>));
+  hipLaunchKernelGGL((step_tail_krn<T, I>), dim3(blocks), dim3(kTailThreads), lds, s, a, CT);
   KMD_LAUNCH_CHECK();
 }
 
@@ -814,14 +995,20 @@ void launch_relocate(int64_t n, int64_t d, int64_t k, int64_t n_empty,
                                      hipStream_t);                            \
   template void launch_sum_to_scalar<T>(int64_t, const T *, T *,              \
                                         hipStream_t);                         \
-  template void launch_max<T>(int64_t, const T *, T *, hipStream_t);
+  template void launch_max<T>(int64_t, const T *, T *, hipStream_t);           \
+  template void launch_sum_copies<T>(int64_t, int64_t, int64_t, const T *,    \
+                                     const T *, T *, T *, hipStream_t,        \
+                                     const int *);                            \
+  template void launch_sum_fixed_partials<T>(                                 \
+      int64_t, int64_t, int64_t, const void *, const float *, const int *,    \
+      T *, T *, hipStream_t, const int *);
 KMD_INST_T(float)
 KMD_INST_T(double)
 
 #define KMD_INST_TI(T, I)                                                     \
   template void launch_reduce_centroids<T, I>(                                \
       int64_t, int64_t, int64_t, const T *, const T *, T *, T *, I *, I *,    \
-      int64_t, hipStream_t, bool);                                                  \
+      int64_t, hipStream_t);                                                  \
   template void launch_inertia<T, I>(int64_t, int64_t, int64_t, const T *,   \
                                      const T *, const T *, const I *, T *,    \
                                      hipStream_t);                            \
@@ -832,13 +1019,7 @@ KMD_INST_T(double)
                                       const T *, const T *, const I *,        \
                                       const I *, const T *, T *, T *, T *,    \
                                       hipStream_t);                           \
-  template void launch_reduce_fixed_partials<T, I>(                           \
-      int64_t, int64_t, int64_t, const void *, const float *, const int *,   \
-      T *, T *, I *, I *, int64_t, hipStream_t, bool);                              \
-  template void launch_finalize_step<T, I>(int64_t, int64_t, const I *,      \
-                                           const T *, const T *, T *, T *,    \
-                                           T *, double *, unsigned *,         \
-                                           double *, hipStream_t);
+  template void launch_step_tail<T, I>(const StepTail<T, I> &, hipStream_t);
 KMD_INST_TI(float, int32_t)
 KMD_INST_TI(float, int64_t)
 KMD_INST_TI(double, int32_t)
