@@ -28,6 +28,7 @@
 // bit.
 #include <algorithm>
 
+#include "fp32_tile.hpp"
 #include "lloyd_fast.hpp"
 
 namespace kmd {
@@ -35,7 +36,6 @@ namespace kmd {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned long long u64;
 
@@ -70,12 +70,13 @@ __device__ inline void wait_dma_and_sync() {
 
 // ---- FP32 assignment --------------------------------------------------------
 
-// FP32 k-steps (2 features each), bucketed.
+// FP32 k-steps (2 features each), bucketed.  Every k-step of padding is a
+// product per tile and column block that nobody needs: with buckets of 16, 32
+// and 64 k-steps alone, d = 96 did a third more products than it has (n =
+// 500,000, k = 512: 0.449 ms per pass, 0.348 with 48).
 inline int ks_of(int64_t d) {
   const int64_t ks = (d + 1) / 2;
-  if (ks <= 16) return 16;
-  if (ks <= 32) return 32;
-  return 64;
+  return ks <= 16 ? 16 : (int)ceil_div<int64_t>(ks, 8) * 8;
 }
 
 template <int KS>
@@ -218,12 +219,15 @@ __global__ void __launch_bounds__(kTNT) tiled_fp32_krn(TiledArgs a) {
         }
       }
     }
-    float bestv[S];
-    int besti[S];
+    // running best: its value, tile and that tile's accumulators
+    float bestm[S];
+    int bestt[S];
+    f32x16 besta[S];
 #pragma unroll
     for (int q = 0; q < S; ++q) {
-      bestv[q] = __builtin_huge_valf();
-      besti[q] = 0;
+      bestm[q] = -__builtin_huge_valf();
+      bestt[q] = 0;
+      besta[q] = f32x16{};
     }
     for (int ci = 0; ci < n_chunks; ++ci, ++g) {
       const int c0 = ci * CPC;
@@ -238,7 +242,6 @@ __global__ void __launch_bounds__(kTNT) tiled_fp32_krn(TiledArgs a) {
       if (active) {
         for (int t = 0; t < cnt; ++t) {
           const float *At = Cl + t * TF;
-          // rows of this lane: m = 8 (r / 4) + 4 half + (r % 4), ascending;
           // the chain starts from -hn (the tile stores it), so -acc = hn - c.x
           const float *Ht = At + 2 * KS * 32;
           f32x16 h;
@@ -267,22 +270,19 @@ __global__ void __launch_bounds__(kTNT) tiled_fp32_krn(TiledArgs a) {
               }
             }
           }
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const int m0 = 8 * g + 4 * half;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-#pragma unroll
-              for (int q = 0; q < S; ++q) {
-                const float v = -acc[q][4 * g + e];
-                const bool upd = v < bestv[q];
-                bestv[q] = upd ? v : bestv[q];
-                besti[q] = upd ? ((c0 + t) * 32 + m0 + e) : besti[q];
-              }
-            }
-          }
+          tile_track_best<S>(c0 + t, acc, bestm, bestt, besta);
         }
       }
+    }
+    // no row of any tile below +inf: centroid 0, as the scan would give
+    float bestv[S];
+    int besti[S];
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+      bestv[q] = -bestm[q];
+      besti[q] = (bestv[q] < __builtin_huge_valf())
+                     ? best_index(bestt[q], best_row(besta[q], bestm[q]), half)
+                     : 0;
     }
 #pragma unroll
     for (int q = 0; q < S; ++q) {
@@ -1525,19 +1525,33 @@ __global__ void __launch_bounds__(320)
 using TiledFn = void (*)(TiledArgs);
 using TiledMixedFn = void (*)(TiledMixedArgs);
 
+// f(integral constant KS) for the bucket of d
+template <typename F>
+auto with_ks(int64_t d, F &&f) {
+  switch (ks_of(d)) {
+    case 16: return f(std::integral_constant<int, 16>{});
+    case 24: return f(std::integral_constant<int, 24>{});
+    case 32: return f(std::integral_constant<int, 32>{});
+    case 40: return f(std::integral_constant<int, 40>{});
+    case 48: return f(std::integral_constant<int, 48>{});
+    case 56: return f(std::integral_constant<int, 56>{});
+    default: return f(std::integral_constant<int, 64>{});
+  }
+}
+
 template <typename I, bool GATHER>
 TiledFn pick_fp32(int64_t d) {
-  switch (ks_of(d)) {
-    case 16: return &tiled_fp32_krn<16, I, GATHER>;
-    case 32: return &tiled_fp32_krn<32, I, GATHER>;
-    default: return &tiled_fp32_krn<64, I, GATHER>;
-  }
+  return with_ks(d, [](auto ks) -> TiledFn { return &tiled_fp32_krn<ks(), I, GATHER>; });
 }
 
 }  // namespace
 
 size_t tiled_tiles_bytes(int64_t d, int64_t k) {
-  const int TF = 2 * ks_of(d) * 32 + 32;
+  // in whole buckets of 16, 32 or 64 k-steps, whatever the kernel's own
+  // bucket needs of it: callers with a fixed scratch accept or refuse a shape
+  // by this size
+  const int64_t ks = ks_of(d) <= 16 ? 16 : ks_of(d) <= 32 ? 32 : 64;
+  const int64_t TF = 2 * ks * 32 + 32;
   return sizeof(float) * (size_t)(ceil_div<int64_t>(k, 32) * TF) + 1024;
 }
 
@@ -1561,19 +1575,10 @@ void prep_fp32_tiles_into(int64_t d, int64_t k, const float *C, const float *hn,
   const int n_ct = (int)ceil_div<int64_t>(k, 32);
   const int64_t total = (int64_t)n_ct * TF;
   const dim3 grid((unsigned)ceil_div<int64_t>(total, 256));
-  switch (KS) {
-    case 16:
-      hipLaunchKernelGGL(tiled_fp32_prep_krn<16>, grid, dim3(256), 0, s, (int)d,
-                         (int)k, n_ct, C, hn, t);
-      break;
-    case 32:
-      hipLaunchKernelGGL(tiled_fp32_prep_krn<32>, grid, dim3(256), 0, s, (int)d,
-                         (int)k, n_ct, C, hn, t);
-      break;
-    default:
-      hipLaunchKernelGGL(tiled_fp32_prep_krn<64>, grid, dim3(256), 0, s, (int)d,
-                         (int)k, n_ct, C, hn, t);
-  }
+  with_ks(d, [&](auto ks) {
+    hipLaunchKernelGGL(tiled_fp32_prep_krn<ks()>, grid, dim3(256), 0, s, (int)d, (int)k,
+                       n_ct, C, hn, t);
+  });
   KMD_LAUNCH_CHECK();
 }
 
@@ -1799,16 +1804,9 @@ void launch_tiled_cand_rescore(int64_t n, int64_t d, int64_t k, const float *X_r
   hipLaunchKernelGGL(cand_scatter_krn, dim3(n_segments), dim3(256), 0, s, a);
   KMD_LAUNCH_CHECK();
   const int grid = device_cu_count() * 2;
-  switch (ks_of(d)) {
-    case 16:
-      hipLaunchKernelGGL(cand_rescore_krn<16>, dim3(grid), dim3(kTNT), 0, s, a);
-      break;
-    case 32:
-      hipLaunchKernelGGL(cand_rescore_krn<32>, dim3(grid), dim3(kTNT), 0, s, a);
-      break;
-    default:
-      hipLaunchKernelGGL(cand_rescore_krn<64>, dim3(grid), dim3(kTNT), 0, s, a);
-  }
+  with_ks(d, [&](auto ks) {
+    hipLaunchKernelGGL(cand_rescore_krn<ks()>, dim3(grid), dim3(kTNT), 0, s, a);
+  });
   KMD_LAUNCH_CHECK();
   hipLaunchKernelGGL((cand_finalize_krn<I>), dim3(n_segments), dim3(256), 0, s, a);
   KMD_LAUNCH_CHECK();
