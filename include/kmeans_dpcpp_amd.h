@@ -391,6 +391,26 @@ int kmd_column_mean_var(int dtype, int64_t n_samples, int64_t n_features,
 int kmd_transpose(int dtype, int64_t rows, int64_t cols, const void *src,
                   const double *shift, void *dst, kmd_stream_t stream);
 
+/* distances[s, c] = ||X[s, :] - centers[c, :]|| for sample-major X
+ * (n_samples, n_features), centers (n_clusters, n_features) and distances
+ * (n_samples, n_clusters): the values of
+ * kmd_compute_centroid_to_sample_distances, without the transposes.
+ * kmd_row_distances_scratch: elements of dtype that `scratch` needs, 0 when
+ * n_features is beyond the kernel (128 for float32, 64 for float64). */
+int64_t kmd_row_distances_scratch(int dtype, int64_t n_features, int64_t n_clusters);
+int kmd_row_distances(int dtype, int64_t n_samples, int64_t n_features,
+                      int64_t n_clusters, const void *X, const void *centers,
+                      void *scratch, void *distances, kmd_stream_t stream);
+
+/* labels[s] = kmd_assignment's label of row s for sample-major float32 X
+ * (n_samples, n_features) and centers (n_clusters, n_features), without the
+ * transpose.  kmd_assign_rows_scratch: bytes of device memory `scratch`
+ * needs, 0 when the shape is not served. */
+int64_t kmd_assign_rows_scratch(int64_t n_features, int64_t n_clusters);
+int kmd_assign_rows(int64_t n_samples, int64_t n_features, int64_t n_clusters,
+                    const float *X, const float *centers, void *scratch,
+                    int32_t *labels, kmd_stream_t stream);
+
 /* out_t[:, j] = X_t[:, indices[j]] for j < n_indices (indices: device
  * int64, each in [0, n_samples)). */
 int kmd_gather_columns(int dtype, int64_t n_samples, int64_t n_features,

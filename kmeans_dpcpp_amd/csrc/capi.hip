@@ -929,6 +929,77 @@ int kmd_transpose(int dtype, int64_t rows, int64_t cols, const void *src,
   });
 }
 
+int64_t kmd_row_distances_scratch(int dtype, int64_t n_features, int64_t n_clusters) {
+  if (n_features < 1 || n_clusters < 1) return 0;
+  if (dtype == KMD_F32) return row_distances_scratch<float>(n_features, n_clusters);
+  if (dtype == KMD_F64) return row_distances_scratch<double>(n_features, n_clusters);
+  return 0;
+}
+
+int kmd_row_distances(int dtype, int64_t n_samples, int64_t n_features,
+                      int64_t n_clusters, const void *X, const void *centers,
+                      void *scratch, void *distances, kmd_stream_t stream) {
+  return guarded([&] {
+    check_dtype(dtype);
+    require(n_samples >= 0 && n_features >= 1 && n_clusters >= 1,
+            "Inputs have inconsistent dimensions.");
+    require(n_clusters <= INT32_MAX - 64 && n_features <= INT32_MAX,
+            "n_clusters and n_features must fit in 32 bits");
+    check_ptr(X, n_samples * n_features, "X");
+    check_ptr(centers, n_clusters * n_features, "centers");
+    check_ptr(scratch, 1, "scratch");
+    check_ptr(distances, n_samples * n_clusters, "distances");
+    dispatch_t(dtype, [&](auto *tp) {
+      using T = std::remove_pointer_t<decltype(tp)>;
+      require(row_distances_scratch<T>(n_features, n_clusters) > 0,
+              "row distances: too many features");
+      launch_row_distances<T>(n_samples, n_features, n_clusters, (const T *)X,
+                              (const T *)centers, (T *)scratch, (T *)distances,
+                              as_stream(stream));
+    });
+  });
+}
+
+// scratch: the transposed centres, their half norms, then the tiled kernel's
+// centroid tiles
+int64_t kmd_assign_rows_scratch(int64_t n_features, int64_t n_clusters) {
+  if (n_features < 1 || n_clusters < 1 || n_clusters > INT32_MAX) return 0;
+  const int64_t base =
+      ceil_div<int64_t>((n_features * n_clusters + n_clusters) * 4, 256) * 256;
+  if (fast_assign_rows_supported(n_features, n_clusters)) return base;
+  if (tiled_supported(n_features, n_clusters))
+    return base + (int64_t)tiled_tiles_bytes(n_features, n_clusters);
+  return 0;
+}
+
+int kmd_assign_rows(int64_t n_samples, int64_t n_features, int64_t n_clusters,
+                    const float *X, const float *centers, void *scratch,
+                    int32_t *labels, kmd_stream_t stream) {
+  return guarded([&] {
+    require(n_samples >= 0 && n_features >= 1 && n_clusters >= 1,
+            "Inputs have inconsistent dimensions.");
+    require(kmd_assign_rows_scratch(n_features, n_clusters) > 0,
+            "row assignment: unsupported shape");
+    check_ptr(X, n_samples * n_features, "X");
+    check_ptr(centers, n_clusters * n_features, "centers");
+    check_ptr(scratch, 1, "scratch");
+    check_ptr(labels, n_samples, "labels");
+    hipStream_t s = as_stream(stream);
+    float *C_t = static_cast<float *>(scratch);
+    float *hn = C_t + n_features * n_clusters;
+    launch_transpose_shift<float>(n_clusters, n_features, centers, nullptr, C_t, s);
+    launch_half_l2_norm<float>(n_features, n_clusters, C_t, hn, s);
+    if (fast_assign_rows_supported(n_features, n_clusters)) {
+      launch_fast_assign_rows(n_samples, n_features, n_clusters, X, C_t, hn, labels, s);
+    } else {
+      char *tiles = static_cast<char *>(scratch) +
+                    ceil_div<int64_t>((n_features * n_clusters + n_clusters) * 4, 256) * 256;
+      launch_tiled_assign_rows(n_samples, n_features, n_clusters, X, C_t, hn, labels, tiles,
+                               s);
+    }
+  });
+}
+
 int kmd_gather_columns(int dtype, int64_t n_samples, int64_t n_features,
                        int64_t n_indices, const void *X_t,
                        const int64_t *indices, void *out_t,

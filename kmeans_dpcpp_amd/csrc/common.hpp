@@ -261,6 +261,13 @@ void launch_column_mean_var(int64_t n, int64_t d, const T *X, double *mean,
 template <typename T>
 void launch_transpose_shift(int64_t rows, int64_t cols, const T *src,
                             const double *shift, T *dst, hipStream_t s);
+// Distances (n, k) of the rows of X (n, d) to the centres C (k, d) (rows.hip).
+// scratch: row_distances_scratch<T>(d, k) values; 0: the shape is not served.
+template <typename T>
+int64_t row_distances_scratch(int64_t d, int64_t k);
+template <typename T>
+void launch_row_distances(int64_t n, int64_t d, int64_t k, const T *X, const T *C,
+                          T *scratch, T *D, hipStream_t s);
 template <typename T>
 void launch_gather_columns(int64_t n, int64_t d, int64_t m, const T *X_t,
                            const int64_t *idx, T *out_t, hipStream_t s);

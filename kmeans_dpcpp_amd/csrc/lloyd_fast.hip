@@ -99,6 +99,22 @@ __device__ inline void load_x(const float *__restrict__ X, int64_t n, int d,
   }
 }
 
+// The same from sample-major X (n, d): xr[ks][q] = X[s_first + q][2 ks + half].
+// A load touches 32 rows, 8 bytes of each; a row's KS loads follow each other,
+// so its lines come from HBM once and the rest from the L1 cache.
+template <int KS, int S, bool FULL>
+__device__ inline void load_rows(const float *__restrict__ X, int64_t n, int d,
+                                 int64_t s_first, int half, float (&xr)[KS][S]) {
+#pragma unroll
+  for (int q = 0; q < S; ++q) {
+    // rows past the last one read it and are not stored
+    const float *row = X + min<int64_t>(s_first + q, n - 1) * d + half;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      xr[ks][q] = (FULL || 2 * ks + half < d) ? row[2 * ks] : 0.f;
+  }
+}
+
 // Launch parameters shared by the kernel variants.
 struct FastArgs {
   int64_t n;
@@ -130,8 +146,9 @@ constexpr int kMaxSegments = 1024;
 // re-scoring of samples the BF16 path left undecided.  Item p of the
 // concatenated queue lives in the segment g with off[g] <= p < off[g + 1].
 template <int NT, int KS, int S, bool FULL, typename I, bool UPDATE,
-          bool STORE_FLUSH, bool GATHER = false>
+          bool STORE_FLUSH, bool GATHER = false, bool ROWS = false>
 __global__ void __launch_bounds__(NT) mfma_lloyd_krn(FastArgs a) {
+  static_assert(!ROWS || (!UPDATE && !GATHER), "rows: labels only");
   // an iteration enqueued ahead of a relocation: nothing to compute
   if (a.skip != nullptr && *a.skip != 0) return;
   constexpr int kWavesPerBlock = NT / kWave;
@@ -234,7 +251,10 @@ __global__ void __launch_bounds__(NT) mfma_lloyd_krn(FastArgs a) {
   float xn[KS][S], wn[S];
   auto prefetch = [&](int64_t b) {
     const int64_t pf = b * kSuper + (int64_t)S * col;
-    load_x<KS, S, FULL>(X, n, d, pf, half, vec, xn);
+    if constexpr (ROWS)
+      load_rows<KS, S, FULL>(X, n, d, pf, half, xn);
+    else
+      load_x<KS, S, FULL>(X, n, d, pf, half, vec, xn);
 #pragma unroll
     for (int q = 0; q < S; ++q)
       wn[q] = (UPDATE && pf + q < n) ? __builtin_nontemporal_load(w + pf + q) : 0.f;
@@ -1300,6 +1320,57 @@ void launch_fast_assign(int64_t n, int64_t d, int64_t k, const T *X,
   } else {
     throw RuntimeError("MFMA assignment is FP32 only");
   }
+}
+
+// ---- labels of sample-major rows -------------------------------------------
+
+namespace {
+KernFn pick_rows(int64_t d) {
+  const int ks = ks_bucket(d);
+  const bool full = (d == 2 * ks);
+#define KMD_KS_CASE(KS)                                                          \
+  case KS:                                                                       \
+    return full ? &mfma_lloyd_krn<kThreads, KS, kS, true, int32_t, false, false, \
+                                  false, true>                                   \
+                : &mfma_lloyd_krn<kThreads, KS, kS, false, int32_t, false, false, \
+                                  false, true>;
+  switch (ks) {
+    KMD_KS_CASE(2)
+    KMD_KS_CASE(4)
+    KMD_KS_CASE(8)
+    KMD_KS_CASE(12)
+    KMD_KS_CASE(16)
+    KMD_KS_CASE(24)
+    KMD_KS_CASE(32)
+    default:
+      return nullptr;
+  }
+#undef KMD_KS_CASE
+}
+}  // namespace
+
+bool fast_assign_rows_supported(int64_t d, int64_t k) {
+  return d >= 1 && d <= kMaxD && k >= 1 && k <= (1 << 20) &&
+         lds_bytes(d, k, false) <= kLdsPerCu;
+}
+
+void launch_fast_assign_rows(int64_t n, int64_t d, int64_t k, const float *X,
+                             const float *C, const float *hn, int32_t *labels,
+                             hipStream_t s) {
+  if (n <= 0) return;
+  require(fast_assign_rows_supported(d, k), "row assignment: unsupported shape");
+  MfmaLaunch L;
+  L.fn = pick_rows(d);
+  L.lds = lds_bytes(d, k, false);
+  allow_full_lds(reinterpret_cast<const void *>(L.fn));
+  const int per_cu = std::max(
+      1, blocks_per_cu(reinterpret_cast<const void *>(L.fn), L.threads, L.lds));
+  L.blocks = (int)std::min<int64_t>(
+      (int64_t)device_cu_count() * per_cu,
+      ceil_div<int64_t>(ceil_div<int64_t>(n, 32 * kS), L.threads / kWave));
+  FastArgs a = make_args(n, d, k, X, nullptr, C, hn, labels);
+  a.n_copies = 1;
+  run(L, a, s);
 }
 
 // ---- FP32 re-score of queued samples (mixed-precision path) ---------------

@@ -85,6 +85,12 @@ template <typename T, typename I>
 void launch_fast_assign(int64_t n, int64_t d, int64_t k, const T *X,
                         const T *C, const T *hn, I *labels, hipStream_t s);
 
+// The same labels (int32) from sample-major X (n, d).
+bool fast_assign_rows_supported(int64_t d, int64_t k);
+void launch_fast_assign_rows(int64_t n, int64_t d, int64_t k, const float *X,
+                             const float *C, const float *hn, int32_t *labels,
+                             hipStream_t s);
+
 // Fixed-point scales of the MFMA update: scale[f] = 2^E_f (f < d) and
 // scale[d] = 2^E_w such that max|w| max|x_f| 2^E_f < 2^30 (one element fits
 // an int32) and n max|w| max|x_f| 2^E_f < 2^61 (the sum fits an int64);
@@ -196,6 +202,11 @@ void launch_tiled_assign(int64_t n, int64_t d, int64_t k, const float *X_t,
                          void *tiles_scratch = nullptr);
 // The reference fused step's accumulate-into update from given labels
 // (FP32 sums, LDS-privatised per feature group), for the tiled shapes
+// The same labels (int32) from sample-major X (n, d); tiles: the prepared
+// centroid tiles' buffer, tiled_tiles_bytes(d, k) bytes.
+void launch_tiled_assign_rows(int64_t n, int64_t d, int64_t k, const float *X,
+                              const float *C, const float *hn, int32_t *labels,
+                              void *tiles, hipStream_t s);
 template <typename I>
 void launch_label_update(int64_t n, int64_t d, int64_t k, int64_t n_copies,
                          const float *X_t, const float *w, const I *labels,

@@ -98,7 +98,7 @@ constexpr int fp32_s() {
 struct TiledArgs {
   int64_t n;
   int d, k, n_ct;
-  const float *X;      // X_t (d, n); gather mode: X_r (n, d)
+  const float *X;      // X_t (d, n); gather and rows modes: X_r (n, d)
   const float *tiles;  // [n_ct][tile_floats] in the LDS layout (+1 KB pad)
   void *labels;
   const int *queue, *queue_counts;  // gather mode
@@ -112,7 +112,8 @@ struct TiledArgs {
 // Tile layout in LDS: element (ks, half, col) = C[2 ks + half][tile*32 + col]
 // at ((ks / 4) * 2 + half) * 128 + col * 4 + ks % 4, so each lane reads four
 // k-steps with one 16-byte load; then the 32 half norms (+inf padded).
-template <int KS, typename I, bool GATHER>
+// ROWS: every sample in turn, read from sample-major X (n, d).
+template <int KS, typename I, bool GATHER, bool ROWS = false>
 __global__ void __launch_bounds__(kTNT) tiled_fp32_krn(TiledArgs a) {
   // an iteration enqueued ahead of a relocation: nothing to compute
   if (a.skip != nullptr && *a.skip != 0) return;
@@ -157,7 +158,7 @@ __global__ void __launch_bounds__(kTNT) tiled_fp32_krn(TiledArgs a) {
   const int64_t n_super = ceil_div<int64_t>(n_items, kSuper);
   const int64_t per_round = (int64_t)gridDim.x * kTW;
   const int64_t rounds = ceil_div<int64_t>(n_super, per_round);
-  const bool vec = !GATHER && S == 2 &&
+  const bool vec = !GATHER && !ROWS && S == 2 &&
                    ((reinterpret_cast<uintptr_t>(a.X) & 7u) == 0) && (n % 2 == 0);
 
   // centroid chunks stream through two LDS buffers: chunk g + 1 is copied
@@ -192,7 +193,7 @@ __global__ void __launch_bounds__(kTNT) tiled_fp32_krn(TiledArgs a) {
       }
     }
     float xr[KS][S];
-    if (GATHER) {
+    if (GATHER || ROWS) {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         const int f = 2 * ks + half;
@@ -1539,9 +1540,10 @@ auto with_ks(int64_t d, F &&f) {
   }
 }
 
-template <typename I, bool GATHER>
+template <typename I, bool GATHER, bool ROWS = false>
 TiledFn pick_fp32(int64_t d) {
-  return with_ks(d, [](auto ks) -> TiledFn { return &tiled_fp32_krn<ks(), I, GATHER>; });
+  return with_ks(
+      d, [](auto ks) -> TiledFn { return &tiled_fp32_krn<ks(), I, GATHER, ROWS>; });
 }
 
 }  // namespace
@@ -1679,33 +1681,50 @@ void launch_transpose(int64_t n, int64_t d, const float *X_t, float *X_r,
   KMD_LAUNCH_CHECK();
 }
 
-template <typename I>
-void launch_tiled_assign(int64_t n, int64_t d, int64_t k, const float *X_t,
-                         const float *C, const float *hn, I *labels,
-                         hipStream_t s, const int *skip, void *tiles_scratch) {
-  if (n <= 0) return;
+namespace {
+template <typename I, bool ROWS>
+void tiled_assign(int64_t n, int64_t d, int64_t k, const float *X, const float *C,
+                  const float *hn, I *labels, float *tiles, hipStream_t s,
+                  const int *skip) {
   require(tiled_supported(d, k), "tiled assignment: unsupported shape");
-  TiledFn fn = pick_fp32<I, false>(d);
+  TiledFn fn = pick_fp32<I, false, ROWS>(d);
   const size_t lds = fp32_lds_bytes(d, false);
   const int grid_max = occupancy_grid(fn, lds);
   if (grid_max < 1) throw RuntimeError("tiled assignment: no launch plan");
   const int S = ks_of(d) <= 32 ? 2 : 1;
   const int64_t need = ceil_div<int64_t>(ceil_div<int64_t>(n, 32 * S), kTW);
   const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>(grid_max, need));
-  TempBuffer own(tiles_scratch ? 0 : tiled_tiles_bytes(d, k), s);
-  float *tiles = tiles_scratch ? static_cast<float *>(tiles_scratch) : own.as<float>();
   prep_fp32_tiles_into(d, k, C, hn, tiles, s);
   TiledArgs a{};
   a.n = n;
   a.d = (int)d;
   a.k = (int)k;
   a.n_ct = (int)ceil_div<int64_t>(k, 32);
-  a.X = X_t;
+  a.X = X;
   a.tiles = tiles;
   a.labels = labels;
   a.skip = skip;
   hipLaunchKernelGGL(fn, dim3(blocks), dim3(kTNT), lds, s, a);
   KMD_LAUNCH_CHECK();
+}
+}  // namespace
+
+template <typename I>
+void launch_tiled_assign(int64_t n, int64_t d, int64_t k, const float *X_t,
+                         const float *C, const float *hn, I *labels,
+                         hipStream_t s, const int *skip, void *tiles_scratch) {
+  if (n <= 0) return;
+  TempBuffer own(tiles_scratch ? 0 : tiled_tiles_bytes(d, k), s);
+  float *tiles = tiles_scratch ? static_cast<float *>(tiles_scratch) : own.as<float>();
+  tiled_assign<I, false>(n, d, k, X_t, C, hn, labels, tiles, s, skip);
+}
+
+void launch_tiled_assign_rows(int64_t n, int64_t d, int64_t k, const float *X,
+                              const float *C, const float *hn, int32_t *labels,
+                              void *tiles, hipStream_t s) {
+  if (n <= 0) return;
+  tiled_assign<int32_t, true>(n, d, k, X, C, hn, labels, static_cast<float *>(tiles), s,
+                              nullptr);
 }
 
 namespace {

@@ -799,6 +799,52 @@ std::pair<Event, Event> py_transpose(py::object src_, py::object dst_,
   return record(s, has_shift ? keep_of({&src, &dst, &shift}) : keep_of({&src, &dst}));
 }
 
+std::pair<Event, Event> py_row_distances(py::object X_, py::object C_, py::object scratch_,
+                                         py::object D_, py::object q) {
+  kmd_stream_t s = resolve_stream(q);
+  Arr X = to_arr(X_, s, "X"), C = to_arr(C_, s, "centers"),
+      scratch = to_arr(scratch_, s, "scratch"), D = to_arr(D_, s, "distances");
+  if (X.ndim != 2 || C.ndim != 2 || D.ndim != 2 || scratch.ndim != 1)
+    throw py::value_error("X, centers and distances must be matrices, scratch a vector");
+  std::vector<const Arr *> all = {&X, &C, &scratch, &D};
+  if (!all_contig(all)) throw py::value_error("All input arrays must be C-contiguous");
+  if (!same_device(all)) throw py::value_error(kQueueMsg);
+  if (!X.is_float() || !X.same_type(C) || !X.same_type(D) || !X.same_type(scratch))
+    throw py::value_error("All arrays must share a float dtype");
+  const int64_t need = kmd_row_distances_scratch(X.dtype(), X.dim(1), C.dim(0));
+  if (C.dim(1) != X.dim(1) || D.dim(0) != X.dim(0) || D.dim(1) != C.dim(0) ||
+      scratch.dim(0) < need)
+    throw py::value_error("Array dimensions are not consistent");
+  use_device(X);
+  check_rc(kmd_row_distances(X.dtype(), X.dim(0), X.dim(1), C.dim(0), X.data, C.data,
+                             scratch.data, D.data, s));
+  return record(s, keep_of({&X, &C, &scratch, &D}));
+}
+
+std::pair<Event, Event> py_assign_rows(py::object X_, py::object C_, py::object scratch_,
+                                       py::object lab_, py::object q) {
+  kmd_stream_t s = resolve_stream(q);
+  Arr X = to_arr(X_, s, "X"), C = to_arr(C_, s, "centers"),
+      scratch = to_arr(scratch_, s, "scratch"), lab = to_arr(lab_, s, "labels");
+  if (X.ndim != 2 || C.ndim != 2 || lab.ndim != 1 || scratch.ndim != 1)
+    throw py::value_error("X and centers must be matrices, scratch and labels vectors");
+  std::vector<const Arr *> all = {&X, &C, &scratch, &lab};
+  if (!all_contig(all)) throw py::value_error("All input arrays must be C-contiguous");
+  if (!same_device(all)) throw py::value_error(kQueueMsg);
+  if (!X.is_float() || X.bits != 32 || !X.same_type(C) || !X.same_type(scratch) ||
+      !lab.is_int() || lab.bits != 32)
+    throw py::value_error("X, centers and scratch must be float32, labels int32");
+  const int64_t need = kmd_assign_rows_scratch(X.dim(1), C.dim(0));
+  if (C.dim(1) != X.dim(1) || lab.dim(0) != X.dim(0) || scratch.dim(0) * 4 < need)
+    throw py::value_error("Array dimensions are not consistent");
+  use_device(X);
+  check_rc(kmd_assign_rows(X.dim(0), X.dim(1), C.dim(0),
+                           static_cast<const float *>(X.data),
+                           static_cast<const float *>(C.data), scratch.data,
+                           static_cast<int32_t *>(lab.data), s));
+  return record(s, keep_of({&X, &C, &scratch, &lab}));
+}
+
 std::pair<Event, Event> py_gather_columns(py::object X_, py::object idx_,
                                           py::object out_, py::object q,
                                           py::list depends) {
@@ -1317,6 +1363,13 @@ PYBIND11_MODULE(_kmeans_dpcpp_amd, m) {
         "dst = src.T - shift (shift: float64 per column of src, or None).",
         py::arg("src"), py::arg("dst"), py::arg("shift") = py::none(),
         py::arg("sycl_queue") = py::none(), py::arg("depends") = py::list());
+  m.def("_row_distances_scratch",
+        [](bool f64, int64_t d, int64_t k) {
+          return kmd_row_distances_scratch(f64 ? KMD_F64 : KMD_F32, d, k);
+        });
+  m.def("_row_distances", &py_row_distances);
+  m.def("_assign_rows_scratch", &kmd_assign_rows_scratch);
+  m.def("_assign_rows", &py_assign_rows);
   m.def("gather_columns", &py_gather_columns,
         "gather_columns(X_t, indices, out_t, sycl_queue=None, depends=[]): "
         "out_t[:, j] = X_t[:, indices[j]] (indices int64 on the device).",

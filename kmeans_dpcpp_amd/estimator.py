@@ -306,7 +306,7 @@ class KMeans:
             out.append((lab, res, it, float(inertia)))
         return out
 
-    def _prep_predict(self, X):
+    def _check_predict(self, X):
         torch = _torch()
         if not hasattr(self, "_centers_dev"):
             raise RuntimeError("This KMeans instance is not fitted yet")
@@ -316,11 +316,18 @@ class KMeans:
         if Xd.ndim != 2 or Xd.shape[1] != C.shape[1]:
             raise ValueError(f"X has {Xd.shape[-1]} features, but KMeans is expecting "
                              f"{C.shape[1]} features as input.")
-        q = torch.cuda.current_stream(dev)
+        return Xd, host, torch.cuda.current_stream(dev)
+
+    def _transposed(self, Xd, q):
+        """Feature-major samples and centres."""
         n, d = Xd.shape
-        X_t = torch.empty((d, n), dtype=Xd.dtype, device=dev)
+        X_t = _torch().empty((d, n), dtype=Xd.dtype, device=Xd.device)
         _native.transpose(Xd, X_t, None, q)
-        C_t = C.t().contiguous()
+        return X_t, self._centers_dev.t().contiguous()
+
+    def _prep_predict(self, X):
+        Xd, host, q = self._check_predict(X)
+        X_t, C_t = self._transposed(Xd, q)
         return X_t, C_t, host, q
 
     def _labels(self, X_t, C_t, q):
@@ -333,8 +340,18 @@ class KMeans:
         return lab
 
     def predict(self, X, sample_weight=None):
-        X_t, C_t, host, q = self._prep_predict(X)
-        lab = self._labels(X_t, C_t, q)
+        torch = _torch()
+        Xd, host, q = self._check_predict(X)
+        C = self._centers_dev
+        scratch = (_native._assign_rows_scratch(C.shape[1], C.shape[0])
+                   if C.dtype == torch.float32 else 0)
+        if scratch > 0:
+            # straight from the rows
+            lab = torch.empty(Xd.shape[0], dtype=torch.int32, device=Xd.device)
+            buf = torch.empty((scratch + 3) // 4, dtype=torch.float32, device=Xd.device)
+            _native._assign_rows(Xd, C, buf, lab, q)
+        else:
+            lab = self._labels(*self._transposed(Xd, q), q)
         return lab.cpu().numpy() if host else lab
 
     def fit_predict(self, X, y=None, sample_weight=None):
@@ -353,13 +370,21 @@ class KMeans:
 
     def transform(self, X):
         torch = _torch()
-        X_t, C_t, host, q = self._prep_predict(X)
-        d, n = X_t.shape
-        k = C_t.shape[1]
-        D = torch.empty((k, n), dtype=X_t.dtype, device=X_t.device)
-        _native.compute_centroid_to_sample_distances(X_t, C_t, D, 128, 32, q)
-        out = torch.empty((n, k), dtype=X_t.dtype, device=X_t.device)
-        _native.transpose(D, out, None, q)
+        Xd, host, q = self._check_predict(X)
+        C = self._centers_dev
+        n, d = Xd.shape
+        k = C.shape[0]
+        scratch = _native._row_distances_scratch(C.dtype == torch.float64, d, k)
+        out = torch.empty((n, k), dtype=Xd.dtype, device=Xd.device)
+        if scratch > 0:
+            # straight from the rows to the (n, k) result
+            pad = torch.empty(scratch, dtype=Xd.dtype, device=Xd.device)
+            _native._row_distances(Xd, C, pad, out, q)
+        else:
+            X_t, C_t = self._transposed(Xd, q)
+            D = torch.empty((k, n), dtype=Xd.dtype, device=Xd.device)
+            _native.compute_centroid_to_sample_distances(X_t, C_t, D, 128, 32, q)
+            _native.transpose(D, out, None, q)
         return out.cpu().numpy() if host else out
 
     def fit_transform(self, X, y=None, sample_weight=None):
