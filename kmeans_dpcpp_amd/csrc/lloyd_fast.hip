@@ -156,7 +156,8 @@ __global__ void __launch_bounds__(NT) mfma_lloyd_krn(FastArgs a) {
   // where the sample operands leave room for 16 more without spilling (not
   // beside the binade-window sums of the atomic-flush form).
   constexpr bool kKeepTile =
-      KS * S <= 16 && (FULL || KS * S <= 12) && !(UPDATE && !STORE_FLUSH);
+      UPDATE ? KS * S <= 16 && (FULL || KS * S <= 12) && STORE_FLUSH
+             : KS * S <= (ROWS ? 24 : 16);
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int64_t n = a.n;
   const int d = a.d, k = a.k, kpad = a.kpad;

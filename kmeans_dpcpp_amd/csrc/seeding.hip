@@ -43,6 +43,36 @@ constexpr int kMaxTrials = 16;
 
 __device__ inline int lane_of() { return threadIdx.x & (kWave - 1); }
 
+// v of another lane of the same 16, by a register move (an LDS exchange, which
+// __shfl is, costs a trip through the CU's one LDS: 72 per wave of them were
+// a tenth of a scoring pass).
+template <int CTRL>
+__device__ inline double dpp(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+// Sum over each 16 lanes in the order of exchanges with lane ^ 1, 2, 4, 8
+// (equal values within the lanes already summed make a mirror as good as an
+// exchange).
+__device__ inline double sum16(double v) {
+  v += dpp<0xB1>(v);     // quad_perm [1,0,3,2]
+  v += dpp<0x4E>(v);     // quad_perm [2,3,0,1]
+  v += dpp<0x141>(v);    // row_half_mirror
+  v += dpp<0x140>(v);    // row_mirror
+  return v;
+}
+// Sum over the wave in the order of exchanges with lane ^ 32, 16, 8, 4, 2, 1.
+__device__ inline double sum64(double v) {
+  v += __shfl_xor(v, 32, kWave);
+  v += __shfl_xor(v, 16, kWave);
+  v += dpp<0x128>(v);    // row_ror:8
+  v += dpp<0x124>(v);    // row_ror:4
+  v += dpp<0x4E>(v);
+  v += dpp<0xB1>(v);
+  return v;
+}
+
 // ---- per-feature mean and variance -----------------------------------------
 // Block (x, y) covers features [y FC, y FC + FC) (FC = min(d, 256)) of rows
 // x P + r, r < P = 256 / FC, striding over rows by gridDim.x P.
@@ -78,15 +108,36 @@ __global__ void __launch_bounds__(kNT)
   }
 }
 
-// out[f] = sum over blocks of part[b][f] / n
+// out[f] = sum over blocks of part[b][f] / n: 16 features per block, 16
+// thread groups over the blocks' sums, then the groups' sums in order (one
+// thread per feature walking up to 1024 sums took 0.24 ms, this form 8 us).
+constexpr int kFinF = 16, kFinG = kNT / kFinF;
+
 __global__ void __launch_bounds__(kNT)
-    col_finish_krn(int64_t n, int64_t d, int64_t nblk, const double *part,
-                   double *out) {
-  const int64_t f = (int64_t)blockIdx.x * kNT + threadIdx.x;
-  if (f >= d) return;
+    col_finish_krn(int64_t n, int64_t d, int64_t nblk, const double *__restrict__ part,
+                   double *__restrict__ out) {
+  __shared__ double red[kFinG][kFinF];
+  const int e = threadIdx.x % kFinF, g = threadIdx.x / kFinF;
+  const int64_t f = (int64_t)blockIdx.x * kFinF + e;
   double s = 0.0;
-  for (int64_t b = 0; b < nblk; ++b) s += part[b * d + f];
-  out[f] = n > 0 ? s / (double)n : 0.0;
+  if (f < d) {
+    int64_t b = g;
+    for (; b + 7 * kFinG < nblk; b += 8 * kFinG) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = part[(b + u * kFinG) * d + f];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += v[u];
+    }
+    for (; b < nblk; b += kFinG) s += part[b * d + f];
+  }
+  red[g][e] = s;
+  __syncthreads();
+  if (g == 0 && f < d) {
+    double t = 0.0;
+    for (int i = 0; i < kFinG; ++i) t += red[i][e];
+    out[f] = n > 0 ? t / (double)n : 0.0;
+  }
 }
 
 // ---- transpose with per-column shift ----------------------------------------
@@ -132,8 +183,8 @@ constexpr int kSub = 64;                  // samples per sub-segment
 constexpr int kSubPerSeg = kSeg / kSub;   // 32
 constexpr int kUF = 4;                    // feature rows loaded together
 constexpr int kStage = 4;                 // rows per LDS DMA stage (float)
-constexpr int kPickD = 1024;              // center features the pick keeps in LDS
 
+static_assert(kSub / kSPT == 16, "one sub-segment per 16 scoring lanes");
 static_assert(kSubPerSeg <= kWave, "one lane per sub-segment of a segment");
 static_assert(kSub == kWave, "one lane per sample of a sub-segment");
 
@@ -174,10 +225,11 @@ struct KppArgs {
   double *part2;              // [T][nsub] sub-segment sums of w m_t
   int64_t *cand;              // [T] candidates of the current center
   double *csq;                // [T + 1] |staged row|^2 of the last scoring pass
+  double *crow;               // [T + 1][d] staged rows of the last scoring pass
 };
 
 struct SearchLds {
-  double wtot[kPNT / kWave];  // wave totals, then their exclusive prefix
+  double wtot[kPNT / kWave];  // wave totals
   double r[kMaxTrials];
   double before[kMaxTrials];
   int seg[kMaxTrials];
@@ -200,9 +252,11 @@ __device__ inline double wave_incl_scan(double y, int lane) {
 // first reaching r from the segment's exclusive prefix (else its last);
 // inside that the 64 values, the first reaching r (else the last).  One
 // block; writes out[0 : nt].
-template <typename VF>
+// seg0: seg[tid] where a thread's range is one segment (nb <= kPNT), as the
+// caller already has it, else unused.
+template <int TT, typename VF>
 __device__ void pick_search(int64_t n, int64_t nb, int64_t nsub, const double *seg,
-                            const double *sub, VF value, int nt, bool right,
+                            double seg0, const double *sub, VF value, int nt, bool right,
                             int64_t *out, SearchLds &L) {
   const int tid = threadIdx.x, lane = lane_of(), wv = tid / kWave;
   const int64_t per = ceil_div<int64_t>(nb, kPNT);
@@ -211,9 +265,13 @@ __device__ void pick_search(int64_t n, int64_t nb, int64_t nsub, const double *s
   constexpr int kKeep = 8;              // range values kept in registers
   double keep[kKeep];
   double tsum = 0.0;
+  if (per == 1) {
 #pragma unroll
-  for (int q = 0; q < kKeep; ++q) {
-    keep[q] = (lo + q < hi) ? seg[lo + q] : 0.0;
+    for (int q = 0; q < kKeep; ++q) keep[q] = 0.0;
+    keep[0] = (lo < hi) ? seg0 : 0.0;
+  } else {
+#pragma unroll
+    for (int q = 0; q < kKeep; ++q) keep[q] = (lo + q < hi) ? seg[lo + q] : 0.0;
   }
 #pragma unroll
   for (int q = 0; q < kKeep; ++q)
@@ -225,24 +283,21 @@ __device__ void pick_search(int64_t n, int64_t nb, int64_t nsub, const double *s
   if (lane == kWave - 1) L.wtot[wv] = y;
   if (tid < nt) L.seg[tid] = INT32_MAX;
   __syncthreads();
-  if (tid == 0) {                                   // exclusive wave prefix
-    double run = 0.0;
-    for (int i = 0; i < kPNT / kWave; ++i) {
-      const double t = L.wtot[i];
-      L.wtot[i] = run;
-      run += t;
-    }
-  }
-  __syncthreads();
-  int found[kMaxTrials];
-  double bef[kMaxTrials], rj[kMaxTrials];
+  double wbefore = 0.0;                             // waves before this one
 #pragma unroll
-  for (int j = 0; j < kMaxTrials; ++j) {
+  for (int i = 0; i < kPNT / kWave - 1; ++i) {
+    const double t = L.wtot[i];
+    wbefore = i < wv ? wbefore + t : wbefore;
+  }
+  int found[TT];
+  double bef[TT], rj[TT];
+#pragma unroll
+  for (int j = 0; j < TT; ++j) {
     found[j] = INT32_MAX;
     bef[j] = 0.0;
     rj[j] = (j < nt) ? L.r[j] : 0.0;
   }
-  double run = L.wtot[wv] + yp;                     // prefix before this range
+  double run = wbefore + yp;                        // prefix before this range
   for (int64_t s = lo; s < hi; ++s) {
     double v = 0.0;
 #pragma unroll
@@ -250,7 +305,7 @@ __device__ void pick_search(int64_t n, int64_t nb, int64_t nsub, const double *s
       if (s == lo + q) v = keep[q];
     const double nxt = run + ((s < lo + kKeep) ? v : seg[s]);
 #pragma unroll
-    for (int j = 0; j < kMaxTrials; ++j) {
+    for (int j = 0; j < TT; ++j) {
       const bool hit = right ? (nxt > rj[j]) : (nxt >= rj[j]);
       if (j < nt && hit && found[j] == INT32_MAX) {
         found[j] = (int)s;
@@ -259,12 +314,18 @@ __device__ void pick_search(int64_t n, int64_t nb, int64_t nsub, const double *s
     }
     run = nxt;
   }
+  // ranges ascend with the lane, so a wave's first hit is its smallest: one
+  // atomic per wave and target.  (Every thread past the draw has a hit; an
+  // atomic from each of them on one LDS word took 10 us of the search's 16.)
 #pragma unroll
-  for (int j = 0; j < kMaxTrials; ++j)
-    if (j < nt && found[j] != INT32_MAX) atomicMin(&L.seg[j], found[j]);
+  for (int j = 0; j < TT; ++j) {
+    const unsigned long long hits = __ballot(found[j] != INT32_MAX);
+    if (j < nt && hits != 0 && lane == __ffsll((long long)hits) - 1)
+      atomicMin(&L.seg[j], found[j]);
+  }
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < kMaxTrials; ++j)
+  for (int j = 0; j < TT; ++j)
     if (j < nt && found[j] != INT32_MAX && found[j] == L.seg[j]) L.before[j] = bef[j];
   __syncthreads();
   for (int j = wv; j < nt; j += kPNT / kWave) {    // one wave per target
@@ -334,8 +395,9 @@ __global__ void __launch_bounds__(kPNT) kpp_first_pick_krn(KppArgs a) {
     for (int i = 0; i < kPNT / kWave; ++i) tot += lds[i];
     L.r[0] = a.u[0] * tot;
   }
-  pick_search(a.n, a.nb, a.nsub, a.part, a.part2,
-              [&](int64_t i) { return (double)w[i]; }, 1, true, a.cand, L);
+  const double seg0 = threadIdx.x < a.nb ? a.part[threadIdx.x] : 0.0;
+  pick_search<1>(a.n, a.nb, a.nsub, a.part, seg0, a.part2,
+                 [&](int64_t i) { return (double)w[i]; }, 1, true, a.cand, L);
 }
 
 // Squared distance in the scoring pass's arithmetic: |x|^2 + |c|^2 - 2 x.c
@@ -347,9 +409,13 @@ __device__ inline double kpp_dist(double xsq, double csq, double xc) {
 }
 
 // One center, scoring pass (pure streaming; the pick is the next launch).
-// cache-policy operand of the LDS-DMA row loads: non-temporal (X is read
-// once per center and is larger than the caches; D^2 is what is reused)
+// Cache-policy operand of the LDS-DMA row loads: non-temporal where X, read
+// once per center, is larger than the caches (D^2 is then what is reused).
 constexpr int kLoadNT = 2;
+// An X up to this size is kept: the 256 MB last-level cache holds it beside
+// the two D^2 arrays from one center to the next (128 MB, n = 1,000,000, d =
+// 32: 32.8 us per pass against 34.4 us non-temporal).
+constexpr int64_t kCachedX = int64_t(160) << 20;
 
 // Row 0 of the staged points is center c - 1 (the first center when
 // c == 0): D^2 <- min(D^2, dist0) is written to d2[c & 1].  Rows 1..T are
@@ -410,7 +476,9 @@ __global__ void __launch_bounds__(kSNT, 4) kpp_score_krn(KppArgs a, int c, int64
     for (int e = threadIdx.x; e < (TT + 1) * fcn; e += kSNT) {
       const int r = e / fcn, f = e % fcn;
       const int64_t src = (r == 0) ? idx0 : ((r < rows) ? a.cand[r - 1] : -1);
-      cl[r * kFC + f] = (src >= 0) ? (double)X[(f0 + f) * n + src] : 0.0;
+      const double v = (src >= 0) ? (double)X[(f0 + f) * n + src] : 0.0;
+      cl[r * kFC + f] = v;
+      if (blk == 0 && r < rows) a.crow[r * d + f0 + f] = v;   // for the pick
     }
     __syncthreads();
     if (threadIdx.x <= TT) {    // |c|^2 of each staged row, features ascending
@@ -426,6 +494,7 @@ __global__ void __launch_bounds__(kSNT, 4) kpp_score_krn(KppArgs a, int c, int64
         // rows by LDS DMA (global_load_lds_dwordx4): the next stage of
         // kStage rows is in flight while the current one is scored, with no
         // registers held for it; a wave reads back only what it loaded
+        // (four stages of two rows, three in flight: no faster)
         const int wv = threadIdx.x / kWave, ln = lane_of();
         // lanes past n (ragged last segment) copy the row's last 4 samples
         // instead: in bounds and 16-byte aligned (n % 4 == 0); their
@@ -435,6 +504,7 @@ __global__ void __launch_bounds__(kSNT, 4) kpp_score_krn(KppArgs a, int c, int64
                              (s_lane + kSPT <= n ? s_lane : n - kSPT);
         float *lbase = xs + wv * (kWave * kSPT);
         const int ns = (fcn + kStage - 1) / kStage;
+        const bool cached = n * d * (int64_t)sizeof(float) <= kCachedX;
         auto issue = [&](int st) {
           float *buf = lbase + (st & 1) * (kStage * kSeg);
 #pragma unroll
@@ -442,10 +512,12 @@ __global__ void __launch_bounds__(kSNT, 4) kpp_score_krn(KppArgs a, int c, int64
             // always kStage copies (a short last stage repeats its last row),
             // so the vmcnt the reads wait for is a constant
             const int f = (st * kStage + r < fcn) ? st * kStage + r : fcn - 1;
-            __builtin_amdgcn_global_load_lds(
-                (const void *)(gbase + (int64_t)f * n),
-                (__attribute__((address_space(3))) void *)(buf + r * kSeg), 16, 0,
-                kLoadNT);
+            const void *from = (const void *)(gbase + (int64_t)f * n);
+            auto *to = (__attribute__((address_space(3))) void *)(buf + r * kSeg);
+            if (cached)
+              __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+            else
+              __builtin_amdgcn_global_load_lds(from, to, 16, 0, kLoadNT);
           }
         };
         issue(0);
@@ -556,7 +628,7 @@ __global__ void __launch_bounds__(kSNT, 4) kpp_score_krn(KppArgs a, int c, int64
         p += (i0 + j < n) ? wv[j] * mv : 0.0;
       }
       // sub-segment sum (16 lanes), then the wave sum
-      for (int o = 1; o < kSub / kSPT; o <<= 1) p += __shfl_xor(p, o, kWave);
+      p = sum16(p);
       if (sub_lead) a.part2[(int64_t)t * a.nsub + sb] = p;
       for (int o = kSub / kSPT; o < kWave; o <<= 1) p += __shfl_xor(p, o, kWave);
       if (lane_of() == 0) wsum[(threadIdx.x / kWave) * TT + t] = p;
@@ -574,88 +646,114 @@ __global__ void __launch_bounds__(kSNT, 4) kpp_score_krn(KppArgs a, int c, int64
 // next center's candidates.  One block.  The values w_i m_t*(i) the last
 // search level needs are recomputed for 64 samples per target with the
 // scoring pass's arithmetic (the pass does not store m).
-template <typename T>
+//
+// Nothing but latency: a chain of dependent reads, exchanges and barriers on
+// one CU.  So everything that does not depend on the winner is read at the
+// start (segment sums, the candidates' rows as the scoring pass staged them,
+// their indices, norms and the next draws), a search over at most kPNT
+// segments takes its values from registers, and the arrays are sized to the
+// trials (16 of each spilled): n = 1,000,000, d = 32, 6 trials: 10.2 us
+// per center, 28 us before.
+constexpr int kPickRows = 2048;   // candidate row values kept in LDS
+
+template <typename T, int TT>
 __global__ void __launch_bounds__(kPNT) kpp_pick_krn(KppArgs a, int c) {
-  __shared__ double red[kPNT / kWave][kMaxTrials];
+  __shared__ double red[kPNT / kWave][TT];
   __shared__ SearchLds L;
-  __shared__ double s_pot[kMaxTrials];
-  __shared__ double s_csq;
-  __shared__ int64_t s_idx;
-  __shared__ int s_ts;
-  __shared__ double s_c[kPickD];               // center c (d <= kPickD)
+  __shared__ double s_pot[TT], s_csq[TT + 1], s_u[TT];
+  __shared__ int64_t s_cand[TT];
+  __shared__ double s_row[kPickRows];          // the candidates' rows, or the winner's
   const T *X = static_cast<const T *>(a.X_t);
   const T *w = static_cast<const T *>(a.w);
   const int64_t n = a.n, d = a.d, k = a.k;
+  const int tid = threadIdx.x;
   const int ns = (c == 0) ? 1 : a.trials;
+  // candidate t's row of crow: row 0 is the first center (c == 0) or the
+  // previous one
+  const int row0 = (c == 0) ? 0 : 1;
+  const bool all_rows = ns * d <= kPickRows;
+  if (all_rows)
+    for (int i = tid; i < ns * d; i += kPNT) s_row[i] = a.crow[row0 * d + i];
+  if (tid < ns) s_cand[tid] = a.cand[tid];
+  if (tid <= ns) s_csq[tid] = a.csq[tid];
+  if (c + 1 < k && tid < a.trials) s_u[tid] = a.u[1 + (int64_t)c * a.trials + tid];
   // all potentials in one pass: per thread, each trial's segment sums in
   // ascending order; the ns loads of one segment are in flight together
-  double v[kMaxTrials];
+  double v[TT], first[TT];
 #pragma unroll
-  for (int t = 0; t < kMaxTrials; ++t) v[t] = 0.0;
-  for (int64_t b = threadIdx.x; b < a.nb; b += kPNT) {
-    double p[kMaxTrials];
+  for (int t = 0; t < TT; ++t) {
+    first[t] = (t < ns && tid < a.nb) ? a.part[(int64_t)t * a.nb + tid] : 0.0;
+    v[t] = first[t];
+  }
+  for (int64_t b = tid + kPNT; b < a.nb; b += kPNT) {
+    double p[TT];
 #pragma unroll
-    for (int t = 0; t < kMaxTrials; ++t) p[t] = (t < ns) ? a.part[(int64_t)t * a.nb + b] : 0.0;
+    for (int t = 0; t < TT; ++t) p[t] = (t < ns) ? a.part[(int64_t)t * a.nb + b] : 0.0;
 #pragma unroll
-    for (int t = 0; t < kMaxTrials; ++t)
+    for (int t = 0; t < TT; ++t)
       if (t < ns) v[t] += p[t];
   }
 #pragma unroll
-  for (int t = 0; t < kMaxTrials; ++t) {
-    double vt = v[t];
-    for (int o = kWave / 2; o > 0; o >>= 1) vt += __shfl_xor(vt, o, kWave);
-    if (lane_of() == 0) red[threadIdx.x / kWave][t] = vt;
+  for (int t = 0; t < TT; ++t) {
+    const double vt = sum64(v[t]);
+    if (lane_of() == 0) red[tid / kWave][t] = vt;
   }
   __syncthreads();
-  if ((int)threadIdx.x < ns) {
+  if (tid < ns) {
     double tot = 0.0;
-    for (int i = 0; i < kPNT / kWave; ++i) tot += red[i][threadIdx.x];
-    s_pot[threadIdx.x] = tot;
+#pragma unroll
+    for (int i = 0; i < kPNT / kWave; ++i) tot += red[i][tid];
+    s_pot[tid] = tot;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int ts = 0;
-    for (int t = 1; t < ns; ++t)
-      if (s_pot[t] < s_pot[ts]) ts = t;
-    s_ts = ts;
-    s_idx = a.cand[ts];
-    a.indices[c] = s_idx;
-    s_csq = a.csq[ts + 1];                     // |center c|^2 as the pass has it
+  int ts = 0;                                  // every thread for itself
+  double best = s_pot[0];
+#pragma unroll
+  for (int t = 1; t < TT; ++t) {
+    const double p = t < ns ? s_pot[t] : __builtin_inf();
+    if (t < ns && p < best) {
+      best = p;
+      ts = t;
+    }
   }
-  __syncthreads();
-  const int64_t idx = s_idx;
+  const int64_t idx = s_cand[ts];
+  const double ccsq = s_csq[ts + 1];           // |center c|^2 as the pass has it
+  if (tid == 0) a.indices[c] = idx;
   T *C = static_cast<T *>(a.centers_t);
-  for (int64_t f = threadIdx.x; f < d; f += kPNT) {
-    const T v = X[f * n + idx];
-    C[f * k + c] = v;
-    if (f < kPickD) s_c[f] = (double)v;
+  const double *crow = a.crow + (row0 + ts) * d;
+  const double *s_c = s_row + (all_rows ? ts * d : 0);   // features below n_lds
+  const int64_t n_lds = all_rows ? d : (d < kPickRows ? d : kPickRows);
+  for (int64_t f = tid; f < d; f += kPNT) {
+    const double cf = all_rows ? s_c[f] : crow[f];
+    C[f * k + c] = (T)cf;
+    if (!all_rows && f < kPickRows) s_row[f] = cf;
   }
+  if (c + 1 >= k) return;
+  if (tid < a.trials) L.r[tid] = s_u[tid] * best;
   __syncthreads();
-  if (c + 1 < k) {
-    const int ts = s_ts;
-    if ((int)threadIdx.x < a.trials)
-      L.r[threadIdx.x] = a.u[1 + (int64_t)c * a.trials + threadIdx.x] * s_pot[ts];
-    const double *dn = a.d2[c & 1];
-    const double ccsq = s_csq;
-    auto value = [&](int64_t i) {
-      double m = dn[i];
-      if (c != 0) {                            // min(D^2, |x_i - center c|^2)
-        double xsq = 0.0, xc = 0.0;
-#pragma unroll 16
-        for (int64_t f = 0; f < d; ++f) {
-          const double x = (double)X[f * n + i];
-          const double cf = (f < kPickD) ? s_c[f] : (double)X[f * n + idx];
-          xsq = fma(x, x, xsq);
-          xc = fma(x, cf, xc);
-        }
-        const double dd = kpp_dist(xsq, ccsq, xc);
-        m = (m <= dd) ? m : dd;
+  const double *dn = a.d2[c & 1];
+  auto value = [&](int64_t i) {
+    double m = dn[i];
+    const double wi = (double)w[i];
+    if (c != 0) {                              // min(D^2, |x_i - center c|^2)
+      double xsq = 0.0, xc = 0.0;
+#pragma unroll 32
+      for (int64_t f = 0; f < d; ++f) {
+        const double x = (double)X[f * n + i];
+        const double cf = (f < n_lds) ? s_c[f] : crow[f];
+        xsq = fma(x, x, xsq);
+        xc = fma(x, cf, xc);
       }
-      return (double)w[i] * m;
-    };
-    pick_search(n, a.nb, a.nsub, a.part + (int64_t)ts * a.nb,
-                a.part2 + (int64_t)ts * a.nsub, value, a.trials, false, a.cand, L);
-  }
+      const double dd = kpp_dist(xsq, ccsq, xc);
+      m = (m <= dd) ? m : dd;
+    }
+    return wi * m;
+  };
+  double seg0 = 0.0;
+#pragma unroll
+  for (int t = 0; t < TT; ++t) seg0 = t == ts ? first[t] : seg0;
+  pick_search<TT>(n, a.nb, a.nsub, a.part + (int64_t)ts * a.nb, seg0,
+                  a.part2 + (int64_t)ts * a.nsub, value, a.trials, false, a.cand, L);
 }
 
 template <typename T, int TT>
@@ -670,7 +768,10 @@ void launch_kpp_step(const KppArgs &a, int c, hipStream_t s) {
     hipLaunchKernelGGL((kpp_score_krn<T, TT, false>), dim3((unsigned)a.nb),
                        dim3(kSNT), 0, s, a, c, (int64_t)0);
   KMD_LAUNCH_CHECK();
-  hipLaunchKernelGGL(kpp_pick_krn<T>, dim3(1), dim3(kPNT), 0, s, a, c);
+  // (after the first center: TT trials' candidates; the first pick already
+  // searches for all of them)
+  hipLaunchKernelGGL((kpp_pick_krn<T, (TT > 1 ? TT : kMaxTrials)>), dim3(1), dim3(kPNT), 0,
+                     s, a, c);
   KMD_LAUNCH_CHECK();
 }
 
@@ -689,7 +790,7 @@ void launch_column_mean_var(int64_t n, int64_t d, const T *X, double *mean,
   if (gx > cap) gx = cap > 0 ? cap : 1;
   TempBuffer part((size_t)(gx * d) * sizeof(double), s);
   const dim3 grid((unsigned)gx, (unsigned)gy);
-  const unsigned fb = (unsigned)ceil_div<int64_t>(d, kNT);
+  const unsigned fb = (unsigned)ceil_div<int64_t>(d, kFinF);
   hipLaunchKernelGGL(col_moment_krn<T>, grid, dim3(kNT), 0, s, n, d, X,
                      (const double *)nullptr, part.as<double>());
   KMD_LAUNCH_CHECK();
@@ -742,6 +843,7 @@ void launch_kmeans_plusplus(int64_t n, int64_t d, int64_t k, int trials,
   TempBuffer dbuf(2 * (size_t)n * sizeof(double), s);
   TempBuffer part((size_t)trials * (size_t)(nb + nsub) * sizeof(double), s);
   TempBuffer small(512, s);
+  TempBuffer crow((size_t)(trials + 1) * (size_t)d * sizeof(double), s);
   KppArgs a{};
   a.n = n; a.d = d; a.k = k; a.nb = nb; a.nsub = nsub; a.trials = trials;
   a.X_t = X_t; a.w = w; a.u = u_dev; a.centers_t = centers_t;
@@ -753,6 +855,7 @@ void launch_kmeans_plusplus(int64_t n, int64_t d, int64_t k, int trials,
   char *sm = small.as<char>();
   a.cand = reinterpret_cast<int64_t *>(sm);              // 16 x 8 bytes
   a.csq = reinterpret_cast<double *>(sm + 128);          // 17 x 8 bytes
+  a.crow = crow.as<double>();
   KMD_HIP_CHECK(hipMemsetAsync(sm, 0, 512, s));
   hipLaunchKernelGGL(kpp_wsum_krn<T>, dim3((unsigned)nb), dim3(kSNT), 0, s, a);
   KMD_LAUNCH_CHECK();

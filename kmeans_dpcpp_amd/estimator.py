@@ -266,7 +266,8 @@ class KMeans:
                 best = (labels, res, n_iter, inertia)
         labels, res, n_iter, inertia = best
         centers = (res.t() + mean.to(res.dtype)[None, :]).contiguous()   # (k, d)
-        distinct = torch.unique(labels).numel()
+        used = torch.zeros(k, dtype=torch.bool, device=labels.device)
+        distinct = int(used.scatter_(0, labels.to(torch.int64), True).sum())
         if distinct < k:
             warnings.warn(f"Number of distinct clusters ({distinct}) found smaller than "
                           f"n_clusters ({k}). Possibly due to duplicate points in X.",
