@@ -43,6 +43,17 @@
 
 namespace kmd {
 
+// A part of one allocation.
+struct Slice {
+  char *ptr = nullptr;
+  size_t size = 0;
+  template <typename U>
+  U *as() const {
+    return reinterpret_cast<U *>(ptr);
+  }
+  size_t bytes() const { return size; }
+};
+
 template <typename T, typename I>
 struct LloydWorkspace {
   int64_t n, d, k;
@@ -59,8 +70,11 @@ struct LloydWorkspace {
   // LDS-resident mixed path: undecided samples re-scored inside the kernel
   bool mixed_ink = false;
   FusedPlan plan;
-  TempBuffer hn, sizes, shifts, per_sample, copies, sizes_copies, list,
-      scalars, scales;
+  // one allocation for what every path has (a stream-ordered allocation and
+  // its release cost several microseconds of host time each)
+  TempBuffer arena{0, nullptr};
+  Slice hn, sizes, shifts, per_sample, copies, sizes_copies, list, scalars, scales;
+  Slice stats;   // of the fixed-point scales
   TempBuffer aop{0, nullptr}, bound{0, nullptr}, queue{0, nullptr},
       queue_counts{0, nullptr};
   TempBuffer xr{0, nullptr}, upd{0, nullptr};  // tiled: X sample-major, update scratch
@@ -70,23 +84,40 @@ struct LloydWorkspace {
   // `sums`: the undivided sums of the iteration (kept until the next one's
   // reduction, for the relocation of empty clusters); `scalars`: the loop's
   // state @0, an iteration's re-scored count @48, the epilogue's sum @56
-  TempBuffer sums, tail_part, tail_ticket;
+  Slice sums, tail_part, tail_ticket;
   // copies_bytes / sizes_bytes: private copies of the generic kernel, or the
   // fast path's per-block partials (in `copies`, sizes_bytes = 0)
   LloydWorkspace(int64_t n_, int64_t d_, int64_t k_, int blocks_, bool fast_,
                  bool store_, const FusedPlan &plan_, size_t copies_bytes,
                  size_t sizes_bytes, hipStream_t s)
       : n(n_), d(d_), k(k_), blocks(blocks_), fast(fast_), store_flush(store_),
-        plan(plan_), hn(sizeof(T) * k_, s), sizes(sizeof(T) * k_, s),
-        shifts(sizeof(T) * k_, s), per_sample(sizeof(T) * (n_ > 0 ? n_ : 1), s),
-        copies(copies_bytes, s), sizes_copies(sizes_bytes, s),
-        list(sizeof(I) * (k_ + 1), s), scalars(64, s),
-        scales(fast_ ? sizeof(float) * (d_ + 1) + 16 : 0, s),
-        sums(sizeof(T) * d_ * k_, s),
-        tail_part(sizeof(double) * step_tail_partials(k_), s),
-        tail_ticket(sizeof(unsigned), s) {
-    KMD_HIP_CHECK(hipMemsetAsync(tail_ticket.as<unsigned>(), 0, sizeof(unsigned), s));
-    KMD_HIP_CHECK(hipMemsetAsync(scalars.as<char>(), 0, scalars.bytes(), s));
+        plan(plan_) {
+    size_t used = 0;
+    auto take = [&](Slice &q, size_t bytes) {
+      q.ptr = reinterpret_cast<char *>(used);   // offset, until the base is known
+      q.size = bytes;
+      used += (bytes + 255) / 256 * 256;
+    };
+    Slice *const all[] = {&scalars, &tail_ticket, &hn,   &sizes,     &shifts, &list,
+                          &scales,  &stats,       &sums, &tail_part, &per_sample,
+                          &copies,  &sizes_copies};
+    take(scalars, 64);
+    take(tail_ticket, 64);
+    take(hn, sizeof(T) * k_);
+    take(sizes, sizeof(T) * k_);
+    take(shifts, sizeof(T) * k_);
+    take(list, sizeof(I) * (k_ + 1));
+    take(scales, fast_ ? sizeof(float) * (d_ + 1) + 16 : 0);
+    take(stats, fast_ ? fixed_point_stats_bytes(d_) : 0);
+    take(sums, sizeof(T) * d_ * k_);
+    take(tail_part, sizeof(double) * step_tail_partials(k_));
+    take(per_sample, sizeof(T) * (n_ > 0 ? n_ : 1));
+    take(copies, copies_bytes);
+    take(sizes_copies, sizes_bytes);
+    arena = TempBuffer(used, s);
+    for (Slice *q : all) q->ptr = arena.as<char>() + reinterpret_cast<size_t>(q->ptr);
+    // scalars and the ticket lie at the front
+    KMD_HIP_CHECK(hipMemsetAsync(arena.as<char>(), 0, 512, s));
   }
   LoopState *state() const { return scalars.as<LoopState>(); }
   const int *stop() const { return &state()->stop; }
@@ -148,7 +179,8 @@ static std::unique_ptr<LloydWorkspace<T, I>> make_mixed_workspace(
     ws->seg_cap = ink ? 0 : mixed_seg_cap(n, d, ba);
     ws->queue = TempBuffer(sizeof(int) * (size_t)ba * ws->seg_cap, s);
     ws->queue_counts = TempBuffer(sizeof(int) * (size_t)ba, s);
-    launch_fixed_point_scales(n, d, X, w, ws->scale(), ws->nonfinite(), s);
+    launch_fixed_point_scales(n, d, X, w, ws->scale(), ws->nonfinite(), s,
+                              ws->stats.template as<void>());
     int bad = 0;
     KMD_HIP_CHECK(hipMemcpyAsync(&bad, ws->nonfinite(), sizeof(int),
                                  hipMemcpyDeviceToHost, s));
@@ -180,7 +212,8 @@ static std::unique_ptr<LloydWorkspace<T, I>> make_tiled_workspace(
     auto ws = std::make_unique<LloydWorkspace<T, I>>(
         n, d, k, 1, true, true, FusedPlan{}, sizeof(int64_t) * (size_t)(d * k + k),
         0, s);
-    launch_fixed_point_scales(n, d, X, w, ws->scale(), ws->nonfinite(), s);
+    launch_fixed_point_scales(n, d, X, w, ws->scale(), ws->nonfinite(), s,
+                              ws->stats.template as<void>());
     int bad = 0;
     KMD_HIP_CHECK(hipMemcpyAsync(&bad, ws->nonfinite(), sizeof(int),
                                  hipMemcpyDeviceToHost, s));
@@ -326,7 +359,8 @@ static std::unique_ptr<LloydWorkspace<T, I>> make_workspace(int64_t n,
         sizeof(int64_t) * (size_t)blocks * (d * k + k), 0, s);
     // fixed-point scales: X and w do not change during the fit
     if constexpr (std::is_same<T, float>::value)
-      launch_fixed_point_scales(n, d, X, w, ws->scale(), ws->nonfinite(), s);
+      launch_fixed_point_scales(n, d, X, w, ws->scale(), ws->nonfinite(), s,
+                              ws->stats.template as<void>());
     return ws;
   }
   FusedPlan p = plan_generic_fused<T>(n, d, k);

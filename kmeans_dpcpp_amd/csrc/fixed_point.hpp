@@ -46,48 +46,65 @@ constexpr int kMaxWeightSpread = 13;
 // quantised (spreads above kMaxTypicalSpread / kMaxWeightSpread; estat may be
 // NULL to skip this test); else 0.  Kernels sum in floating point whenever
 // *flag != 0.
+// The scale of one row whose largest |w x_f| (or |w|) is m.
+__device__ inline float fixed_point_scale(int64_t n, double m) {
+  int e = 0;
+  if (m > 0.0 && m < 1e300) {
+    int ex_elem, ex_sum;
+    frexp(m, &ex_elem);                       // m < 2^ex_elem
+    frexp(m * (double)(n > 0 ? n : 1), &ex_sum);
+    const int e1 = 30 - ex_elem, e2 = 61 - ex_sum;
+    e = e1 < e2 ? e1 : e2;
+    e = e > 120 ? 120 : (e < -120 ? -120 : e);
+  }
+  return ldexpf(1.f, e);
+}
+
+// Binary orders of magnitude from the geometric mean of row f's normal values
+// to its largest.
+__device__ inline double fixed_point_spread(int f, const unsigned *maxbits,
+                                            const unsigned long long *estat) {
+  const unsigned long long cnt = estat[2 * f + 1];
+  if (cnt == 0) return 0.0;
+  const double mean_e = (double)estat[2 * f] / (double)cnt;
+  return (double)(maxbits[f] >> 23) - mean_e;
+}
+
+// *flag from what the rows gave: bad, any value not finite; sx, the largest
+// spread of a feature (estat != NULL).
+__device__ inline int fixed_point_flag(int d, bool bad, double sx, const unsigned *maxbits,
+                                       const unsigned long long *estat) {
+  if (bad) return 1;
+  bool coarse = false;
+  if (estat != nullptr) {
+    coarse |= sx + fixed_point_spread(d, maxbits, estat) > kMaxTypicalSpread;
+    const unsigned wmin_inv = maxbits[d + 1];
+    if (wmin_inv != 0u) {
+      const int emin = (int)((~wmin_inv & 0x7fffffffu) >> 23);
+      coarse |= (int)(maxbits[d] >> 23) - emin > kMaxWeightSpread;
+    }
+  }
+  return coarse ? 2 : 0;
+}
+
+// One thread.
 __device__ inline void fixed_point_scales_from_bits(
     int64_t n, int d, const unsigned *maxbits, const unsigned long long *estat,
     float *scale, int *flag) {
   const unsigned wb = maxbits[d];
-  int bad = wb >= 0x7f800000u;
+  bool bad = wb >= 0x7f800000u;
   const double wmax = (double)__uint_as_float(wb);
+  double sx = 0.0;
   for (int f = 0; f <= d; ++f) {
     const unsigned b = maxbits[f];
     bad |= b >= 0x7f800000u;
-    const double m = wmax * (f < d ? (double)__uint_as_float(b) : 1.0);
-    int e = 0;
-    if (m > 0.0 && m < 1e300) {
-      int ex_elem, ex_sum;
-      frexp(m, &ex_elem);                       // m < 2^ex_elem
-      frexp(m * (double)(n > 0 ? n : 1), &ex_sum);
-      const int e1 = 30 - ex_elem, e2 = 61 - ex_sum;
-      e = e1 < e2 ? e1 : e2;
-      e = e > 120 ? 120 : (e < -120 ? -120 : e);
-    }
-    scale[f] = ldexpf(1.f, e);
-  }
-  int coarse = 0;
-  if (estat != nullptr && !bad) {
-    auto spread = [&](int f) {
-      const unsigned long long cnt = estat[2 * f + 1];
-      if (cnt == 0) return 0.0;
-      const double mean_e = (double)estat[2 * f] / (double)cnt;
-      return (double)(maxbits[f] >> 23) - mean_e;
-    };
-    double sx = 0.0;
-    for (int f = 0; f < d; ++f) {
-      const double sf = spread(f);
+    scale[f] = fixed_point_scale(n, wmax * (f < d ? (double)__uint_as_float(b) : 1.0));
+    if (f < d && estat != nullptr) {
+      const double sf = fixed_point_spread(f, maxbits, estat);
       sx = sf > sx ? sf : sx;
     }
-    coarse |= sx + spread(d) > kMaxTypicalSpread;
-    const unsigned wmin_inv = maxbits[d + 1];
-    if (wmin_inv != 0u) {
-      const int emin = (int)((~wmin_inv & 0x7fffffffu) >> 23);
-      coarse |= (int)(wb >> 23) - emin > kMaxWeightSpread;
-    }
   }
-  flag[0] = bad ? 1 : (coarse ? 2 : 0);
+  flag[0] = fixed_point_flag(d, bad, sx, maxbits, estat);
 }
 
 // Exact binade-window sums (for the steps that run no pass over X for

@@ -917,11 +917,36 @@ __global__ void zero_words_krn(unsigned *words, int64_t count) {
     words[i] = 0u;
 }
 
-// Scales and flag from the statistics (fixed_point.hpp), one thread.
-__global__ void scales_krn(int64_t n, int d, const unsigned *maxbits,
-                           const unsigned long long *estat, float *scale,
-                           int *flag) {
-  fixed_point_scales_from_bits(n, d, maxbits, estat, scale, flag);
+// Scales and flag from the statistics (fixed_point.hpp), a thread per row (one
+// thread for all took 5 us at d = 16 and 30 us at d = 128, this form 3 us).
+__global__ void __launch_bounds__(256)
+    scales_krn(int64_t n, int d, const unsigned *maxbits,
+               const unsigned long long *estat, float *scale, int *flag) {
+  __shared__ double lds[256 / kWave];
+  __shared__ int any_bad;
+  if (threadIdx.x == 0) any_bad = 0;
+  __syncthreads();
+  const double wmax = (double)__uint_as_float(maxbits[d]);
+  double sx = 0.0;
+  for (int f = threadIdx.x; f <= d; f += 256) {
+    const unsigned b = maxbits[f];
+    if (b >= 0x7f800000u) any_bad = 1;
+    scale[f] = fixed_point_scale(n, wmax * (f < d ? (double)__uint_as_float(b) : 1.0));
+    if (f < d) {
+      const double sf = fixed_point_spread(f, maxbits, estat);
+      sx = sf > sx ? sf : sx;
+    }
+  }
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    const double t = __shfl_xor(sx, o, kWave);
+    sx = t > sx ? t : sx;
+  }
+  if ((threadIdx.x & (kWave - 1)) == 0) lds[threadIdx.x / kWave] = sx;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < 256 / kWave; ++i) sx = lds[i] > sx ? lds[i] : sx;
+    flag[0] = fixed_point_flag(d, any_bad != 0, sx, maxbits, estat);
+  }
 }
 
 // ---- launch planning -----------------------------------------------------
@@ -1221,7 +1246,7 @@ void launch_fixed_point_scales(int64_t n, int64_t d, const float *X,
                        0, s, n, (int)d, X, w, maxbits, estat);
     KMD_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(scales_krn, dim3(1), dim3(1), 0, s, n, (int)d, maxbits, estat,
+  hipLaunchKernelGGL(scales_krn, dim3(1), dim3(256), 0, s, n, (int)d, maxbits, estat,
                      scale, nonfinite);
   KMD_LAUNCH_CHECK();
 }
