@@ -187,8 +187,10 @@ void launch_inertia(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
 // once while stop != 0, so iterations can be enqueued ahead of the host's
 // knowledge of how the one before ended.
 constexpr int kLoopConverged = 1, kLoopEmpty = 2;
+// a one-block loop that left the fit to the kernels of one iteration each
+constexpr int kLoopRefused = 3;
 struct LoopState {
-  int stop;            // 0, kLoopConverged or kLoopEmpty
+  int stop;            // 0 or one of the above
   int pad;
   long long done;      // iterations finished
   long long n_empty;   // kLoopEmpty: clusters to relocate
@@ -198,6 +200,7 @@ struct LoopState {
 struct LoopHost {
   unsigned long long word;   // done * 4 + stop
   long long n_empty;         // valid when the word says kLoopEmpty
+  double total;              // a one-block fit's inertia, when it has ended
 };
 
 // Writes the state to host memory, the word after the rest (which only a loop

@@ -357,11 +357,7 @@ static std::unique_ptr<LloydWorkspace<T, I>> make_workspace(int64_t n,
     auto ws = std::make_unique<LloydWorkspace<T, I>>(
         n, d, k, blocks, true, true, FusedPlan{},
         sizeof(int64_t) * (size_t)blocks * (d * k + k), 0, s);
-    // fixed-point scales: X and w do not change during the fit
-    if constexpr (std::is_same<T, float>::value)
-      launch_fixed_point_scales(n, d, X, w, ws->scale(), ws->nonfinite(), s,
-                              ws->stats.template as<void>());
-    return ws;
+    return ws;   // its fixed-point scales: driver_impl
   }
   FusedPlan p = plan_generic_fused<T>(n, d, k);
   // features streamed through the matrix core: the same sums into the same
@@ -415,14 +411,14 @@ struct FusedTimer {
   void end(hipStream_t s) {
     if (on) KMD_HIP_CHECK(hipEventRecord(stop[slot], s));
   }
-  // the launch timed in slot i has finished
-  void collect(int i) {
+  // the launch timed in slot i, of `count` iterations, has finished
+  void collect(int i, int64_t count) {
     if (!on) return;
     float ms = 0.f;
     KMD_HIP_CHECK(hipEventSynchronize(stop[i]));
     KMD_HIP_CHECK(hipEventElapsedTime(&ms, start[i], stop[i]));
     total_ms += ms;
-    ++launches;
+    launches += count;
   }
 };
 
@@ -767,11 +763,62 @@ static void driver_impl(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
     tail.relocated = relocated ? 1 : 0;
     launch_step_tail<T, I>(tail, s);
   };
-  launch_half_l2_norm<T>(d, k, init, ws.hn.template as<T>(), s);
   // verbose mode prints between iterations: nothing is enqueued ahead there
   const int ahead = verbose ? 0 : kAhead;
-  while (it < max_iter) {
-    while (queued < max_iter && queued <= it + ahead) {
+  const bool resident = std::is_same<T, float>::value && ws.fast &&
+                        ws.mixed_terms == 0 && !ws.tiled;
+  auto finish = [&](double total, int64_t rescored) {
+    *inertia_out = static_cast<double>(static_cast<T>(total));
+    *n_iters_out = it;
+    if (stats) {
+      stats->fused_kernel_ms = timer.total_ms;
+      stats->fused_launches = timer.launches;
+      int path = ws.mixed_terms > 0 ? (ws.mixed_terms == 3 ? 3 : 2)
+                                    : (ws.fast ? 1 : 0);
+      if (ws.tiled) path += 3;  // 4 tiled FP32, 5 tiled BF16, 6 tiled BF16x3
+      if (ws.tiled && ws.mixed_terms == 8) path = 7;  // tiled FP8
+      stats->fused_path = path;
+      stats->n_rescored = rescored;
+    }
+  };
+  auto start = [&] {   // fixed-point scales (X and w stay as they are), half norms
+    if constexpr (std::is_same<T, float>::value) {
+      if (resident)
+        launch_fixed_point_scales(n, d, X, w, ws.scale(), ws.nonfinite(), s,
+                                  ws.stats.template as<void>());
+    }
+    launch_half_l2_norm<T>(d, k, init, ws.hn.template as<T>(), s);
+  };
+  // small fits: everything in one launch (up to a relocation)
+  bool one_block = resident && !verbose && small_loop_serves(n, d, k);
+  if (!one_block) start();
+  while (it < max_iter || one_block) {
+    if constexpr (std::is_same<T, float>::value) {
+      if (one_block) {
+        timer.slot = 0;
+        timer.begin(s);
+        SmallLoop<I> sl{};
+        sl.n = n;
+        sl.d = (int)d;
+        sl.k = (int)k;
+        sl.iters = max_iter - it;
+        sl.X = X;
+        sl.w = w;
+        sl.bufs[0] = bufs[0];
+        sl.bufs[1] = bufs[1];
+        sl.labels = labels;
+        sl.sums = ws.sums.template as<float>();
+        sl.sizes = ws.sizes.template as<float>();
+        sl.per_sample = ws.per_sample.template as<float>();
+        sl.list = ws.list.template as<I>();
+        sl.state = ws.state();
+        sl.host = host;
+        sl.tol = tol_t;
+        launch_small_loop<I>(sl, s);
+        timer.end(s);
+      }
+    }
+    while (!one_block && queued < max_iter && queued <= it + ahead) {
       timer.slot = (int)(queued % (kAhead + 1));
       lloyd_front<T, I>(ws, X, w, bufs[queued % 2], labels, s, timer);
       enqueue_tail(queued, false);
@@ -780,7 +827,24 @@ static void driver_impl(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
     const unsigned long long word = wait_loop(host, it, s);
     const int64_t done = (int64_t)(word >> 2);
     int stop = (int)(word & 3);
-    for (; it < done; ++it) timer.collect((int)(it % (kAhead + 1)));
+    if (stop == kLoopRefused) {   // the inputs' range: an iteration per launch
+      KMD_HIP_CHECK(hipStreamSynchronize(s));
+      KMD_HIP_CHECK(hipMemsetAsync(ws.state(), 0, sizeof(LoopState), s));
+      host->word = 0;
+      one_block = false;
+      start();
+      continue;
+    }
+    if (one_block) {
+      timer.collect(0, done - it);
+      it = done;
+      if (stop == kLoopConverged) {
+        KMD_HIP_CHECK(hipStreamSynchronize(s));
+        finish(host->total, 0);
+        return;
+      }
+    }
+    for (; it < done; ++it) timer.collect((int)(it % (kAhead + 1)), 1);
     T *cur = bufs[(it + 1) % 2];   // of iteration it - 1, the last finished
     if (verbose) {
       launch_inertia<T, I>(n, d, k, X, w, cur, labels,
@@ -878,18 +942,7 @@ static void driver_impl(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
   std::memcpy(&final_state, end, sizeof(final_state));
   double total;
   std::memcpy(&total, end + 56, sizeof(total));
-  *inertia_out = static_cast<double>(static_cast<T>(total));
-  *n_iters_out = it;
-  if (stats) {
-    stats->fused_kernel_ms = timer.total_ms;
-    stats->fused_launches = timer.launches;
-    int path = ws.mixed_terms > 0 ? (ws.mixed_terms == 3 ? 3 : 2)
-                                  : (ws.fast ? 1 : 0);
-    if (ws.tiled) path += 3;  // 4 tiled FP32, 5 tiled BF16, 6 tiled BF16x3
-    if (ws.tiled && ws.mixed_terms == 8) path = 7;  // tiled FP8
-    stats->fused_path = path;
-    stats->n_rescored = final_state.rescored;
-  }
+  finish(total, final_state.rescored);
 }
 
 #define KMD_INST_DRIVER(T, I)                                                 \

@@ -847,6 +847,284 @@ __global__ void __launch_bounds__((smallk_threads<DB, G>()))
   }
 }
 
+// ---- small fits: the whole loop in one block ----------------------------------
+//
+// With a thousand samples an iteration of three launches is all latency: 5.6 +
+// 2.2 + 3.9 us of kernels with one block's work in them, and the launches.
+// Here one block of 16 waves runs iteration after iteration, 1024 samples at a
+// time (the only ones stay in registers, several slots of them are read again
+// from the caches), with centroids, sums and half norms in LDS.  Cross term and argmin as in smallk_lloyd_krn, sums as there (int64
+// fixed point, lane-keyed copies), then the reduction's conversion and the
+// tail's division, chains and FP64 sum in their order: every value is the bit
+// the three kernels give.  n = 1000, d = 16, k = 8: 4.3 us
+// per iteration against 13.8.  The ranges for the scales, the half norms and the
+// epilogue are done here too: ten launches fewer per fit.
+template <int DB, int G>
+constexpr int loop_copies() {  // copies of the sums: at most 96 KB
+  return DB <= 16 ? (G == 8 ? 16 : 32) : smallk_copies<DB, G>();
+}
+
+template <int DB, int G, typename I>
+__global__ void __launch_bounds__(1024) small_loop_krn(SmallLoop<I> a) {
+  constexpr int NT = 1024;
+  constexpr int R = loop_copies<DB, G>();
+  constexpr int KP = 4 * G;
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  float *Ca = reinterpret_cast<float *>(lds_raw);   // [KP][DB] centroids
+  float *Hl = Ca + KP * DB;                         // [KP] -hn, -inf padded
+  float *Sc = Hl + KP;                              // [DB + 4] scales
+  float *Sn = Sc + DB + 4;                          // [KP][DB + 1] undivided sums
+  float *Sz = Sn + KP * (DB + 1);                   // [KP] sizes
+  float *Sh = Sz + KP;                              // [KP] squared shifts
+  // [k][DB + 1][R] sums; before them the rows' statistics, after them the
+  // waves' sums of the inertia
+  u64 *S64 = reinterpret_cast<u64 *>(Sh + KP);
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  const int d = a.d, k = a.k;
+  const int64_t n = a.n;
+  LoopState *st = a.state;
+  const long long first = st->done;
+
+  // The statistics of fixed_point.hpp, a wave per row of X (row d: w); then
+  // its scales and flag.
+  u64 *estat = S64;                                            // [2 (DB + 1)]
+  unsigned *maxbits = reinterpret_cast<unsigned *>(estat + 2 * (DB + 1));   // [DB + 2]
+  for (int f = wave; f <= d; f += NT / kWave) {
+    const float *row = f < d ? a.X + (int64_t)f * n : a.w;
+    unsigned m = 0u, esum = 0u, ecnt = 0u, wmin_inv = 0u;
+    for (int64_t i = lane; i < n; i += kWave) {
+      const unsigned v = __float_as_uint(row[i]);
+      range_accumulate(v, m, esum, ecnt);
+      const unsigned bits = v & 0x7fffffffu;
+      if (bits != 0u) wmin_inv = max(wmin_inv, ~bits);
+    }
+    for (int o = kWave / 2; o > 0; o >>= 1) {   // n <= 8192: the sums fit 32 bits
+      m = max(m, (unsigned)__shfl_xor((int)m, o, kWave));
+      wmin_inv = max(wmin_inv, (unsigned)__shfl_xor((int)wmin_inv, o, kWave));
+      esum += (unsigned)__shfl_xor((int)esum, o, kWave);
+      ecnt += (unsigned)__shfl_xor((int)ecnt, o, kWave);
+    }
+    if (lane == 0) {
+      maxbits[f] = m;
+      estat[2 * f] = esum;
+      estat[2 * f + 1] = ecnt;
+      if (f == d) maxbits[d + 1] = wmin_inv;
+    }
+  }
+  __syncthreads();
+  if (tid < DB + 4) Sc[tid] = 0.f;
+  bool bad = lane <= d && maxbits[lane] >= 0x7f800000u;
+  double sx = lane < d ? fixed_point_spread(lane, maxbits, estat) : 0.0;
+  if (d == kWave) bad |= maxbits[d] >= 0x7f800000u;
+  const bool any_bad = __ballot(bad) != 0;
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    const double t = __shfl_xor(sx, o, kWave);
+    sx = t > sx ? t : sx;
+  }
+  const int flag = fixed_point_flag(d, any_bad, sx, maxbits, estat);   // every thread's
+  const double wmax = (double)__uint_as_float(maxbits[d]);
+  const float own_scale =
+      tid <= d ? fixed_point_scale(
+                     n, wmax * (tid < d ? (double)__uint_as_float(maxbits[tid]) : 1.0))
+               : 0.f;
+  __syncthreads();
+  if (flag != 0) {
+    if (tid == 0) {
+      st->stop = kLoopRefused;
+      publish(a.host, *st);
+    }
+    return;
+  }
+  if (tid <= d) Sc[tid < d ? tid : DB] = own_scale;
+  const float *C0 = a.bufs[first & 1];
+  for (int i = tid; i < KP * DB; i += NT) {
+    const int c = i / DB, f = i % DB;
+    Ca[i] = (f < d && c < k) ? C0[(int64_t)f * k + c] : 0.f;
+  }
+  __syncthreads();
+  if (tid < KP) {
+    float h = 0.f;
+    for (int f = 0; f < d; ++f) h = fmaf(Ca[tid * DB + f], Ca[tid * DB + f], h);
+    Hl[tid] = tid < k ? -(h / 2.f) : -__builtin_huge_valf();
+  }
+
+  const int slots = (int)((n + NT - 1) / NT);
+  float x[DB], ws;
+  auto load = [&](int64_t s) {
+    // lanes past the last sample read it and add nothing
+    const int64_t at = min<int64_t>(s, n - 1);
+#pragma unroll
+    for (int f = 0; f < DB; ++f) x[f] = f < d ? a.X[(int64_t)f * n + at] : 0.f;
+    ws = a.w[at];
+  };
+  // the label of this lane's sample
+  auto score = [&]() {
+    f32x4 acc[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) acc[g] = *reinterpret_cast<const f32x4 *>(Hl + 4 * g);
+#pragma unroll
+    for (int f4 = 0; f4 < DB; f4 += 4) {
+      f32x4 av = {};
+      if (lane < KP) av = *reinterpret_cast<const f32x4 *>(Ca + lane * DB + f4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mfma4_groups<G>(av[e], x[f4 + e], acc);
+    }
+    float m = -__builtin_huge_valf();
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      m = vmax3(m, acc[g][0], acc[g][1]);
+      m = vmax3(m, acc[g][2], acc[g][3]);
+    }
+    int l = 0;
+#pragma unroll
+    for (int c = KP - 1; c >= 0; --c) l = (acc[c / 4][c % 4] == m) ? c : l;
+    return (-m < __builtin_huge_valf()) ? l : 0;
+  };
+  if (slots == 1) load(tid);
+  const int n_sums = k * (DB + 1) * R;
+  long long it = 0;
+  int stop = 0;
+  double shift = 0.0;
+  while (it < a.iters) {
+    for (int i = tid; i < n_sums; i += NT) S64[i] = 0ull;
+    __syncthreads();
+    for (int j = 0; j < slots; ++j) {
+      const int64_t s = (int64_t)j * NT + tid;
+      if (s - lane >= n) break;   // no samples for this wave
+      if (slots > 1) load(s);
+      const int l = score();
+      if (s < n) {
+        a.labels[s] = (I)l;       // a relocation needs them
+        u64 *Sp = S64 + l * (DB + 1) * R + (lane & (R - 1));
+#pragma unroll
+        for (int f = 0; f < DB; ++f) {
+          if (f < d) {
+            const int q = __float2int_rn((x[f] * ws) * Sc[f]);
+            atomicAdd(Sp + f * R, (u64)(long long)q);
+          }
+        }
+        atomicAdd(Sp + DB * R, (u64)(long long)__float2int_rn(ws * Sc[DB]));
+      }
+    }
+    __syncthreads();
+    // the copies' totals, converted: feature rows, then (f == d) the sizes
+    for (int i = tid; i < k * (d + 1); i += NT) {
+      const int c = i / (d + 1), f = i - c * (d + 1);
+      const int fs = f < d ? f : DB;
+      const u64 *src = S64 + (c * (DB + 1) + fs) * R;
+      u64 t = 0;
+#pragma unroll
+      for (int r = 0; r < R; ++r) t += src[(r + lane) & (R - 1)];
+      const float v = (float)((double)(long long)t / (double)Sc[fs]);
+      if (f < d)
+        Sn[c * (DB + 1) + f] = v;
+      else
+        Sz[c] = v;
+    }
+    __syncthreads();
+    ++it;
+    if (__ballot(lane < k && Sz[lane] == 0.f) != 0) {   // the same in every wave
+      stop = kLoopEmpty;
+      break;
+    }
+    // a wave per centroid: the quotients side by side, the chains over the
+    // features by its first lane
+    for (int c = wave; c < k; c += NT / kWave) {
+      const float size = Sz[c];
+      if (lane < d) {
+        const float q = Sn[c * (DB + 1) + lane] / size;
+        Sn[c * (DB + 1) + lane] = Ca[c * DB + lane] - q;
+        Ca[c * DB + lane] = q;
+      }
+      if (lane == 0) {
+        float acc = 0.f, h = 0.f;
+#pragma unroll 8
+        for (int f = 0; f < d; ++f) {
+          const float diff = Sn[c * (DB + 1) + f], q = Ca[c * DB + f];
+          acc = fmaf(diff, diff, acc);
+          h = fmaf(q, q, h);
+        }
+        Hl[c] = -(h / 2.f);
+        Sh[c] = acc;
+      }
+    }
+    __syncthreads();
+    double v = lane < k ? (double)Sh[lane] : 0.0;
+    for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+    shift = v;
+    if (!((float)v > a.tol)) {
+      stop = kLoopConverged;
+      break;
+    }
+  }
+  const long long done = first + it;
+  if (stop == kLoopEmpty) {
+    // the centroids of this iteration's labels, the undivided sums, the sizes
+    // and the list, as the tail leaves them
+    for (int i = tid; i < k * d; i += NT) {
+      const int f = i / k, c = i - f * k;
+      a.bufs[(done - 1) & 1][i] = Ca[c * DB + f];
+      a.sums[i] = Sn[c * (DB + 1) + f];
+    }
+    if (tid < k) {   // k <= 32: the first wave, the list ascends with the lane
+      a.sizes[tid] = Sz[tid];
+      const unsigned long long empty = __ballot(Sz[tid] == 0.f);
+      if (Sz[tid] == 0.f) a.list[__popcll(empty & ((1ull << lane) - 1ull))] = (I)tid;
+      if (tid == 0) st->n_empty = __popcll(empty);
+    }
+  } else {
+    // the fit's end: labels and inertia of the final centroids, which go to
+    // res; the sum in the order of launch_reduce_sum
+    for (int i = tid; i < k * d; i += NT) {
+      const int f = i / k, c = i - f * k;
+      a.bufs[1][i] = Ca[c * DB + f];
+    }
+    __syncthreads();   // (no iteration: the half norms)
+    for (int j = 0; j < slots; ++j) {
+      const int64_t s = (int64_t)j * NT + tid;
+      if (s - lane >= n) break;
+      if (slots > 1) load(s);
+      const int l = score();
+      if (s < n) {
+        a.labels[s] = (I)l;
+        float acc = 0.f;
+#pragma unroll
+        for (int f = 0; f < DB; ++f) {
+          if (f < d) {
+            const float diff = x[f] - Ca[l * DB + f];
+            acc = fmaf(diff, diff, acc);
+          }
+        }
+        a.per_sample[s] = acc * ws;
+      }
+    }
+    __threadfence_block();
+    __syncthreads();
+    // blocks of 256 threads, 4096 samples or more each (two of them at most)
+    const int nb = (int)((n + 4095) / 4096);
+    double acc = 0.0;
+    if (tid < 256 * nb)
+      for (int64_t i = tid; i < n; i += 256 * nb) acc += (double)a.per_sample[i];
+    for (int o = kWave / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kWave);
+    double *lds = reinterpret_cast<double *>(S64);
+    if (lane == 0) lds[wave] = acc;
+    __syncthreads();
+    if (tid == 0) {
+      double p[2] = {0.0, 0.0};
+      for (int q = 0; q < nb; ++q)
+        for (int i = 0; i < 4; ++i) p[q] += lds[4 * q + i];
+      a.host->total = p[0] + p[1];
+    }
+  }
+  if (tid == 0) {
+    st->done = done;
+    st->shift = shift;
+    st->stop = stop != 0 ? stop : kLoopConverged;   // or out of iterations
+    __threadfence_system();
+    publish(a.host, *st);
+  }
+}
+
 // ---- fixed-point scales ------------------------------------------------------
 
 // The range statistics of fixed_point.hpp for row f = blockIdx.y of X (f ==
@@ -1082,6 +1360,15 @@ inline int smallk_copies_of(int64_t d, int64_t k) {
                                                   : smallk_copies<64, 2>();
 }
 
+inline size_t small_loop_lds(int64_t d, int64_t k) {
+  const int db = smallk_db(d), g = smallk_groups(k), kp = 4 * g;
+  const int r = db <= 16 ? (g == 8 ? 16 : 32) : smallk_copies_of(d, k);
+  // the rows' statistics (row db + 1 of maxbits included) share the sums' place
+  const size_t sums = std::max<size_t>(sizeof(u64) * (size_t)k * (db + 1) * r,
+                                       sizeof(u64) * 2 * (db + 1) + 4 * (db + 4));
+  return sizeof(float) * ((size_t)kp * db + kp + db + 4 + kp * (db + 1) + 2 * kp) + sums;
+}
+
 // KMD_NO_SMALLK=1 sends k <= 32 to the 32-row tile kernel (the two compute
 // the same labels and sums; the switch exists to compare them).
 inline bool smallk_enabled() {
@@ -1265,6 +1552,44 @@ bool fast_smallk_serves(int64_t d, int64_t k) {
   return d >= 1 && d <= kMaxD && k >= 1 && k <= kSmallK && smallk_enabled() &&
          plan_smallk<int32_t, true>(1, d, k).fn != nullptr;
 }
+
+bool small_loop_serves(int64_t n, int64_t d, int64_t k) {
+  if (n < 1 || !fast_smallk_serves(d, k)) return false;
+  // Products and updates of one lane (an iteration costs 0.035 us for each)
+  // against what three launches take for the shape, 12 us and more with the
+  // features: one block is ahead up to there (1000 x 32 x 32: 12 against 17 us,
+  // 4000 x 16 x 8: 13.7 / 14.7; behind beyond: 4000 x 8 x 32: 13.7 / 13.3).
+  const int db = smallk_db(d);
+  return n <= 8192 && small_loop_lds(d, k) <= kLdsPerCu &&
+         ceil_div<int64_t>(n, 1024) * db * (4 + smallk_groups(k)) <= 320 + 4 * db;
+}
+
+template <typename I>
+void launch_small_loop(const SmallLoop<I> &a, hipStream_t s) {
+  require(small_loop_serves(a.n, a.d, a.k), "small loop: unsupported shape");
+  void (*fn)(SmallLoop<I>) = nullptr;
+  const int g = smallk_groups(a.k);
+#define KMD_SL_CASE(DB)                            \
+  case DB:                                         \
+    fn = g == 1   ? &small_loop_krn<DB, 1, I>      \
+         : g == 2 ? &small_loop_krn<DB, 2, I>      \
+         : g == 4 ? &small_loop_krn<DB, 4, I>      \
+                  : &small_loop_krn<DB, (DB < 64 ? 8 : 4), I>;   /* (64, 8): not served */ \
+    break;
+  switch (smallk_db(a.d)) {
+    KMD_SL_CASE(8)
+    KMD_SL_CASE(16)
+    KMD_SL_CASE(32)
+    default:
+    KMD_SL_CASE(64)
+  }
+#undef KMD_SL_CASE
+  allow_full_lds(reinterpret_cast<const void *>(fn));
+  hipLaunchKernelGGL(fn, dim3(1), dim3(1024), small_loop_lds(a.d, a.k), s, a);
+  KMD_LAUNCH_CHECK();
+}
+template void launch_small_loop<int32_t>(const SmallLoop<int32_t> &, hipStream_t);
+template void launch_small_loop<int64_t>(const SmallLoop<int64_t> &, hipStream_t);
 
 template <typename I>
 int fast_fused_blocks(int64_t n, int64_t d, int64_t k) {

@@ -73,6 +73,32 @@ int fast_fused_blocks(int64_t n, int64_t d, int64_t k);
 // kernel (KMD_NO_SMALLK=1 turns it off)
 bool fast_smallk_serves(int64_t d, int64_t k);
 
+// A whole small fit (few samples and clusters) in one launch of one block, in
+// the arithmetic of the kernels it stands for: range statistics, half norms,
+// iterations, final labels and inertia.  Ends with the fit (kLoopConverged,
+// also when out of iterations; the centroids in bufs[1], the inertia in
+// host->total) or with clusters to relocate (state, sums, sizes, list and
+// bufs[(done - 1) & 1] as launch_step_tail leaves them).  Refuses
+// (kLoopRefused, nothing else written) inputs whose range the fixed-point sums
+// cannot hold.
+template <typename I>
+struct SmallLoop {
+  int64_t n;
+  int d, k;
+  long long iters;
+  const float *X, *w;
+  float *bufs[2];          // bufs[state->done & 1]: the centroids to start from
+  I *labels;
+  float *sums, *sizes, *per_sample;
+  I *list;
+  LoopState *state;
+  LoopHost *host;
+  float tol;
+};
+bool small_loop_serves(int64_t n, int64_t d, int64_t k);
+template <typename I>
+void launch_small_loop(const SmallLoop<I> &a, hipStream_t s);
+
 // The reference's fused step on the MFMA kernel: FP32 block sums in LDS,
 // flushed into the caller's private copies with FP32 atomics (no scales, no
 // pre-pass, no working memory).
