@@ -729,6 +729,163 @@ __global__ void __launch_bounds__(1024)
     int64_t pos = g + r;
     if (pos < m) order[pos] = (int64_t)selected[n - 1 - r];
   }
+  // NaN distances can leave fewer samples than m: no sample for the rest
+  for (int64_t pos = g + (e > 0 ? e : 0) + threadIdx.x; pos < m; pos += blockDim.x)
+    order[pos] = -1;
+}
+
+// The same order in one launch of one block, for n <= kFarN samples and m <=
+// kFarM of them: thirteen launches of the general way (threshold, selection,
+// order) are mostly latency there.  The whole relocation of m = 2 of n = 50,000:
+// 237 -> 111 us (this kernel 19), n = 262,144: 253 -> 147 us; one CU reads at 60 -
+// 70 GB/s, and past that n the general way's cost stays where it is while this
+// one's grows with n.  The m-th largest of the threads' own maxima bounds the
+// m-th largest distance from below; the samples above it, about 1.4 m at half as
+// many as threads, are gathered in LDS and ranked (m = 200 of 50,000: 331 -> 212
+// us).  With m near the number of threads that bound is no bound any more (m =
+// 1000 of 50,000: 775 -> 963 us), hence kFarM.  Many equal distances can make the
+// list overflow all the same: then the m-th largest is found over all samples,
+// and the equal ones are taken in index order.  A NaN distance is never far.
+constexpr int64_t kFarN = 262144;
+constexpr int kFarThreads = 1024;
+constexpr int64_t kFarM = kFarThreads / 2;
+constexpr int kFarList = 2048;
+
+template <typename T>
+struct FarKey;
+template <>
+struct FarKey<float> {
+  using U = unsigned;
+  static __device__ U of(float v) {
+    const U b = __float_as_uint(v + 0.f);   // -0 as +0
+    return v != v ? 0u : (b >> 31) ? ~b : (b | 0x80000000u);
+  }
+};
+template <>
+struct FarKey<double> {
+  using U = unsigned long long;
+  static __device__ U of(double v) {
+    const U b = (U)__double_as_longlong(v + 0.0);
+    return v != v ? 0ull : (b >> 63) ? ~b : (b | (1ull << 63));
+  }
+};
+
+template <typename T>
+__global__ void __launch_bounds__(kFarThreads)
+    far_order_krn(int n, int m, const T *__restrict__ dist, int64_t *__restrict__ order) {
+  using U = typename FarKey<T>::U;
+  constexpr int kWaves = kFarThreads / kWave;
+  __shared__ U lkey[kFarList];
+  __shared__ int lidx[kFarList];
+  __shared__ int wc[2][kWaves];
+  __shared__ int count;
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+  // sum of every wave's v over the block; par alternates between calls
+  auto block_count = [&](int v, int par) {
+    if (lane == 0) wc[par][wave] = v;
+    __syncthreads();
+    int t = 0;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) t += wc[par][i];
+    return t;
+  };
+  if (tid == 0) count = 0;
+  U mine = 0;
+  constexpr int kU = 8;
+  for (int i0 = tid; i0 < n; i0 += kU * kFarThreads) {
+    T v[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int i = i0 + u * kFarThreads;
+      v[u] = i < n ? dist[i] : std::numeric_limits<T>::quiet_NaN();
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const U q = FarKey<T>::of(v[u]);
+      mine = q > mine ? q : mine;
+    }
+  }
+  // largest key that at least m of the threads' maxima reach, bit by bit
+  U low = 0;
+  int par = 0;
+  for (int b = 8 * (int)sizeof(U) - 1; b >= 0; --b, par ^= 1) {
+    const U probe = low | (U(1) << b);
+    if (block_count(__popcll(__ballot(mine >= probe)), par) >= m) low = probe;
+  }
+  for (int i0 = tid; i0 < n; i0 += kU * kFarThreads) {
+    T v[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int i = i0 + u * kFarThreads;
+      v[u] = i < n ? dist[i] : T(0);
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int i = i0 + u * kFarThreads;
+      const U q = FarKey<T>::of(v[u]);
+      if (i < n && q >= low) {
+        const int at = atomicAdd(&count, 1);
+        if (at < kFarList) {
+          lkey[at] = q;
+          lidx[at] = i;
+        }
+      }
+    }
+  }
+  __syncthreads();
+  int listed = count;
+  if (listed > kFarList) {
+    // the exact m-th largest key, then the samples above it and the first
+    // ones equal to it
+    U thr = 0;
+    for (int b = 8 * (int)sizeof(U) - 1; b >= 0; --b, par ^= 1) {
+      const U probe = thr | (U(1) << b);
+      int c = 0;
+      for (int i = tid; i - lane < n; i += kFarThreads)
+        c += __popcll(__ballot(i < n && FarKey<T>::of(dist[min(i, n - 1)]) >= probe));
+      if (block_count(c, par) >= m) thr = probe;
+    }
+    __syncthreads();
+    if (tid == 0) count = 0;
+    __syncthreads();
+    for (int i = tid; i < n; i += kFarThreads) {
+      const U q = FarKey<T>::of(dist[i]);
+      if (q > thr) {
+        const int at = atomicAdd(&count, 1);   // fewer than m <= kFarM of them
+        lkey[at] = q;
+        lidx[at] = i;
+      }
+    }
+    __syncthreads();
+    int have = count;
+    for (int i0 = 0; i0 < n && have < m; i0 += kFarThreads, par ^= 1) {
+      const int i = i0 + tid;
+      const bool eq = i < n && FarKey<T>::of(dist[min(i, n - 1)]) == thr;
+      const unsigned long long mask = __ballot(eq);
+      const int total = block_count(__popcll(mask), par);
+      int before = 0;
+      for (int q = 0; q < wave; ++q) before += wc[par][q];
+      const int at = have + before + __popcll(mask & ((1ull << lane) - 1ull));
+      if (eq && at < m) {
+        lkey[at] = thr;
+        lidx[at] = i;
+      }
+      have += total;
+    }
+    __syncthreads();
+    listed = min(have, m);
+  }
+  for (int i = tid; i < listed; i += kFarThreads) {
+    const U ki = lkey[i];
+    const int si = lidx[i];
+    int rank = 0;
+    for (int j = 0; j < listed; ++j) {
+      const U kj = lkey[j];
+      rank += (kj > ki) || (kj == ki && lidx[j] < si);
+    }
+    if (rank < m) order[rank] = si;
+  }
+  for (int r = listed + tid; r < m; r += kFarThreads) order[r] = -1;   // m > n
 }
 
 template <typename T, typename I>
@@ -741,9 +898,10 @@ __global__ void __launch_bounds__(kBlock)
   if (f >= d) return;
   for (int64_t j = 0; j < m; ++j) {
     int64_t s = order[j];
+    if (s < 0 || s >= n) continue;
     int64_t p = (int64_t)labels[s];
     int64_t e = (int64_t)empty_list[j];
-    if (s < 0 || s >= n || p < 0 || p >= k || e < 0 || e >= k) continue;
+    if (p < 0 || p >= k || e < 0 || e >= k) continue;
     T ws = w[s];
     T add = X[f * n + s] * ws;
     C[f * k + p] -= add;
@@ -961,21 +1119,24 @@ void launch_relocate(int64_t n, int64_t d, int64_t k, int64_t n_empty,
                      T *sizes, T *per_sample_inertia, hipStream_t s) {
   const int64_t m = n_empty < n ? n_empty : n;
   if (m <= 0 || d <= 0) return;
-  TempBuffer thr(sizeof(T), s);
-  TempBuffer sel(sizeof(I) * (n + 2), s);
   TempBuffer order(sizeof(int64_t) * m, s);
-  I *n_gt = sel.as<I>() + n;
-  I *n_eq = n_gt + 1;
-  launch_threshold<T>(n, sq_dist, m, thr.as<T>(), s);
-  hipLaunchKernelGGL((init_counters_krn<T, I>), dim3(1), dim3(1), 0, s, n_gt,
-                     n_eq);
-  KMD_LAUNCH_CHECK();
-  launch_select_far<T, I>(m, n, sq_dist, thr.as<const T>(), sel.as<I>(), n_gt,
-                          n_eq, s);
-  hipLaunchKernelGGL((relocation_order_krn<T, I>), dim3(1), dim3(1024), 0, s, n,
-                     m, sq_dist, sel.as<const I>(), n_gt, n_eq,
-                     order.as<int64_t>());
-  KMD_LAUNCH_CHECK();
+  if (n <= kFarN && m <= kFarM) {
+    hipLaunchKernelGGL(far_order_krn<T>, dim3(1), dim3(kFarThreads), 0, s, (int)n, (int)m,
+                       sq_dist, order.as<int64_t>());
+    KMD_LAUNCH_CHECK();
+  } else {
+    TempBuffer thr(sizeof(T), s);
+    TempBuffer sel(sizeof(I) * (n + 2), s);
+    I *n_gt = sel.as<I>() + n;
+    I *n_eq = n_gt + 1;
+    launch_threshold<T>(n, sq_dist, m, thr.as<T>(), s);
+    hipLaunchKernelGGL((init_counters_krn<T, I>), dim3(1), dim3(1), 0, s, n_gt, n_eq);
+    KMD_LAUNCH_CHECK();
+    launch_select_far<T, I>(m, n, sq_dist, thr.as<const T>(), sel.as<I>(), n_gt, n_eq, s);
+    hipLaunchKernelGGL((relocation_order_krn<T, I>), dim3(1), dim3(1024), 0, s, n, m,
+                       sq_dist, sel.as<const I>(), n_gt, n_eq, order.as<int64_t>());
+    KMD_LAUNCH_CHECK();
+  }
   hipLaunchKernelGGL((relocate_apply_krn<T, I>), dim3(ceil_div<int64_t>(d, kBlock)),
                      dim3(kBlock), 0, s, n, d, k, m, X, w, labels, empty_list,
                      order.as<const int64_t>(), centroids, sizes,
