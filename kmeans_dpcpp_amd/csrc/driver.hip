@@ -221,7 +221,7 @@ static std::unique_ptr<LloydWorkspace<T, I>> make_tiled_workspace(
     if (bad) return nullptr;
     ws->tiled = true;
     ws->xr = TempBuffer(sizeof(float) * (size_t)n * d, s);
-    launch_transpose(n, d, X, ws->xr.template as<float>(), s);
+    bool have_xr = false;
     ws->upd = TempBuffer(tiled_update_scratch_bytes(n, k), s);
     if (precision != KMD_PREC_FP32) {
       // BF16 terms, or 8: the FP8 (e4m3) kernel
@@ -245,15 +245,18 @@ static std::unique_ptr<LloydWorkspace<T, I>> make_tiled_workspace(
           ws->xb = TempBuffer(tiled_xb_bytes(n, d), s);
           ws->xnb = TempBuffer(sizeof(float) * (size_t)n, s);
           if (terms == 1)
-            launch_tiled_xb_prep(n, d, X, ws->xb.template as<void>(),
+            launch_tiled_xb_prep(n, d, X, ws->xr.template as<float>(),
+                                 ws->xb.template as<void>(),
                                  ws->xnb.template as<float>(), s);
           else
             launch_tiled_x8_prep(n, d, X, ws->xb.template as<void>(),
                                  ws->xnb.template as<float>(),
                                  ws->bound.template as<float>(), s);
+          have_xr = terms == 1;
         }
       }
     }
+    if (!have_xr) launch_transpose(n, d, X, ws->xr.template as<float>(), s);
     return ws;
   } else {
     (void)n, (void)d, (void)k, (void)precision, (void)X, (void)w, (void)s;

@@ -215,7 +215,7 @@ void launch_fast_rescore(int64_t n, int64_t d, int64_t k, const float *X,
 
 // ---- tiled path (lloyd_tiled.hip): d <= 128, centroids streamed via LDS ----
 bool tiled_supported(int64_t d, int64_t k);
-// X_r (n, d) = transpose of X_t (d, n)
+// X_r (n, d) = transpose of X_t (d, n), d <= 128
 void launch_transpose(int64_t n, int64_t d, const float *X_t, float *X_r,
                       hipStream_t s);
 // FP32 MFMA assignment (labels only); tiles_scratch (tiled_tiles_bytes(d, k)
@@ -261,10 +261,10 @@ void launch_tiled_mixed_assign(int64_t n, int64_t d, int64_t k, int T,
                                int *queue_counts, unsigned *qmask, hipStream_t s,
                                const int *skip = nullptr, const void *xb = nullptr,
                                const float *xnb = nullptr);
-// BF16 samples (sample-major, d rounded up to the kernel's bucket) and norm
-// bounds for launch_tiled_mixed_assign with T = 1
+// launch_transpose's X_r, and BF16 samples (sample-major, d rounded up to the
+// kernel's bucket) and norm bounds for launch_tiled_mixed_assign with T = 1
 size_t tiled_xb_bytes(int64_t n, int64_t d);
-void launch_tiled_xb_prep(int64_t n, int64_t d, const float *X_t, void *xb,
+void launch_tiled_xb_prep(int64_t n, int64_t d, const float *X_t, float *X_r, void *xb,
                           float *xnb, hipStream_t s);
 // FP8 (T = 8 in the tiled mixed launchers): e4m3 samples x8 (n bf16_d bytes,
 // within tiled_xb_bytes), norm bounds and the fit's sample scale in bound

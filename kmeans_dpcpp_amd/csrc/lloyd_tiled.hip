@@ -380,23 +380,30 @@ __global__ void __launch_bounds__(256) cand_count_krn(CandArgs a) {
     atomicAdd(&a.tile_cnt[threadIdx.x], cnt[threadIdx.x]);
 }
 
-__global__ void cand_scan_krn(CandArgs a) {
+// One wave: the at most 32 tiles' counts by shuffles, the segments' by lane (one
+// thread's chain of dependent loads took 15 us; here 4.3).
+__global__ void __launch_bounds__(kWave) cand_scan_krn(CandArgs a) {
   if (skipped(a)) return;
-  if (threadIdx.x != 0) return;
-  int run = 0, wrun = 0;
-  for (int t = 0; t < a.n_ct; ++t) {
-    const int c = a.tile_cnt[t];
-    a.tile_start[t] = run;
-    a.tile_witem[t] = wrun;
-    run += c;
-    wrun += (c + 31) / 32;
+  const int lane = threadIdx.x;
+  const int c = lane < a.n_ct ? a.tile_cnt[lane] : 0;
+  const int wi = (c + 31) / 32;
+  int run = c, wrun = wi;
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int r = __shfl_up(run, o, kWave), w = __shfl_up(wrun, o, kWave);
+    if (lane >= o) {
+      run += r;
+      wrun += w;
+    }
   }
-  a.tile_start[a.n_ct] = run;
-  a.tile_witem[a.n_ct] = wrun;
-  a.overflow[0] = (int64_t)run > a.pair_cap ? 1 : 0;
+  if (lane <= a.n_ct) {
+    a.tile_start[lane] = run - c;
+    a.tile_witem[lane] = wrun - wi;
+  }
+  if (lane == a.n_ct) a.overflow[0] = (int64_t)run > a.pair_cap ? 1 : 0;
   int q = 0;
-  for (int g = 0; g < a.n_segments; ++g) q += a.queue_counts[g];
-  a.n_rescored[0] = q;
+  for (int g = lane; g < a.n_segments; g += kWave) q += a.queue_counts[g];
+  for (int o = kWave / 2; o > 0; o >>= 1) q += __shfl_xor(q, o, kWave);
+  if (lane == 0) a.n_rescored[0] = q;
 }
 
 __global__ void __launch_bounds__(256) cand_scatter_krn(CandArgs a) {
@@ -1293,30 +1300,6 @@ __global__ void __launch_bounds__(256)
   aop[gid] = v;
 }
 
-// xb[s] = the sample's features as BF16 (row of D, zero past d) and xnb[s]
-// = 1.0001 ||x_s|| (FP32; an upper bound of the norm), for the BF16 kernel's
-// streamed operands.  One thread per sample; the features are read
-// feature-major (coalesced over samples) and written 16 bytes at a time.
-__global__ void __launch_bounds__(256)
-    tiled_xb_prep_krn(int64_t n, int d, int D, const float *__restrict__ X_t,
-                      bf16x8 *__restrict__ xb, float *__restrict__ xnb) {
-  const int64_t s = blockIdx.x * 256ll + threadIdx.x;
-  if (s >= n) return;
-  float ss = 0.f;
-  for (int f0 = 0; f0 < D; f0 += 8) {
-    bf16x8 v;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int f = f0 + j;
-      const float x = (f < d) ? X_t[(int64_t)f * n + s] : 0.f;
-      ss = fmaf(x, x, ss);
-      v[j] = (__bf16)x;
-    }
-    xb[s * (D / 8) + f0 / 8] = v;
-  }
-  xnb[s] = sqrtf(ss) * 1.0001f;
-}
-
 __global__ void __launch_bounds__(256)
     tiled_bound_krn(int k, const float *__restrict__ hn, float *bound) {
   __shared__ float red[256 / kWave];
@@ -1335,23 +1318,71 @@ __global__ void __launch_bounds__(256)
 
 // ---- transpose and update ----------------------------------------------------
 
+// X_r (n, d) = transpose of X_t, and with XB also the BF16 kernel's streamed
+// operands: xb[s] = the sample's features as BF16 (row of D, zero past d) and
+// xnb[s] = 1.0001 ||x_s|| (FP32; an upper bound of the norm).  Bound by memory:
+// X_t is read once for all three.  A block takes S samples with all their
+// features through LDS (feature f of sample s at f (S + 1) + s), so that its part
+// of X_r and of xb is one contiguous piece; tiles of 32 x 32 wrote 128-byte pieces
+// of rows, and a thread per sample wrote xb in 16-byte pieces D apart.  S = 64
+// keeps the tile at 33 KB for the widest rows (four blocks a CU), S = 256 for d <=
+// 32 keeps the pieces long.  n = 2M, d = 128: 1164 us in two kernels, 474 us here
+// (5.4 TB/s).
+template <int S, bool XB>
 __global__ void __launch_bounds__(256)
-    transpose_krn(int64_t n, int d, const float *__restrict__ X_t,
-                  float *__restrict__ X_r) {
-  __shared__ float tile[32][33];
-  const int64_t s0 = (int64_t)blockIdx.x * 32;
-  const int f0 = blockIdx.y * 32;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 8 rows per pass
-  for (int r = ty; r < 32; r += 8) {
-    const int f = f0 + r;
-    const int64_t s = s0 + tx;
-    tile[r][tx] = (f < d && s < n) ? X_t[(int64_t)f * n + s] : 0.f;
+    tiled_layout_krn(int64_t n, int d, int D, const float *__restrict__ X_t,
+                     float *__restrict__ X_r, bf16x8 *__restrict__ xb,
+                     float *__restrict__ xnb) {
+  extern __shared__ __align__(16) float lay_smem[];
+  constexpr int LD = S + 1, G = 256 / S, kU = 16;
+  const int tid = threadIdx.x;
+  const int64_t s0 = (int64_t)blockIdx.x * S;
+  const int m = (int)min((int64_t)S, n - s0);
+  {
+    const int sl = tid % S, fl = tid / S;
+    const float *src = X_t + s0 + min(sl, m - 1);
+    for (int f0 = fl; f0 < d; f0 += kU * G) {
+      float v[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) v[u] = f0 + u * G < d ? src[(int64_t)(f0 + u * G) * n] : 0.f;
+#pragma unroll
+      for (int u = 0; u < kU; ++u)
+        if (f0 + u * G < d) lay_smem[(f0 + u * G) * LD + sl] = v[u];
+    }
   }
   __syncthreads();
-  for (int r = ty; r < 32; r += 8) {
-    const int64_t s = s0 + r;
-    const int f = f0 + tx;
-    if (s < n && f < d) X_r[s * d + f] = tile[tx][r];
+  {
+    const int qs = 256 / d, qf = 256 % d;
+    int sl = tid / d, f = tid % d;
+    float *dst = X_r + s0 * d;
+    for (int e = tid; e < m * d; e += 256) {
+      dst[e] = lay_smem[f * LD + sl];
+      sl += qs;
+      f += qf;
+      if (f >= d) {
+        f -= d;
+        ++sl;
+      }
+    }
+  }
+  if constexpr (XB) {
+    const int g8 = D / 8;
+    for (int e = tid; e < m * g8; e += 256) {
+      const int sl = e / g8, f0 = 8 * (e % g8);
+      bf16x8 v;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        v[j] = (__bf16)(f0 + j < d ? lay_smem[(f0 + j) * LD + sl] : 0.f);
+      xb[s0 * g8 + e] = v;
+    }
+    if (tid < m) {
+      float ss = 0.f;
+      for (int f = 0; f < d; ++f) {
+        const float x = lay_smem[f * LD + tid];
+        ss = fmaf(x, x, ss);
+      }
+      xnb[s0 + tid] = sqrtf(ss) * 1.0001f;
+    }
   }
 }
 
@@ -1673,12 +1704,25 @@ bool tiled_supported(int64_t d, int64_t k) {
   return d >= 1 && d <= kMaxTiledD && k >= 1 && k <= 32768;
 }
 
+namespace {
+template <bool XB>
+void layout(int64_t n, int64_t d, int D, const float *X_t, float *X_r, void *xb,
+            float *xnb, hipStream_t s) {
+  if (n <= 0) return;
+  require(d >= 1 && d <= kMaxTiledD, "transpose: more features than a tile holds");
+  const int S = d <= 32 ? 256 : 64;
+  const size_t lds = sizeof(float) * (size_t)d * (S + 1);
+  const dim3 grid((unsigned)ceil_div<int64_t>(n, S));
+  auto fn = S == 256 ? tiled_layout_krn<256, XB> : tiled_layout_krn<64, XB>;
+  hipLaunchKernelGGL(fn, grid, dim3(256), lds, s, n, (int)d, D, X_t, X_r,
+                     reinterpret_cast<bf16x8 *>(xb), xnb);
+  KMD_LAUNCH_CHECK();
+}
+}  // namespace
+
 void launch_transpose(int64_t n, int64_t d, const float *X_t, float *X_r,
                       hipStream_t s) {
-  if (n <= 0) return;
-  const dim3 grid((unsigned)ceil_div<int64_t>(n, 32), (unsigned)ceil_div<int64_t>(d, 32));
-  hipLaunchKernelGGL(transpose_krn, grid, dim3(256), 0, s, n, (int)d, X_t, X_r);
-  KMD_LAUNCH_CHECK();
+  layout<false>(n, d, 0, X_t, X_r, nullptr, nullptr, s);
 }
 
 namespace {
@@ -1860,13 +1904,9 @@ size_t tiled_xb_bytes(int64_t n, int64_t d) {
   return sizeof(unsigned short) * (size_t)(n > 0 ? n : 1) * bf16_d_of(d) + 256;
 }
 
-void launch_tiled_xb_prep(int64_t n, int64_t d, const float *X_t, void *xb,
+void launch_tiled_xb_prep(int64_t n, int64_t d, const float *X_t, float *X_r, void *xb,
                           float *xnb, hipStream_t s) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(tiled_xb_prep_krn, dim3((unsigned)ceil_div<int64_t>(n, 256)),
-                     dim3(256), 0, s, n, (int)d, bf16_d_of(d), X_t,
-                     reinterpret_cast<bf16x8 *>(xb), xnb);
-  KMD_LAUNCH_CHECK();
+  layout<true>(n, d, bf16_d_of(d), X_t, X_r, xb, xnb, s);
 }
 
 size_t tiled_aop_bytes(int64_t d, int64_t k, int T) {
