@@ -499,6 +499,69 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
+// The same for centroids beyond kInertiaLds: kF features of all centroids at a
+// time in LDS (feature-major rows as they are in memory), the chains of P samples
+// a thread in registers meanwhile.  A gather of C[f][labels] from L2 touches up to
+// 64 lines per wave load and bounds inertia_krn (n = 2M, d = 128, k = 1024: 594
+// us); here the gather is an LDS read and X's own pass is what is left (239 us,
+// 4.3 TB/s).  Each tile of 1024 P samples stages all of C and few tiles leave the
+// chip idle, so the rule asks for n >= kInertiaRatio k: at n = 64 k the gather is
+// the faster one (n = 65,536, d = 128, k = 1024, double: 65 us against 53 or
+// less), at 250 k and 16 features both take the same (67 us), at 488 k and 64
+// features 181 us against 73 (double: 334 against 134).
+constexpr int kInertiaThreads = 1024;
+constexpr int64_t kInertiaRatio = 256;
+template <int kF, int P, typename T, typename I>
+__global__ void __launch_bounds__(kInertiaThreads)
+    inertia_chunk_krn(int64_t n, int d, int k, const T *__restrict__ X,
+                      const T *__restrict__ w, const T *__restrict__ C,
+                      const I *__restrict__ labels, T *out) {
+  extern __shared__ __align__(16) unsigned char inertia_smem[];
+  T *Cs = reinterpret_cast<T *>(inertia_smem);
+  constexpr int kTile = kInertiaThreads * P;
+  for (int64_t s0 = blockIdx.x * (int64_t)kTile; s0 < n; s0 += (int64_t)gridDim.x * kTile) {
+    int64_t at[P];
+    int c[P];
+    T acc[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int64_t s = s0 + p * kInertiaThreads + threadIdx.x;
+      at[p] = s < n ? s : n - 1;
+      const int64_t l = (int64_t)labels[at[p]];
+      acc[p] = (l >= 0 && l < k) ? T(0) : std::numeric_limits<T>::quiet_NaN();
+      c[p] = (l >= 0 && l < k) ? (int)l : 0;
+    }
+    for (int f0 = 0; f0 < d; f0 += kF) {
+      const int nf = min(kF, d - f0);
+      T xv[P][kF];
+#pragma unroll
+      for (int u = 0; u < kF; ++u)
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+          xv[p][u] = u < nf ? X[(int64_t)(f0 + u) * n + at[p]] : T(0);
+      __syncthreads();
+      for (int e = threadIdx.x; e < nf * k; e += kInertiaThreads)
+        Cs[e] = C[(int64_t)f0 * k + e];
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < kF; ++u) {
+        if (u < nf) {
+#pragma unroll
+          for (int p = 0; p < P; ++p) {
+            const T diff = xv[p][u] - Cs[u * k + c[p]];
+            acc[p] = fma(diff, diff, acc[p]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int64_t s = s0 + p * kInertiaThreads + threadIdx.x;
+      if (s < n) out[s] = (w != nullptr) ? acc[p] * w[s] : acc[p];
+    }
+  }
+}
+
 // ---- deterministic two-stage sum (src/compute_inertia.hpp:104-135) ---------
 // Stage 1: fixed grid, each block sums a grid-stride slice in FP64.
 template <typename T>
@@ -1045,6 +1108,20 @@ void launch_inertia(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
                                            (int64_t)device_cu_count() * per_cu);
     hipLaunchKernelGGL((inertia_lds_krn<T, I>), dim3((unsigned)grid), dim3(kBlock), lds, s,
                        n, d, k, X, w, C, labels, out);
+    KMD_LAUNCH_CHECK();
+    return;
+  }
+  constexpr int64_t kRow = kInertiaLds / sizeof(T);   // values of C a block stages
+  if (4 * k <= kRow && n >= kInertiaRatio * k && d <= INT32_MAX) {
+    const bool f8 = 8 * k <= kRow;
+    const bool two = n > (int64_t)device_cu_count() * 2 * kInertiaThreads;
+    auto fn = f8 ? (two ? inertia_chunk_krn<8, 2, T, I> : inertia_chunk_krn<8, 1, T, I>)
+                 : (two ? inertia_chunk_krn<4, 2, T, I> : inertia_chunk_krn<4, 1, T, I>);
+    const int64_t tiles = ceil_div<int64_t>(n, kInertiaThreads * (two ? 2 : 1));
+    const int64_t grid = std::min<int64_t>(tiles, (int64_t)device_cu_count() * 2);
+    hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(kInertiaThreads),
+                       sizeof(T) * (size_t)k * (f8 ? 8 : 4), s, n, (int)d, (int)k, X, w, C,
+                       labels, out);
     KMD_LAUNCH_CHECK();
     return;
   }
