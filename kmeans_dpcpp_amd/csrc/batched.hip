@@ -34,6 +34,7 @@
 
 #include "common.hpp"
 #include "fixed_point.hpp"
+#include "fp32_tile.hpp"
 #include "lloyd_fast.hpp"
 
 namespace kmd {
@@ -48,7 +49,7 @@ typedef unsigned long long u64;
 // Assignment items are sized by their MFMA work: about kItemMacs
 // multiply-adds (samples x centroids padded to 32-tiles x features padded to
 // the kernel's feature bucket), at least kItemMin and at most kItemMax
-// samples, in multiples of kItemMin (one sub-tile of either block shape).
+// samples, in multiples of kItemMin (whole sub-tiles of either block shape).
 constexpr int64_t kItemMacs = int64_t(2048) * 256 * 64;
 constexpr int kItemMin = 512, kItemMax = 2048;
 // assignment block: one 32-sample column block per wave; 16 waves, or 8 for
@@ -234,18 +235,25 @@ __global__ void __launch_bounds__(NT)
           const int f = 2 * ks + half;
           xr[ks] = (f < d && p < end) ? gptr(F.X)[(int64_t)f * n + p] : 0.f;
         }
-        float bestv = __builtin_huge_valf();
-        int besti = 0;
+        // the single-fit kernels' first minimum: a max3 tree a tile, the row once
+        // a sample (16 compares and 32 selects a tile took as long as a quarter
+        // of the products of 16 features: 84 / 123 / 238 us for the three
+        // buckets of a full iteration, 82 / 127 / 213 here)
+        float bestm[1] = {-__builtin_huge_valf()};
+        int bestt[1] = {0};
+        f32x16 besta[1];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) besta[0][e] = -__builtin_huge_valf();
         for (int t = 0; t < n_ct; ++t) {
           const float *At = Cl + t * TF;
           // the chain starts from the tile's -hn, so -acc = hn - c.x
           const float *Ht = At + 2 * KS * 32;
-          f32x16 acc;
+          f32x16 acc[1];
 #pragma unroll
           for (int gg = 0; gg < 4; ++gg) {
             const f32x4 h4 = *reinterpret_cast<const f32x4 *>(Ht + 8 * gg + 4 * half);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[4 * gg + e] = h4[e];
+            for (int e = 0; e < 4; ++e) acc[0][4 * gg + e] = h4[e];
           }
 #pragma unroll
           for (int k4 = 0; k4 < KS / 4; ++k4) {
@@ -253,23 +261,15 @@ __global__ void __launch_bounds__(NT)
                 *reinterpret_cast<const f32x4 *>(At + (k4 * 2 + half) * 128 + col * 4);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-              acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[j], xr[4 * k4 + j], acc, 0, 0, 0);
+              acc[0] =
+                  __builtin_amdgcn_mfma_f32_32x32x2f32(av[j], xr[4 * k4 + j], acc[0], 0, 0, 0);
           }
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const int m0 = 8 * g + 4 * half;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float v = -acc[4 * g + e];
-              const bool upd = v < bestv;
-              bestv = upd ? v : bestv;
-              besti = upd ? (t * 32 + m0 + e) : besti;
-            }
-          }
+          tile_track_best<1>(t, acc, bestm, bestt, besta);
         }
-        const float ov = __shfl_xor(bestv, 32, kWave);
+        int besti = best_index(bestt[0], best_row(besta[0], bestm[0]), half);
+        const float om = __shfl_xor(bestm[0], 32, kWave);
         const int oi = __shfl_xor(besti, 32, kWave);
-        const bool take = (ov < bestv) || (ov == bestv && oi < besti);
+        const bool take = (om > bestm[0]) || (om == bestm[0] && oi < besti);
         besti = take ? oi : besti;
         if (half == 0 && p < end) F.labels[p] = besti;
       }
