@@ -50,8 +50,11 @@ typedef unsigned long long u64;
 // multiply-adds (samples x centroids padded to 32-tiles x features padded to
 // the kernel's feature bucket), at least kItemMin and at most kItemMax
 // samples, in multiples of kItemMin (whole sub-tiles of either block shape).
-constexpr int64_t kItemMacs = int64_t(2048) * 256 * 64;
-constexpr int kItemMin = 512, kItemMax = 2048;
+// Heavy items of 2048 samples left the last round of each launch uneven (d <= 64:
+// 100 us a launch over a whole run, 94 with 1024 and 98 with 512, which loads the
+// centroids twice as often; d <= 32: 65 with 2048, 61 with 1024).
+constexpr int64_t kItemMacs = int64_t(2048) * 256 * 16;
+constexpr int kItemMin = 1024, kItemMax = 2048;
 // assignment block: one 32-sample column block per wave; 16 waves, or 8 for
 // d > 32, whose 32 x-registers per lane do not fit the 128 VGPRs of 16 waves
 constexpr int assign_threads(int KS) { return KS <= 16 ? 1024 : 512; }
@@ -67,7 +70,7 @@ constexpr int kFB = 256;                  // finalize / per-fit block
 
 struct BState {
   int it, active, cur, n_empty;
-  int seg_items, seg_base;
+  int seg_items;
   double shift;
   double inertia;
 };
@@ -88,8 +91,8 @@ struct BFit {
   float *dist;      // (n) relocation distances / per-sample inertia
   u64 *sums;        // ((d + 1) k) int64 fixed-point sums
   float *scale;     // (d + 1) fixed-point scales
-  float *hn, *sizes;                        // (k + 1)
-  int *list, *totals, *cursor, *start, *citems;  // (k + 1)
+  float *hn;                               // (k + 1)
+  int *totals, *cursor, *start, *citems;   // (k + 1)
   int *nonfinite;   // (1) 0: fixed-point sums; 1: inf/NaN; 2: range too wide
   unsigned *maxbits;  // (d + 2) range maxima (fixed_point.hpp)
   u64 *estat;         // (2 (d + 1)) exponent sums and counts (fixed_point.hpp)
@@ -132,11 +135,22 @@ __device__ inline double block_sum256(double v, double *lds) {
 }
 
 // ---- half norms -------------------------------------------------------------
+// Also clears the sums and counts that the iteration's update adds to (a
+// launch of its own, 4.7 us, only for that before); all: the epilogue, which has
+// no update.
 __global__ void __launch_bounds__(kFB)
     bt_hn_krn(const BFit *__restrict__ fits, int all) {
   const int f = blockIdx.x;
   if (!all && !fits[f].st[0].active) return;
   const BFit F = fits[f];
+  if (!all) {
+    const int m = (F.d + 1) * F.k;
+    for (int i = threadIdx.x; i < m; i += kFB) F.sums[i] = 0ull;
+    for (int c = threadIdx.x; c <= F.k; c += kFB) {
+      F.totals[c] = 0;
+      F.cursor[c] = 0;
+    }
+  }
   const float *C = cbuf(F, fits[f].st[0].cur);
   constexpr int kU = 8;  // loads in flight per thread; the fmaf order is j = 0, 1, ...
   for (int c = threadIdx.x; c < F.k; c += kFB) {
@@ -585,19 +599,6 @@ __global__ void __launch_bounds__(NT)
 }
 
 // ---- update -------------------------------------------------------------------
-__global__ void __launch_bounds__(kFB)
-    bt_zero_krn(const BFit *__restrict__ fits) {
-  const int f = blockIdx.x;
-  if (!fits[f].st[0].active) return;
-  const BFit F = fits[f];
-  const int64_t m = (int64_t)(F.d + 1) * F.k;
-  for (int64_t i = threadIdx.x; i < m; i += kFB) F.sums[i] = 0ull;
-  for (int c = threadIdx.x; c <= F.k; c += kFB) {
-    F.totals[c] = 0;
-    F.cursor[c] = 0;
-  }
-}
-
 __global__ void __launch_bounds__(256)
     bt_hist_krn(const BFit *__restrict__ fits, const CItem *__restrict__ items) {
   __shared__ int h[kMaxK];
@@ -669,38 +670,6 @@ __global__ void __launch_bounds__(kFB)
   }
 }
 
-// exclusive scan of the fits' segment-item counts (one block)
-__global__ void __launch_bounds__(1024)
-    bt_fit_scan_krn(int n_fits, const BFit *__restrict__ fits, int *__restrict__ total) {
-  __shared__ int ws[1024 / kWave];
-  __shared__ int carry;
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-  if (tid == 0) carry = 0;
-  __syncthreads();
-  for (int f0 = 0; f0 < n_fits; f0 += 1024) {
-    const int f = f0 + tid;
-    const int v = (f < n_fits) ? fits[f].st[0].seg_items : 0;
-    int incl = v;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const int t = __shfl_up(incl, o, kWave);
-      if (lane >= o) incl += t;
-    }
-    if (lane == kWave - 1) ws[wave] = incl;
-    __syncthreads();
-    int p = 0, tot = 0;
-    for (int w2 = 0; w2 < 1024 / kWave; ++w2) {
-      if (w2 < wave) p += ws[w2];
-      tot += ws[w2];
-    }
-    if (f < n_fits) fits[f].st[0].seg_base = carry + p + incl - v;
-    __syncthreads();
-    if (tid == 0) carry += tot;
-    __syncthreads();
-  }
-  if (tid == 0) total[0] = carry;
-}
-
 __global__ void __launch_bounds__(256)
     bt_scatter_krn(const BFit *__restrict__ fits, const CItem *__restrict__ items) {
   __shared__ int h[kMaxK];
@@ -731,17 +700,32 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// Segment items of every active fit, flattened: map[seg_base + i] = {fit,
+// Segment items of every active fit, flattened: map[base + i] = {fit,
 // cluster, first member (position in perm), member count} for item i of the
 // fit (items of cluster c are citems[c] .. citems[c + 1] - 1, each up to
-// kMembers consecutive members of the cluster).
+// kMembers consecutive members of the cluster).  Every block sums the counts of
+// the fits before its own for base (one load a thread for 256 fits, instead of a
+// scan launch of 4.7 us in front); the last one writes the total.
 __global__ void __launch_bounds__(kFB)
-    bt_seg_map_krn(const BFit *__restrict__ fits, int4 *__restrict__ map) {
+    bt_seg_map_krn(const BFit *__restrict__ fits, int4 *__restrict__ map,
+                   int *__restrict__ total) {
   __shared__ int ci[kMaxK + 1];
+  __shared__ int part[kFB / kWave];
   const int f = blockIdx.x;
-  if (!fits[f].st[0].active) return;
+  const bool active = fits[f].st[0].active != 0, last = f == (int)gridDim.x - 1;
+  if (!active && !last) return;
+  int before = 0;
+  for (int g = threadIdx.x; g < f; g += kFB) before += fits[g].st[0].seg_items;
+  for (int o = kWave / 2; o > 0; o >>= 1) before += __shfl_xor(before, o, kWave);
+  if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = before;
+  __syncthreads();
+  int base = 0;
+  for (int w = 0; w < kFB / kWave; ++w) base += part[w];
+  const int items = fits[f].st[0].seg_items;   // 0 for an inactive fit
+  if (last && threadIdx.x == 0) total[0] = base + items;
+  if (!active) return;
   const BFit F = fits[f];
-  const int k = F.k, base = fits[f].st[0].seg_base, items = fits[f].st[0].seg_items;
+  const int k = F.k;
   for (int c = threadIdx.x; c <= k; c += kFB) ci[c] = F.citems[c];
   __syncthreads();
   for (int i = threadIdx.x; i < items; i += kFB) {
@@ -820,38 +804,16 @@ __global__ void __launch_bounds__(kSegThreads)
 }
 
 // ---- empty clusters and relocation ----------------------------------------------
-// Ascending list of the fit's empty clusters (a zero int64 count is exactly a
-// zero size after conversion) and n_empty.
-__global__ void __launch_bounds__(kFB)
-    bt_empty_krn(const BFit *__restrict__ fits) {
-  __shared__ int wcount[kFB / kWave];
-  const int f = blockIdx.x;
-  if (!fits[f].st[0].active) return;
-  const BFit F = fits[f];
-  const int tid = threadIdx.x;  // k <= 256 = kFB
-  const bool empty =
-      (tid < F.k) && (F.sums[(int64_t)F.d * F.k + tid] == 0ull);
-  const uint64_t mask = __ballot(empty);
-  const int lane = tid & (kWave - 1), w = tid / kWave;
-  const int before_in_wave = __popcll(mask & ((1ull << lane) - 1ull));
-  if (lane == 0) wcount[w] = __popcll(mask);
-  __syncthreads();
-  int before = 0, tot = 0;
-  for (int i = 0; i < kFB / kWave; ++i) {
-    before += (i < w) ? wcount[i] : 0;
-    tot += wcount[i];
-  }
-  if (empty) F.list[before + before_in_wave] = tid;
-  if (tid == 0) fits[f].st[0].n_empty = tot;
-}
-
+// A zero int64 weight sum is exactly a zero size after conversion.
 // squared distance (unit weights) of every sample to its current centroid,
 // for fits with an empty cluster (the single-fit inertia arithmetic)
 __global__ void __launch_bounds__(256)
     bt_dist_krn(const BFit *__restrict__ fits, const CItem *__restrict__ items) {
   const CItem item = items[blockIdx.x];
-  if (!fits[item.fit].st[0].active || fits[item.fit].st[0].n_empty == 0) return;
+  if (!fits[item.fit].st[0].active) return;
   const BFit F = fits[item.fit];
+  const int cl = threadIdx.x;   // k <= 256
+  if (!__syncthreads_or(cl < F.k && F.sums[(int64_t)F.d * F.k + cl] == 0ull)) return;
   const float *C = cbuf(F, fits[item.fit].st[0].cur);
   for (int j = threadIdx.x; j < item.count; j += 256) {
     const int64_t s = item.first + j;
@@ -882,16 +844,27 @@ __global__ void __launch_bounds__(256)
 }
 
 // ---- finalize (one block per fit) ----------------------------------------------
-__global__ void __launch_bounds__(kFB)
+// One CU per fit, so bound by that CU's instructions and round trips: 16 waves,
+// the sums, quotients and differences in LDS from one step to the next, no integer
+// division per value, and the FP64 division by a scale (a power of two) as the
+// exact product with its reciprocal.  d = 64, k = 256: 34 us with 4 waves and
+// every step through memory, 17 us here.
+constexpr int kFT = 1024;
+constexpr size_t kFinalizeLds = sizeof(float) * (size_t)(kMaxD + 1) * kMaxK;
+__global__ void __launch_bounds__(kFT)
     bt_finalize_krn(const BFit *__restrict__ fits) {
-  __shared__ double red[kFB / kWave];
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  float *cs = reinterpret_cast<float *>(lds_raw);   // [d + 1][k]: centroids, then sizes
+  __shared__ double red[kFT / kWave];
+  __shared__ double inv_scale[kMaxD + 1];
   __shared__ int hist[256];
   __shared__ unsigned sel_prefix;
   __shared__ int sel_left, n_sel, n_eq_taken;
-  __shared__ int wcnt[kFB / kWave];
+  __shared__ int wcnt[kFT / kWave];
   __shared__ unsigned skey[kMaxK];
   __shared__ int sidx[kMaxK];
   __shared__ int order[kMaxK];
+  __shared__ int list[kMaxK];
   const int f = blockIdx.x;
   if (!fits[f].st[0].active) return;
   const BFit F = fits[f];
@@ -900,42 +873,49 @@ __global__ void __launch_bounds__(kFB)
   const int cur = fits[f].st[0].cur;
   const float *Cc = cbuf(F, cur);
   float *Cn = cbuf(F, cur ^ 1);
-  float *sizes = F.sizes;
-  const int *list = F.list;
-  const float *sc = F.scale;
   const int dk = d * k;  // <= kMaxD * kMaxK
-  // Each loop below issues kU loads per thread before using any of them
-  // (one round trip per kU elements, not per element); the arithmetic and
-  // its order per element are unchanged.
+  float *sizes = cs + dk;
+  if (tid <= d) inv_scale[tid] = 1.0 / (double)F.scale[tid];
+  // ascending list of the empty clusters
+  const bool empty = tid < k && F.sums[dk + tid] == 0ull;
+  const unsigned long long emask = __ballot(empty);
+  if ((tid & (kWave - 1)) == 0) wcnt[tid / kWave] = __popcll(emask);
+  __syncthreads();
+  int n_empty = 0, e_before = 0;
+  for (int w = 0; w < kMaxK / kWave; ++w) {
+    e_before += w < tid / kWave ? wcnt[w] : 0;
+    n_empty += wcnt[w];
+  }
+  if (empty) list[e_before + __popcll(emask & ((1ull << (tid & (kWave - 1))) - 1ull))] = tid;
+  // Each loop below issues kU loads per thread before using any of them; the
+  // row of value i is followed from step to step.
   constexpr int kU = 8;
+  const int row0 = tid / k, col0 = tid - row0 * k;
+  const int row_step = kFT / k, col_step = kFT - row_step * k;
   // sums -> centroid sums and sizes (the single-slot partial reduction)
-  for (int i0 = tid; i0 < dk + k; i0 += kU * kFB) {
-    long long q[kU];
-    float sv[kU];
+  {
+    int row = row0, c = col0;
+    for (int i0 = tid; i0 < dk + k; i0 += kU * kFT) {
+      long long q[kU];
 #pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int i = i0 + u * kFB;
-      q[u] = 0;
-      sv[u] = 1.f;
-      if (i < dk + k) {
-        q[u] = (long long)F.sums[i];
-        sv[u] = sc[i / k];
+      for (int u = 0; u < kU; ++u) {
+        const int i = i0 + u * kFT;
+        q[u] = i < dk + k ? (long long)F.sums[i] : 0;
       }
-    }
 #pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int i = i0 + u * kFB;
-      if (i < dk + k) {
-        const float v = (float)((double)q[u] / (double)sv[u]);
-        if (i < dk)
-          Cn[i] = v;
-        else
-          sizes[i - dk] = v;
+      for (int u = 0; u < kU; ++u) {
+        const int i = i0 + u * kFT;
+        if (i < dk + k) cs[i] = (float)((double)q[u] * inv_scale[row]);
+        row += row_step;
+        c += col_step;
+        if (c >= k) {
+          c -= k;
+          ++row;
+        }
       }
     }
   }
   __syncthreads();
-  const int n_empty = fits[f].st[0].n_empty;
   if (n_empty > 0) {
     // the m farthest samples by (distance desc, index asc): radix-select
     // the m-th largest distance (non-negative floats order as their bits),
@@ -948,11 +928,11 @@ __global__ void __launch_bounds__(kFB)
       sel_left = m;
     }
     for (int shift = 24; shift >= 0; shift -= 8) {
-      hist[tid] = 0;
+      if (tid < 256) hist[tid] = 0;
       __syncthreads();
       const unsigned pre = sel_prefix;
       const unsigned hi_mask = (shift == 24) ? 0u : (0xffffffffu << (shift + 8));
-      for (int64_t s = tid; s < n; s += kFB) {
+      for (int64_t s = tid; s < n; s += kFT) {
         const unsigned key = __float_as_uint(dist[s]);
         if ((key & hi_mask) == pre) atomicAdd(&hist[(key >> shift) & 255u], 1);
       }
@@ -975,9 +955,9 @@ __global__ void __launch_bounds__(kFB)
       n_eq_taken = 0;
     }
     __syncthreads();
-    // gather in index order (chunks of kFB samples, ballot ranks)
+    // gather in index order (chunks of kFT samples, ballot ranks)
     const int lane = tid & (kWave - 1), w = tid / kWave;
-    for (int64_t c0 = 0; c0 < n; c0 += kFB) {
+    for (int64_t c0 = 0; c0 < n; c0 += kFT) {
       const int64_t s = c0 + tid;
       const unsigned key = (s < n) ? __float_as_uint(dist[s]) : 0u;
       const bool gt = (s < n) && key > thr;
@@ -986,7 +966,7 @@ __global__ void __launch_bounds__(kFB)
       if (lane == 0) wcnt[w] = __popcll(meq);
       __syncthreads();
       int before = 0, tot = 0;
-      for (int i = 0; i < kFB / kWave; ++i) {
+      for (int i = 0; i < kFT / kWave; ++i) {
         before += (i < w) ? wcnt[i] : 0;
         tot += wcnt[i];
       }
@@ -1001,7 +981,7 @@ __global__ void __launch_bounds__(kFB)
       if (tid == 0) n_eq_taken += tot;
       __syncthreads();
     }
-    for (int i = tid; i < m; i += kFB) {
+    for (int i = tid; i < m; i += kFT) {
       int rank = 0;
       for (int j = 0; j < m; ++j)
         rank += (skey[j] > skey[i]) || (skey[j] == skey[i] && sidx[j] < sidx[i]);
@@ -1009,15 +989,15 @@ __global__ void __launch_bounds__(kFB)
     }
     __syncthreads();
     // move w x of the chosen samples (in order) into the empty clusters
-    for (int fe = tid; fe < d; fe += kFB) {
+    for (int fe = tid; fe < d; fe += kFT) {
       for (int j = 0; j < m; ++j) {
         const int s = order[j];
         const int p = F.labels[s];
         const int e = list[j];
         const float ws = F.w[s];
         const float add = F.X[(int64_t)fe * n + s] * ws;
-        Cn[(int64_t)fe * k + p] -= add;
-        Cn[(int64_t)fe * k + e] = add;
+        cs[fe * k + p] -= add;
+        cs[fe * k + e] = add;
         if (fe == 0) {
           sizes[p] -= ws;
           sizes[e] = ws;
@@ -1027,49 +1007,42 @@ __global__ void __launch_bounds__(kFB)
     __syncthreads();
   }
   // divide, then shifts and their sum in the single-fit order
-  for (int i0 = tid; i0 < dk; i0 += kU * kFB) {
-    float a[kU], b[kU];
+  {
+    int row = row0, c = col0;
+    for (int i0 = tid; i0 < dk; i0 += kU * kFT) {
+      float old[kU];
 #pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int i = i0 + u * kFB;
-      a[u] = 0.f;
-      b[u] = 1.f;
-      if (i < dk) {
-        a[u] = Cn[i];
-        b[u] = sizes[i % k];
+      for (int u = 0; u < kU; ++u) {
+        const int i = i0 + u * kFT;
+        old[u] = i < dk ? Cc[i] : 0.f;
       }
-    }
 #pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int i = i0 + u * kFB;
-      if (i < dk) Cn[i] = a[u] / b[u];
+      for (int u = 0; u < kU; ++u) {
+        const int i = i0 + u * kFT;
+        if (i < dk) {
+          const float v = cs[i] / sizes[c];
+          Cn[i] = v;
+          cs[i] = old[u] - v;
+        }
+        row += row_step;
+        c += col_step;
+        if (c >= k) {
+          c -= k;
+          ++row;
+        }
+      }
     }
   }
   __syncthreads();
   double acc = 0.0;
-  for (int c = tid; c < k; c += kFB) {
+  if (tid < k) {
     float s2 = 0.f;
-    for (int j0 = 0; j0 < d; j0 += kU) {
-      float a[kU], b[kU];
-#pragma unroll
-      for (int u = 0; u < kU; ++u) {
-        const int j = j0 + u;
-        a[u] = 0.f;
-        b[u] = 0.f;
-        if (j < d) {
-          a[u] = Cc[(int64_t)j * k + c];
-          b[u] = Cn[(int64_t)j * k + c];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < kU; ++u) {
-        if (j0 + u < d) {
-          const float diff = a[u] - b[u];
-          s2 = fmaf(diff, diff, s2);
-        }
-      }
+#pragma unroll 8
+    for (int j = 0; j < d; ++j) {
+      const float diff = cs[j * k + tid];
+      s2 = fmaf(diff, diff, s2);
     }
-    acc += (double)s2;
+    acc = (double)s2;
   }
   const double tot = block_sum256(acc, red);
   if (tid == 0) {
@@ -1077,6 +1050,7 @@ __global__ void __launch_bounds__(kFB)
     S.shift = tot;
     S.cur = cur ^ 1;
     S.it += 1;
+    S.n_empty = n_empty;
     const float shift_t = (float)tot;
     S.active = (S.it < F.max_iter) && (shift_t > F.tol);
     fits[f].st[0] = S;
@@ -1358,7 +1332,7 @@ inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
 // Byte layout of one fit's workspace arena.
 struct Arena {
-  size_t st, xr, perm, dist, sums, scale, hn, sizes, list, totals, cursor, start,
+  size_t st, xr, perm, dist, sums, scale, hn, totals, cursor, start,
       citems, nonfinite, maxbits, estat, total;
   Arena(int64_t n, int64_t d, int64_t k) {
     size_t o = 0;
@@ -1374,8 +1348,6 @@ struct Arena {
     sums = take(sizeof(u64) * (size_t)(d + 1) * k);
     scale = take(sizeof(float) * (size_t)(d + 1));
     hn = take(sizeof(float) * (size_t)(k + 1));
-    sizes = take(sizeof(float) * (size_t)(k + 1));
-    list = take(sizeof(int) * (size_t)(k + 1));
     totals = take(sizeof(int) * (size_t)(k + 1));
     cursor = take(sizeof(int) * (size_t)(k + 1));
     start = take(sizeof(int) * (size_t)(k + 1));
@@ -1545,8 +1517,6 @@ int64_t BatchEngine::add(const BatchedFit &f, bool check_now, bool defer_prep,
   F.sums = reinterpret_cast<u64 *>(b + A.sums);
   F.scale = reinterpret_cast<float *>(b + A.scale);
   F.hn = reinterpret_cast<float *>(b + A.hn);
-  F.sizes = reinterpret_cast<float *>(b + A.sizes);
-  F.list = reinterpret_cast<int *>(b + A.list);
   F.totals = reinterpret_cast<int *>(b + A.totals);
   F.cursor = reinterpret_cast<int *>(b + A.cursor);
   F.start = reinterpret_cast<int *>(b + A.start);
@@ -1710,28 +1680,26 @@ void BatchEngine::iteration(hipStream_t q, hipEvent_t ev_a0, hipEvent_t ev_a1) {
   launch_assign_bucket<32>(dF, ai_d_[2]->as<AItem>(), (int)ai_[2].size(), 0, q, mixed_,
                            assign_shape_);
   if (ev_a1 != nullptr) KMD_HIP_CHECK(hipEventRecord(ev_a1, q));
-  hipLaunchKernelGGL(bt_zero_krn, dim3(nf), dim3(kFB), 0, q, dF);
-  KMD_LAUNCH_CHECK();
   hipLaunchKernelGGL(bt_hist_krn, dim3(nci), dim3(256), 0, q, dF, ci_d_->as<CItem>());
   KMD_LAUNCH_CHECK();
   hipLaunchKernelGGL(bt_cluster_scan_krn, dim3(nf), dim3(kFB), 0, q, dF);
   KMD_LAUNCH_CHECK();
-  hipLaunchKernelGGL(bt_fit_scan_krn, dim3(1), dim3(1024), 0, q, nf, dF,
-                     seg_total_->as<int>());
-  KMD_LAUNCH_CHECK();
   hipLaunchKernelGGL(bt_scatter_krn, dim3(nci), dim3(256), 0, q, dF,
                      ci_d_->as<CItem>());
   KMD_LAUNCH_CHECK();
-  hipLaunchKernelGGL(bt_seg_map_krn, dim3(nf), dim3(kFB), 0, q, dF, seg_map_->as<int4>());
+  hipLaunchKernelGGL(bt_seg_map_krn, dim3(nf), dim3(kFB), 0, q, dF, seg_map_->as<int4>(),
+                     seg_total_->as<int>());
   KMD_LAUNCH_CHECK();
   hipLaunchKernelGGL(bt_segsum_krn, dim3((unsigned)seg_bound_), dim3(kSegThreads), 0, q, dF,
                      seg_map_->as<const int4>(), seg_total_->as<int>());
   KMD_LAUNCH_CHECK();
-  hipLaunchKernelGGL(bt_empty_krn, dim3(nf), dim3(kFB), 0, q, dF);
-  KMD_LAUNCH_CHECK();
   hipLaunchKernelGGL(bt_dist_krn, dim3(nci), dim3(256), 0, q, dF, ci_d_->as<CItem>());
   KMD_LAUNCH_CHECK();
-  hipLaunchKernelGGL(bt_finalize_krn, dim3(nf), dim3(kFB), 0, q, dF);
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void *>(&bt_finalize_krn),
+      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFinalizeLds);
+  KMD_HIP_CHECK(attr);
+  hipLaunchKernelGGL(bt_finalize_krn, dim3(nf), dim3(kFT), kFinalizeLds, q, dF);
   KMD_LAUNCH_CHECK();
 }
 
