@@ -1386,22 +1386,49 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// Counting and scattering by label: few blocks of many threads.  Every block adds
+// to every cluster's counter once, and device atomics of one address serialise, so
+// a block takes at least 16K samples; its time is then the round trips of its
+// labels, so 1024 threads have 16 of them in flight each (256 threads with one at
+// a time, n = 500K, k = 512: 15.3 us counting and 24.2 scattering, 4.6 and
+// 12.0 here).
+constexpr int kLabelThreads = 1024;
+constexpr int kLabelRun = 16;
+
+// fn(sample, label) over samples beg .. end - 1
+template <typename I, typename Fn>
+__device__ inline void for_labels(const I *__restrict__ labels, int64_t beg, int64_t end,
+                                  Fn &&fn) {
+  for (int64_t s0 = beg + threadIdx.x; s0 < end; s0 += kLabelThreads * kLabelRun) {
+    int lab[kLabelRun];
+#pragma unroll
+    for (int u = 0; u < kLabelRun; ++u) {
+      const int64_t s = s0 + u * kLabelThreads;
+      lab[u] = s < end ? (int)labels[s] : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < kLabelRun; ++u) {
+      const int64_t s = s0 + u * kLabelThreads;
+      if (s < end) fn(s, lab[u]);
+    }
+  }
+}
+
 // totals[c] += number of samples with label c in block b's chunk (one
 // global atomic per block and non-empty cluster)
 template <typename I>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kLabelThreads)
     label_hist_krn(int64_t n, int k, int64_t chunk, const I *__restrict__ labels,
                    int *__restrict__ totals, const int *skip) {
   if (skip != nullptr && *skip != 0) return;
   extern __shared__ int h[];
-  for (int c = threadIdx.x; c < k; c += 256) h[c] = 0;
+  for (int c = threadIdx.x; c < k; c += kLabelThreads) h[c] = 0;
   __syncthreads();
   const int64_t beg = (int64_t)blockIdx.x * chunk;
   const int64_t end = min(n, beg + chunk);
-  for (int64_t s = beg + threadIdx.x; s < end; s += 256)
-    atomicAdd(&h[(int)labels[s]], 1);
+  for_labels(labels, beg, end, [&](int64_t, int l) { atomicAdd(&h[l], 1); });
   __syncthreads();
-  for (int c = threadIdx.x; c < k; c += 256)
+  for (int c = threadIdx.x; c < k; c += kLabelThreads)
     if (h[c] != 0) atomicAdd(&totals[c], h[c]);
 }
 
@@ -1465,38 +1492,35 @@ __global__ void __launch_bounds__(1024)
 // label c, where base is the block's share of cluster c claimed from
 // cursor[c] (the order inside a cluster is irrelevant: the sums are exact)
 template <typename I>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kLabelThreads)
     scatter_krn(int64_t n, int k, int64_t chunk, const I *__restrict__ labels,
                 const int *__restrict__ start, int *__restrict__ cursor,
                 int *__restrict__ perm, const int *skip) {
   if (skip != nullptr && *skip != 0) return;
   extern __shared__ int h[];
-  for (int c = threadIdx.x; c < k; c += 256) h[c] = 0;
+  for (int c = threadIdx.x; c < k; c += kLabelThreads) h[c] = 0;
   __syncthreads();
   const int64_t beg = (int64_t)blockIdx.x * chunk;
   const int64_t end = min(n, beg + chunk);
-  for (int64_t s = beg + threadIdx.x; s < end; s += 256)
-    atomicAdd(&h[(int)labels[s]], 1);
+  for_labels(labels, beg, end, [&](int64_t, int l) { atomicAdd(&h[l], 1); });
   __syncthreads();
-  for (int c = threadIdx.x; c < k; c += 256)
+  for (int c = threadIdx.x; c < k; c += kLabelThreads)
     h[c] = (h[c] != 0) ? start[c] + atomicAdd(&cursor[c], h[c]) : 0;
   __syncthreads();
-  for (int64_t s = beg + threadIdx.x; s < end; s += 256) {
-    const int pos = atomicAdd(&h[(int)labels[s]], 1);
-    perm[pos] = (int)s;
+  for_labels(labels, beg, end,
+             [&](int64_t s, int l) { perm[atomicAdd(&h[l], 1)] = (int)s; });
+}
+
+// sums[0 .. m) and counts[0 .. mc) to zero
+__global__ void __launch_bounds__(256)
+    clear_update_krn(int64_t m, u64 *sums, int64_t mc, int *counts) {
+  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < m + mc;
+       i += (int64_t)gridDim.x * 256) {
+    if (i < m)
+      sums[i] = 0ull;
+    else
+      counts[i - m] = 0;
   }
-}
-
-__global__ void __launch_bounds__(256) fill_i32_krn(int64_t m, int *p) {
-  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < m;
-       i += (int64_t)gridDim.x * 256)
-    p[i] = 0;
-}
-
-__global__ void __launch_bounds__(256) fill_u64_krn(int64_t m, u64 *p) {
-  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < m;
-       i += (int64_t)gridDim.x * 256)
-    p[i] = 0ull;
 }
 
 // One work item = up to kMembers members of one cluster; thread f sums
@@ -2020,22 +2044,21 @@ void launch_tiled_update(int64_t n, int64_t d, int64_t k, const float *X_r,
   int *perm = items + (k + 1);                     // [n]
   u64 *S = reinterpret_cast<u64 *>(sums);
   const int64_t m = (d + 1) * k;
-  hipLaunchKernelGGL(fill_u64_krn,
-                     dim3((unsigned)std::min<int64_t>(1024, ceil_div<int64_t>(m, 256))),
-                     dim3(256), 0, s, m, S);
+  const int64_t mc = n > 0 ? 2 * (k + 1) : 0;
+  hipLaunchKernelGGL(clear_update_krn,
+                     dim3((unsigned)std::min<int64_t>(1024, ceil_div<int64_t>(m + mc, 256))),
+                     dim3(256), 0, s, m, S, mc, totals);
   KMD_LAUNCH_CHECK();
   if (n <= 0) return;
-  hipLaunchKernelGGL(fill_i32_krn, dim3(8), dim3(256), 0, s, 2 * (k + 1), totals);
-  KMD_LAUNCH_CHECK();
   const size_t hist_lds = sizeof(int) * (size_t)k;
   require(hist_lds <= kLdsPerCu, "tiled update: too many clusters for LDS counts");
-  hipLaunchKernelGGL((label_hist_krn<I>), dim3((unsigned)nb), dim3(256), hist_lds, s,
+  hipLaunchKernelGGL((label_hist_krn<I>), dim3((unsigned)nb), dim3(kLabelThreads), hist_lds, s,
                      n, (int)k, chunk, labels, totals, skip);
   KMD_LAUNCH_CHECK();
   hipLaunchKernelGGL(cluster_scan_krn, dim3(1), dim3(1024), 0, s, (int)k, kMembers,
                      totals, start, items, skip);
   KMD_LAUNCH_CHECK();
-  hipLaunchKernelGGL((scatter_krn<I>), dim3((unsigned)nb), dim3(256), hist_lds, s, n,
+  hipLaunchKernelGGL((scatter_krn<I>), dim3((unsigned)nb), dim3(kLabelThreads), hist_lds, s, n,
                      (int)k, chunk, labels, start, cursor, perm, skip);
   KMD_LAUNCH_CHECK();
   // at most n / kMembers + k work items; blocks beyond items[k] return
