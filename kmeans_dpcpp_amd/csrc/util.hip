@@ -266,18 +266,22 @@ __global__ void __launch_bounds__(kTailThreads)
   int &last = wave_counts[kTailThreads / kWave];
   const int tid = threadIdx.x, wave = tid / kWave;
   const int64_t d = a.d, k = a.k;
-  // the first sizes are read beside the loop's state
-  const T size0 = tid < k ? a.sizes[tid] : T(1);
-  if (!a.relocated && a.state->stop != 0) return;
-
   if (!a.relocated) {
+    // Whether the loop has stopped is read by one thread, so that a block goes
+    // on or returns as one: with clusters empty, block 0 sets `stop` as soon as
+    // it has listed them, while blocks that start later still read it.  Both
+    // answers end such a block (a stopped loop, or its own look at the sizes),
+    // and no block of that launch takes a ticket.
+    if (tid == 0)
+      last = __hip_atomic_load(&a.state->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // every block looks for empty clusters itself; block 0 lists them
-    bool any = size0 == T(0);
+    bool any = tid < k && a.sizes[tid] == T(0);
     for (int64_t c = tid + kTailThreads; c < k; c += kTailThreads)
       any |= a.sizes[c] == T(0);
     const uint64_t any_mask = __ballot(any);
     if (lane_id() == 0) wave_counts[wave] = any_mask != 0;
     __syncthreads();
+    if (last != 0) return;
     int n_any = 0;
     for (int i = 0; i < kTailThreads / kWave; ++i) n_any += wave_counts[i];
     if (n_any != 0) {
@@ -304,8 +308,8 @@ __global__ void __launch_bounds__(kTailThreads)
         st->n_empty = found;
         st->rescored += a.rescored != nullptr ? a.rescored[0] : 0;
         st->done += 1;
-        // the other blocks read sizes, not this
-        st->stop = kLoopEmpty;
+        __hip_atomic_store(&st->stop, kLoopEmpty, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
         publish(a.host, *st);
       }
       return;
