@@ -370,6 +370,11 @@ int kmd_autotune(int dtype, int itype, int precision, int64_t n_samples,
  * back to the autotuner's table, else the automatic choice; shape as in
  * kmd_autotune). */
 int kmd_set_tuning(int path, int blocks_per_cu, int shape);
+/* Iterations that the driver calls of the calling thread enqueue before they
+ * know how the one in front ended: 1 (the default; also for a value outside
+ * 0 .. 1) or 0, for fits that share the GPU with other streams, which then get
+ * on between two iterations.  The results are the same.  Returns what it was. */
+int kmd_set_run_ahead(int iterations);
 
 /* ---- estimator front-end: data preparation and seeding ----------------
  * No counterpart in the reference, whose driver takes init_centroids_t from

@@ -1068,6 +1068,8 @@ int kmd_fp8_roundtrip(int64_t n, const float *in, float *out, kmd_stream_t strea
   });
 }
 
+int kmd_set_run_ahead(int iterations) { return set_run_ahead(iterations); }
+
 int kmd_set_tuning(int path, int blocks_per_cu, int shape) {
   return guarded([&] {
     require(path >= -1 && path <= 2, "path must be -1, 0, 1 or 2");

@@ -380,10 +380,22 @@ static std::unique_ptr<LloydWorkspace<T, I>> make_workspace(int64_t n,
   return ws;
 }
 
-// Iterations enqueued ahead of the last one known to have finished.  Enough
-// to cover the launches of the next ones on the smallest shapes, few enough
-// that what is left to skip when the loop stops costs little.
-constexpr int kAhead = 3;
+// Iterations enqueued ahead of the last one known to have finished.  One covers
+// the launches of the next (50,000 x 14 x 127, 18 us of kernels an iteration: 883
+// us a fit, 902 with three ahead; no fit tried was faster with three), and every
+// further one is a kernel of the whole chip that other streams wait behind.
+// Beside the server's engine three made a stream of 200 requests/s wait 43 ms
+// (median) where one makes it 25 and none 13, and a saturated one 0.56 / 0.41 /
+// 0.20 s, at 278 / 292 / 299 fits/s; a fit alone takes 1.7 % longer with none
+// (2M x 96 x 512).  So a thread whose fits share the GPU can ask for none.
+constexpr int kAhead = 1;
+thread_local int t_run_ahead = kAhead;
+
+int set_run_ahead(int iterations) {
+  const int before = t_run_ahead;
+  t_run_ahead = iterations < 0 || iterations > kAhead ? kAhead : iterations;
+  return before;
+}
 
 // Optional timing of the fused-step kernel with HIP events on the driver's
 // stream: one event pair per iteration that can be in flight, read back once
@@ -767,7 +779,7 @@ static void driver_impl(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
     launch_step_tail<T, I>(tail, s);
   };
   // verbose mode prints between iterations: nothing is enqueued ahead there
-  const int ahead = verbose ? 0 : kAhead;
+  const int ahead = verbose ? 0 : t_run_ahead;
   const bool resident = std::is_same<T, float>::value && ws.fast &&
                         ws.mixed_terms == 0 && !ws.tiled;
   auto finish = [&](double total, int64_t rescored) {

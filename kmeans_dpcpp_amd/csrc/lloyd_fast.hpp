@@ -27,6 +27,9 @@ std::vector<TuneResult> autotune_lloyd(int64_t n, int64_t d, int64_t k,
                                        int precision, int iters, hipStream_t s);
 // Process-wide override of the tuning choice (path < 0 clears it).
 void set_tuning_override(int path, int blocks_per_cu, int shape = 0);
+// Iterations that the calling thread's driver calls enqueue ahead (driver.hip);
+// returns what it was.
+int set_run_ahead(int iterations);
 
 // Launch plan of a persistent fused-step kernel: grid size, dynamic LDS and
 // whether centroid sums are privatised in LDS.

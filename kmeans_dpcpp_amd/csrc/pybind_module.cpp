@@ -1326,6 +1326,7 @@ PYBIND11_MODULE(_kmeans_dpcpp_amd, m) {
         },
         "out = in rounded to FP8 e4m3 and back with the FP8 kernels' conversion.",
         py::arg("in"), py::arg("out"), py::arg("sycl_queue") = py::none());
+  m.def("_set_run_ahead", &kmd_set_run_ahead);
   m.def("set_tuning",
         [](int path, int blocks_per_cu, int shape) {
           check_rc(kmd_set_tuning(path, blocks_per_cu, shape));

@@ -291,6 +291,9 @@ class Server:
         from . import Stream
         if not hasattr(self._local, "stream"):  # one stream per worker thread
             self._local.stream = Stream()
+            # the engine's launches get on between two iterations of this
+            # thread's fits
+            _native._set_run_ahead(0)
         stream = self._local.stream
         X = req.X_t
         n, d, k = req.shape

@@ -97,3 +97,27 @@ def test_server_results_equal_alone_under_a_budget(kd, torch_dev, small_precisio
         same((to_np(r.labels), to_np(r.centroids), r.n_iter, r.inertia),
              alone(kd, X, w, init, 1e-4, mi))
     assert sum(1 for r in reqs if not r.batched) == 1
+
+
+def test_large_fits_of_the_server_do_not_run_ahead(kd, torch_dev):
+    """An iteration that a worker enqueues ahead is a kernel of the whole chip
+    which the engine's launches wait behind: workers enqueue none, the caller's
+    own thread one as before, and the fit is the same either way."""
+    from kmeans_dpcpp_amd import _kmeans_dpcpp_amd as native
+    from kmeans_dpcpp_amd import serving
+    seen = []
+
+    class Watched(serving.Server):
+        def _run_large(self, req):
+            out = super()._run_large(req)
+            seen.append(native._set_run_ahead(0))
+            return out
+
+    X, w, init = problem(20_000, 96, 40, 77)
+    init[:, [3, 11]] = 1e3            # clusters to relocate in the first iteration
+    before = native._set_run_ahead(1)
+    with Watched(1 << 30) as srv:
+        req = srv.submit(X, w, init, tol=1e-4, max_iter=30)
+        lab, res, it, inertia = req.result(timeout=60)
+    assert not req.batched and seen == [0] and before == native._set_run_ahead(1) == 1
+    same((to_np(lab), to_np(res), it, inertia), alone(kd, X, w, init, 1e-4, 30))
