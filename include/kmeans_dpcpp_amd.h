@@ -267,7 +267,8 @@ int kmd_iterative_merge_sort(int dtype, int64_t n, const void *input,
  * memory, may be NULL): *n_rescored = samples re-scored in FP32 summed over
  * iterations; *fused_kernel_ms = summed HIP-event duration of the fused-step
  * kernel launches (in the mixed modes: BF16 kernel + FP32 re-score),
- * *fused_launches = their number; *fused_path = 0 generic kernel, 1 FP32
+ * *fused_launches = their number (both 0 for a fit that one block does in a
+ * single launch); *fused_path = 0 generic kernel, 1 FP32
  * MFMA, 2 BF16 + re-score, 3 BF16x3 + re-score, 4/5/6 the same three on the
  * tiled path, 7 FP8 + re-score on the tiled path (d <= 128 with centroids or sums beyond LDS: centroid tiles
  * streamed through LDS, update as a separate exact pass); a mixed mode falls
@@ -358,7 +359,8 @@ int kmd_engine_set_precision(kmd_engine_t engine, int precision);
  * of that shape use it.  Results never depend on the plan.  Writes the best
  * plan and up to `capacity` candidates (path: 1 LDS-resident, 2 tiled,
  * 0 generic; blocks_per_cu 0 = occupancy limit; shape; fused-step
- * ms/launch). */
+ * ms/launch).  Fits that one block does in a single launch have no plan: they
+ * run that way whatever the table says. */
 int kmd_autotune(int dtype, int itype, int precision, int64_t n_samples,
                  int64_t n_features, int64_t n_clusters, const void *X_t,
                  const void *sample_weight, const void *init_centroids_t,

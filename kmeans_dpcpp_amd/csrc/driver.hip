@@ -272,6 +272,7 @@ namespace {
 thread_local int t_blocks_cap = 0;
 thread_local int t_path = 0;
 thread_local int t_shape = 0;
+thread_local bool t_separate = false;   // no one-block loop (while timing plans)
 struct TuneChoice {
   int path = 0, blocks_per_cu = 0, shape = 0;
 };
@@ -300,11 +301,19 @@ int log2_bucket(int64_t n) {
   return b;
 }
 
-TuneChoice choose_tuning(int64_t n, int64_t d, int64_t k, int precision) {
-  std::lock_guard<std::mutex> lk(g_tune_mu);
-  if (g_override) return g_override_choice;
-  auto it = g_tune.find(std::make_tuple(d, k, precision, log2_bucket(n)));
-  return it == g_tune.end() ? TuneChoice{} : it->second;
+// A plan is for a fit of several launches: where one block does the whole fit
+// (f32, small_loop_serves, which not every n of a bucket is) the table is not
+// asked.
+TuneChoice choose_tuning(int64_t n, int64_t d, int64_t k, int precision, bool f32) {
+  TuneChoice c;
+  {
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    if (g_override) return g_override_choice;
+    auto it = g_tune.find(std::make_tuple(d, k, precision, log2_bucket(n)));
+    if (it == g_tune.end()) return c;
+    c = it->second;
+  }
+  return f32 && small_loop_serves(n, d, k) ? TuneChoice{} : c;
 }
 }  // namespace
 
@@ -426,14 +435,14 @@ struct FusedTimer {
   void end(hipStream_t s) {
     if (on) KMD_HIP_CHECK(hipEventRecord(stop[slot], s));
   }
-  // the launch timed in slot i, of `count` iterations, has finished
-  void collect(int i, int64_t count) {
+  // the launch timed in slot i has finished
+  void collect(int i) {
     if (!on) return;
     float ms = 0.f;
     KMD_HIP_CHECK(hipEventSynchronize(stop[i]));
     KMD_HIP_CHECK(hipEventElapsedTime(&ms, start[i], stop[i]));
     total_ms += ms;
-    launches += count;
+    ++launches;
   }
 };
 
@@ -669,7 +678,7 @@ void driver_lloyd(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
                   int64_t max_iter, int64_t *n_iters_out, double *inertia_out,
                   kmd_print_fn print_fn, void *print_user, hipStream_t s,
                   int precision, DriverStats *stats) {
-  TuneGuard g(choose_tuning(n, d, k, precision));
+  TuneGuard g(choose_tuning(n, d, k, precision, std::is_same<T, float>::value));
   driver_impl<T, I>(n, d, k, X, w, init, labels, res, tol, verbose, max_iter,
                     n_iters_out, inertia_out, print_fn, print_user, s, precision,
                     stats);
@@ -679,7 +688,8 @@ void driver_lloyd(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
 // fastest for its (d, k, precision, log2 n).  Candidates: LDS-resident or
 // tiled centroids (where each serves the shape) x persistent blocks per CU
 // {occupancy limit, 1, 2, 4}; each runs `iters` Lloyd iterations from the
-// given init on scratch copies, timed by the fused step's HIP events.  The
+// given init on scratch copies, timed by the fused step's HIP events (as fits
+// of separate launches, also where one block would do the whole fit).  The
 // choice never changes results (every plan computes the same labels and
 // exact sums).
 template <typename T, typename I>
@@ -688,6 +698,10 @@ std::vector<TuneResult> autotune_lloyd(int64_t n, int64_t d, int64_t k,
                                        int precision, int iters, hipStream_t s) {
   std::vector<TuneResult> out;
   if (n <= 0) return out;
+  struct Separate {
+    Separate() { t_separate = true; }
+    ~Separate() { t_separate = false; }
+  } separate;
   std::vector<int> paths;
   if (fast_fused_supported<T>(d, k)) paths.push_back(1);
   if (std::is_same<T, float>::value && tiled_supported(d, k)) paths.push_back(2);
@@ -805,13 +819,11 @@ static void driver_impl(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
     launch_half_l2_norm<T>(d, k, init, ws.hn.template as<T>(), s);
   };
   // small fits: everything in one launch (up to a relocation)
-  bool one_block = resident && !verbose && small_loop_serves(n, d, k);
+  bool one_block = resident && !verbose && !t_separate && small_loop_serves(n, d, k);
   if (!one_block) start();
   while (it < max_iter || one_block) {
     if constexpr (std::is_same<T, float>::value) {
       if (one_block) {
-        timer.slot = 0;
-        timer.begin(s);
         SmallLoop<I> sl{};
         sl.n = n;
         sl.d = (int)d;
@@ -830,7 +842,6 @@ static void driver_impl(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
         sl.host = host;
         sl.tol = tol_t;
         launch_small_loop<I>(sl, s);
-        timer.end(s);
       }
     }
     while (!one_block && queued < max_iter && queued <= it + ahead) {
@@ -850,8 +861,7 @@ static void driver_impl(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
       start();
       continue;
     }
-    if (one_block) {
-      timer.collect(0, done - it);
+    if (one_block) {   // no fused step to time
       it = done;
       if (stop == kLoopConverged) {
         KMD_HIP_CHECK(hipStreamSynchronize(s));
@@ -859,7 +869,7 @@ static void driver_impl(int64_t n, int64_t d, int64_t k, const T *X, const T *w,
         return;
       }
     }
-    for (; it < done; ++it) timer.collect((int)(it % (kAhead + 1)), 1);
+    for (; it < done; ++it) timer.collect((int)(it % (kAhead + 1)));
     T *cur = bufs[(it + 1) % 2];   // of iteration it - 1, the last finished
     if (verbose) {
       launch_inertia<T, I>(n, d, k, X, w, cur, labels,

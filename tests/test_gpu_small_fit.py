@@ -85,3 +85,29 @@ def test_small_fit_hands_over_what_fixed_point_cannot_hold(kd, torch_dev, monkey
     # FP32 sums, whose order is not fixed: 500 additions of one rounding each
     assert_array_equal(got[0], exp[0])
     np.testing.assert_allclose(got[1], exp[1], rtol=500 * 2.0 ** -24, atol=1e-3)
+
+
+def test_small_fit_has_no_step_to_time_and_no_plan(kd, torch_dev):
+    """One launch is the whole fit, so there is no fused step to report; plans
+    are timed with separate launches and kept for the sizes that have them."""
+    n, d, k = 1500, 10, 6
+    Xt, w = blobs(n, d, k, 11)
+    Xd, wd, init = to_dev(Xt), to_dev(w), to_dev(Xt[:, :k].copy())
+
+    def stats(Xd, wd):
+        lab = torch.empty(Xd.shape[1], dtype=torch.int32, device="cuda")
+        it, _, st = kd.kmeans_lloyd_driver_ex(Xd, wd, init.clone(), lab, torch.empty_like(init),
+                                              0.0, False, 5, "fp32", torch.cuda.current_stream())
+        return int(it), st
+
+    it, st = stats(Xd, wd)
+    assert it >= 1 and st["path"] == "fp32-mfma"
+    assert st["fused_launches"] == 0 and st["fused_kernel_ms"] == 0.0
+    tuned = kd.autotune(Xd, wd, init, "fp32", 2, torch.cuda.current_stream())
+    assert all(c[3] > 0 for c in tuned["candidates"])
+    it, st = stats(Xd, wd)
+    assert st["fused_launches"] == 0
+    # 9000 samples are beyond the rule: a launch an iteration
+    Xt, w = blobs(9000, d, k, 11)
+    it, st = stats(to_dev(Xt), to_dev(w))
+    assert st["fused_launches"] == it and st["fused_kernel_ms"] > 0
