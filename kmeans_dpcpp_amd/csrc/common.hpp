@@ -247,6 +247,10 @@ void launch_merge_sort(int64_t n, const T *in, T *out, hipStream_t s);
 template <typename T>
 void launch_threshold(int64_t n, const T *data, int64_t topk, T *threshold,
                       hipStream_t s);
+// The relocation's: NaN counts as the smallest value, not the largest.
+template <typename T>
+void launch_far_threshold(int64_t n, const T *data, int64_t topk, T *threshold,
+                          hipStream_t s);
 template <typename T, typename I>
 void launch_select_far(int64_t n_selected, int64_t n, const T *dist,
                        const T *threshold, I *selected, I *n_gt, I *n_eq,

@@ -35,6 +35,7 @@ struct Key<float> {
     if (u == 0x80000000u) u = 0u;                             // -0 -> +0
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
   }
+  static __device__ inline float value(float v) { return v; }
 };
 template <>
 struct Key<double> {
@@ -46,6 +47,7 @@ struct Key<double> {
     if (u == 0x8000000000000000ull) u = 0ull;
     return (u & 0x8000000000000000ull) ? ~u : (u | 0x8000000000000000ull);
   }
+  static __device__ inline double value(double v) { return v; }
 };
 
 template <typename T>
@@ -219,6 +221,17 @@ void launch_merge_sort(int64_t n, const T *in, T *out, hipStream_t s) {
 constexpr int kSelBlock = 256;
 constexpr int kSelChunk = 16 * kSelBlock;   // elements per block in the scans
 
+// The relocation's order: NaN before every number (no sample with a NaN distance
+// is far).  A NaN at the place asked for: -inf, which every other value reaches.
+template <typename T>
+struct NanFirstKey : Key<T> {
+  using U = typename Key<T>::U;
+  __host__ __device__ static inline U of(T v) { return v != v ? U(0) : Key<T>::of(v); }
+  static __device__ inline T value(T v) {
+    return v != v ? -std::numeric_limits<T>::infinity() : v;
+  }
+};
+
 template <typename T>
 struct SelState {
   typename Key<T>::U prefix, mask;
@@ -236,7 +249,7 @@ __global__ void __launch_bounds__(kSelBlock) sel_init_krn(SelState<T> *st, int64
   }
 }
 
-template <typename T>
+template <typename T, typename K>
 __global__ void __launch_bounds__(kSelBlock)
     sel_hist_krn(int64_t n, const T *__restrict__ data, SelState<T> *st, int shift) {
   using U = typename Key<T>::U;
@@ -250,9 +263,9 @@ __global__ void __launch_bounds__(kSelBlock)
   unsigned cur = 0u, run = 0u;
   for (int64_t i = blockIdx.x * (int64_t)kSelBlock + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * kSelBlock) {
-    const U k = Key<T>::of(data[i]);
-    if ((k & mask) == prefix) {
-      const unsigned dg = (unsigned)(k >> shift) & 255u;
+    const U key = K::of(data[i]);
+    if ((key & mask) == prefix) {
+      const unsigned dg = (unsigned)(key >> shift) & 255u;
       if (dg == cur) {
         ++run;
       } else {
@@ -289,7 +302,7 @@ __global__ void __launch_bounds__(kSelBlock) sel_pick_krn(SelState<T> *st, int s
 }
 
 // per chunk: elements whose key is the selected key
-template <typename T>
+template <typename T, typename K>
 __global__ void __launch_bounds__(kSelBlock)
     sel_count_krn(int64_t n, const T *__restrict__ data, const SelState<T> *st,
                   unsigned *counts) {
@@ -297,12 +310,12 @@ __global__ void __launch_bounds__(kSelBlock)
   __shared__ unsigned c;
   if (threadIdx.x == 0) c = 0u;
   __syncthreads();
-  const U K = st->prefix;
+  const U want = st->prefix;
   const int64_t base = (int64_t)blockIdx.x * kSelChunk;
   unsigned mine = 0u;
   for (int j = threadIdx.x; j < kSelChunk; j += kSelBlock) {
     const int64_t i = base + j;
-    mine += (i < n && Key<T>::of(data[i]) == K) ? 1u : 0u;
+    mine += (i < n && K::of(data[i]) == want) ? 1u : 0u;
   }
   if (mine) atomicAdd(&c, mine);
   __syncthreads();
@@ -310,7 +323,7 @@ __global__ void __launch_bounds__(kSelBlock)
 }
 
 // one block: the chunk holding the rank-th match, then the match itself
-template <typename T>
+template <typename T, typename K>
 __global__ void __launch_bounds__(kSelBlock)
     sel_finish_krn(int64_t n, int64_t n_chunks, const T *__restrict__ data,
                    const SelState<T> *st, const unsigned *counts, T *out) {
@@ -347,14 +360,14 @@ __global__ void __launch_bounds__(kSelBlock)
     s_chunk = b;
   }
   __syncthreads();
-  const U K = st->prefix;
+  const U want = st->prefix;
   const int64_t base = s_chunk * kSelChunk;
   const int lane = threadIdx.x & (kWave - 1);
   if (threadIdx.x < kWave) {          // one wave walks the chunk in order
     int64_t r = s_r;
     for (int j0 = 0; j0 < kSelChunk; j0 += kWave) {
       const int64_t i = base + j0 + lane;
-      const bool m = i < n && Key<T>::of(data[i]) == K;
+      const bool m = i < n && K::of(data[i]) == want;
       const unsigned long long bal = __ballot(m);
       const int cnt = __popcll(bal);
       if (r < cnt) {
@@ -362,7 +375,7 @@ __global__ void __launch_bounds__(kSelBlock)
         unsigned long long b = bal;
         for (int q = 0; q < r; ++q) b &= b - 1ull;
         const int pos = __ffsll((long long)b) - 1;
-        if (lane == pos) out[0] = data[i];
+        if (lane == pos) out[0] = K::value(data[i]);
         break;
       }
       r -= cnt;
@@ -370,7 +383,7 @@ __global__ void __launch_bounds__(kSelBlock)
   }
 }
 
-template <typename T>
+template <typename T, typename K>
 void launch_order_statistic(int64_t n, const T *data, int64_t p, T *out,
                             hipStream_t s) {
   using U = typename Key<T>::U;
@@ -379,11 +392,11 @@ void launch_order_statistic(int64_t n, const T *data, int64_t p, T *out,
   hipLaunchKernelGGL(sel_init_krn<T>, dim3(1), dim3(kSelBlock), 0, s,
                      st.as<SelState<T>>(), p);
   KMD_LAUNCH_CHECK();
-  const int64_t want = ceil_div<int64_t>(n, kSelBlock * 16);
+  const int64_t blocks = ceil_div<int64_t>(n, kSelBlock * 16);
   const unsigned grid = (unsigned)std::min<int64_t>(
-      std::max<int64_t>(want, 1), 8 * (int64_t)device_cu_count());
+      std::max<int64_t>(blocks, 1), 8 * (int64_t)device_cu_count());
   for (int shift = kBits - 8; shift >= 0; shift -= 8) {
-    hipLaunchKernelGGL(sel_hist_krn<T>, dim3(grid), dim3(kSelBlock), 0, s, n,
+    hipLaunchKernelGGL((sel_hist_krn<T, K>), dim3(grid), dim3(kSelBlock), 0, s, n,
                        data, st.as<SelState<T>>(), shift);
     KMD_LAUNCH_CHECK();
     hipLaunchKernelGGL(sel_pick_krn<T>, dim3(1), dim3(kSelBlock), 0, s,
@@ -393,11 +406,11 @@ void launch_order_statistic(int64_t n, const T *data, int64_t p, T *out,
   const int64_t n_chunks = ceil_div<int64_t>(n, kSelChunk);
   require(n_chunks <= INT32_MAX, "too many elements");
   TempBuffer counts(sizeof(unsigned) * (size_t)n_chunks, s);
-  hipLaunchKernelGGL(sel_count_krn<T>, dim3((unsigned)n_chunks), dim3(kSelBlock),
+  hipLaunchKernelGGL((sel_count_krn<T, K>), dim3((unsigned)n_chunks), dim3(kSelBlock),
                      0, s, n, data, st.as<const SelState<T>>(),
                      counts.as<unsigned>());
   KMD_LAUNCH_CHECK();
-  hipLaunchKernelGGL(sel_finish_krn<T>, dim3(1), dim3(kSelBlock), 0, s, n,
+  hipLaunchKernelGGL((sel_finish_krn<T, K>), dim3(1), dim3(kSelBlock), 0, s, n,
                      n_chunks, data, st.as<const SelState<T>>(),
                      counts.as<const unsigned>(), out);
   KMD_LAUNCH_CHECK();
@@ -414,13 +427,29 @@ void launch_threshold(int64_t n, const T *data, int64_t topk, T *threshold,
     launch_max<T>(n, data, threshold, s);
     return;
   }
-  launch_order_statistic<T>(n, data, n - topk, threshold, s);
+  launch_order_statistic<T, Key<T>>(n, data, n - topk, threshold, s);
+}
+
+// The topk-th largest of the values that are not NaN; -inf where there are
+// fewer.
+template <typename T>
+void launch_far_threshold(int64_t n, const T *data, int64_t topk, T *threshold,
+                          hipStream_t s) {
+  if (topk == 1) {
+    launch_max<T>(n, data, threshold, s);   // passes over NaN
+    return;
+  }
+  launch_order_statistic<T, NanFirstKey<T>>(n, data, n - topk, threshold, s);
 }
 
 template void launch_merge_sort<float>(int64_t, const float *, float *,
                                        hipStream_t);
 template void launch_merge_sort<double>(int64_t, const double *, double *,
                                         hipStream_t);
+template void launch_far_threshold<float>(int64_t, const float *, int64_t, float *,
+                                          hipStream_t);
+template void launch_far_threshold<double>(int64_t, const double *, int64_t, double *,
+                                           hipStream_t);
 template void launch_threshold<float>(int64_t, const float *, int64_t, float *,
                                       hipStream_t);
 template void launch_threshold<double>(int64_t, const double *, int64_t,

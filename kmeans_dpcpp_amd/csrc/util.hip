@@ -797,6 +797,7 @@ __global__ void __launch_bounds__(1024)
     if (pos < m) order[pos] = (int64_t)selected[n - 1 - r];
   }
   // NaN distances can leave fewer samples than m: no sample for the rest
+  // (as far_order_krn)
   for (int64_t pos = g + (e > 0 ? e : 0) + threadIdx.x; pos < m; pos += blockDim.x)
     order[pos] = -1;
 }
@@ -812,7 +813,8 @@ __global__ void __launch_bounds__(1024)
 // us).  With m near the number of threads that bound is no bound any more (m =
 // 1000 of 50,000: 775 -> 963 us), hence kFarM.  Many equal distances can make the
 // list overflow all the same: then the m-th largest is found over all samples,
-// and the equal ones are taken in index order.  A NaN distance is never far.
+// and the equal ones are taken in index order.  A NaN distance (key 0) is never
+// far: with fewer than m others, the places after them hold no sample (-1).
 constexpr int64_t kFarN = 262144;
 constexpr int kFarThreads = 1024;
 constexpr int64_t kFarM = kFarThreads / 2;
@@ -890,7 +892,7 @@ __global__ void __launch_bounds__(kFarThreads)
     for (int u = 0; u < kU; ++u) {
       const int i = i0 + u * kFarThreads;
       const U q = FarKey<T>::of(v[u]);
-      if (i < n && q >= low) {
+      if (i < n && q != 0 && q >= low) {
         const int at = atomicAdd(&count, 1);
         if (at < kFarList) {
           lkey[at] = q;
@@ -902,6 +904,7 @@ __global__ void __launch_bounds__(kFarThreads)
   __syncthreads();
   int listed = count;
   if (listed > kFarList) {
+    // (kFarList > kFarM: at least m samples are no NaN, so thr below is not 0)
     // the exact m-th largest key, then the samples above it and the first
     // ones equal to it
     U thr = 0;
@@ -952,7 +955,7 @@ __global__ void __launch_bounds__(kFarThreads)
     }
     if (rank < m) order[rank] = si;
   }
-  for (int r = listed + tid; r < m; r += kFarThreads) order[r] = -1;   // m > n
+  for (int r = listed + tid; r < m; r += kFarThreads) order[r] = -1;
 }
 
 template <typename T, typename I>
@@ -1210,7 +1213,7 @@ void launch_relocate(int64_t n, int64_t d, int64_t k, int64_t n_empty,
     TempBuffer sel(sizeof(I) * (n + 2), s);
     I *n_gt = sel.as<I>() + n;
     I *n_eq = n_gt + 1;
-    launch_threshold<T>(n, sq_dist, m, thr.as<T>(), s);
+    launch_far_threshold<T>(n, sq_dist, m, thr.as<T>(), s);
     hipLaunchKernelGGL((init_counters_krn<T, I>), dim3(1), dim3(1), 0, s, n_gt, n_eq);
     KMD_LAUNCH_CHECK();
     launch_select_far<T, I>(m, n, sq_dist, thr.as<const T>(), sel.as<I>(), n_gt, n_eq, s);
