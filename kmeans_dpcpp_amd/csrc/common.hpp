@@ -123,6 +123,14 @@ class TempBuffer {
 
 // ---- device helpers -----------------------------------------------------
 
+// Between LDS stores of a wave's lanes and loads of other lanes of it (and the
+// other way round): the hardware keeps a wave's LDS operations in order, this
+// keeps the compiler from moving or joining them across.
+__device__ inline void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Hardware float atomics (global_atomic_add_f32/f64, ds_add_f32/f64). The
 // library is built with -munsafe-fp-atomics; every buffer it adds into is
 // coarse-grained device memory.

@@ -1036,6 +1036,7 @@ __global__ void __launch_bounds__(1024) small_loop_krn(SmallLoop<I> a) {
         Sn[c * (DB + 1) + lane] = Ca[c * DB + lane] - q;
         Ca[c * DB + lane] = q;
       }
+      wave_lds_order();
       if (lane == 0) {
         float acc = 0.f, h = 0.f;
 #pragma unroll 8

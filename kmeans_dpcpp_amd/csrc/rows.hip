@@ -31,7 +31,7 @@ __global__ void __launch_bounds__(kRNT)
 // wave and so come through the scalar cache as the subtraction's scalar
 // operand.  Rows enter and results leave through a per-wave LDS tile (128
 // bytes of 64 rows), so both sides of global memory move whole lines; no
-// barrier, a wave's LDS operations are in order.
+// block barrier, the lanes of a wave exchange with wave_lds_order.
 //
 // Bound by the vector unit: two operations per (row, centre, feature) and no
 // second unit to share them with (the expanded form on the matrix core would
@@ -62,8 +62,10 @@ __global__ void __launch_bounds__(kRNT)
 #pragma unroll 8
     for (int r = ty; r < kWave; r += kTY)
       tile[r][tx] = (r < rows && f0 + tx < d) ? X[(s0 + r) * d + f0 + tx] : T(0);
+    wave_lds_order();
 #pragma unroll
     for (int f = 0; f < kW; ++f) x[f0 + f] = tile[lane][f];
+    wave_lds_order();
   }
   for (int c0 = 0; c0 < k; c0 += kRF) {
     const int m = min(kRF, k - c0);
@@ -83,9 +85,11 @@ __global__ void __launch_bounds__(kRNT)
 #pragma unroll
       for (int j = 0; j < kRC; ++j) tile[lane][c + j] = sqrt(acc[j]);
     }
+    wave_lds_order();
 #pragma unroll 8
     for (int r = ty; r < kWave; r += kTY)
       if (r < rows && tx < m) D[(s0 + r) * k + c0 + tx] = tile[r][tx];
+    wave_lds_order();
   }
 }
 
