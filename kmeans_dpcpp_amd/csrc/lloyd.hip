@@ -218,8 +218,7 @@ void launch_fused_step_copies(int64_t n, int64_t d, int64_t k,
     // tiles streamed through LDS, then the update from those labels
     if (tiled_supported(d, k)) {
       launch_tiled_assign<I>(n, d, k, X, C, hn, labels, s, nullptr, scratch);
-      // the exact window sums where one row of them fits LDS
-      if (label_sums_supported(k))
+      if (label_sums_first(n, k))
         launch_label_sums<I>(n, d, k, n_copies, X, w, C, labels, copies, sizes_copies, s);
       else
         launch_label_update<I>(n, d, k, n_copies, X, w, labels, copies, sizes_copies, s);

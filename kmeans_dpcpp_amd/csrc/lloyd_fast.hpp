@@ -309,6 +309,8 @@ void launch_wide_assign(int64_t n, int64_t d, int64_t k, const float *X_t,
 // sums per block (windows set from the centroids C), the blocks' totals added
 // into the copies with FP32 atomics.
 bool label_sums_supported(int64_t k);
+// ... and is faster than launch_label_update
+bool label_sums_first(int64_t n, int64_t k);
 template <typename I>
 void launch_label_sums(int64_t n, int64_t d, int64_t k, int64_t n_copies,
                        const float *X_t, const float *w, const float *C,

@@ -350,6 +350,16 @@ bool label_sums_supported(int64_t k) {
   return k >= 1 && (size_t)k * sizeof(u64) + sizeof(int) <= kSumLds;
 }
 
+// label_update_krn's sums are 4 bytes, so it holds twice the rows; the 8 bytes a
+// sum here have to be cleared and flushed for the samples to pay for.  Steps of d
+// = 16 to 128, this against that one: k <= 1024 0.81 - 1.02 x at any n; n >= 8 k up
+// to the k whose rows stand two at a time in LDS 0.83 - 1.02 x; n = 2 k there 1.00 -
+// 1.04 x; one row at a time (n = 1M, d = 128, k = 10,000) 1497 us against 829.
+bool label_sums_first(int64_t n, int64_t k) {
+  return label_sums_supported(k) &&
+         2 * ((size_t)k * sizeof(u64) + sizeof(int)) <= kSumLds && (k <= 1024 || n >= 8 * k);
+}
+
 template <typename I>
 void launch_label_sums(int64_t n, int64_t d, int64_t k, int64_t n_copies,
                        const float *X_t, const float *w, const float *C,
@@ -359,10 +369,10 @@ void launch_label_sums(int64_t n, int64_t d, int64_t k, int64_t n_copies,
   require(label_sums_supported(k), "label sums: too many clusters for one LDS row");
   const int rows = sum_rows(d, k);
   const int64_t groups = ceil_div<int64_t>(d + 1, rows);
-  // one block per CU over all groups, at least 2048 samples each
+  // at most one block per CU over all groups (four blocks more are a second round
+  // of all), at least 2048 samples each
   const int64_t b = std::max<int64_t>(
-      1, std::min<int64_t>(ceil_div<int64_t>(device_cu_count(), groups),
-                           ceil_div<int64_t>(n, 2048)));
+      1, std::min<int64_t>(device_cu_count() / groups, ceil_div<int64_t>(n, 2048)));
   const int64_t chunk = ceil_div<int64_t>(n, b);
   allow_full_lds(reinterpret_cast<const void *>(&label_sums_krn<I>));
   hipLaunchKernelGGL(label_sums_krn<I>, dim3((unsigned)b, (unsigned)groups), dim3(kSNT),

@@ -7,7 +7,7 @@ from numpy.testing import assert_array_equal
 
 from oracle import c_oracle as co
 from oracle import lloyd_oracle as lo
-from tests.conftest import fp64_update, to_dev, to_np
+from tests.conftest import check_label_mismatches, fp64_update, to_dev, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -96,3 +96,33 @@ def test_fused_step_follows_its_labels(kd, torch_dev):
     sums = to_np(cp).astype(np.float64).sum(axis=0) - 0.5 * copies
     exp = np.stack([np.bincount(lab, Xt[f].astype(np.float64), minlength=k) for f in range(d)])
     assert np.abs(sums - exp).max() <= 1e-5 * np.abs(exp).max()
+
+
+# both sides of the rule between the two updates from labels: k = 1024, n = 8 k,
+# and the largest k of which two rows of sums fit LDS (9727)
+@pytest.mark.parametrize("n,d,k", [(2050, 96, 1024), (2050, 96, 1025), (8200, 96, 1025),
+                                   (77_815, 5, 9727), (77_816, 5, 9727), (77_824, 5, 9728)])
+def test_both_updates_of_the_fused_step(kd, torch_dev, n, d, k):
+    rng = np.random.default_rng(n + k)
+    Xt = rng.standard_normal((d, n)).astype(np.float32)
+    init = np.ascontiguousarray(Xt[:, :k])
+    w = rng.uniform(0.5, 2.0, n).astype(np.float32)
+    hn = co.half_norm(init)
+    ids = torch.empty(n, dtype=torch.int32, device=torch_dev)
+    cp = torch.zeros((2, d, k), device=torch_dev)
+    scp = torch.zeros((2, k), device=torch_dev)
+    kd.fused_lloyd_single_step(to_dev(Xt), to_dev(w), to_dev(init), to_dev(hn), ids, cp, scp,
+                               8, 256, q())[0].wait()
+    lab = to_np(ids)
+    # (the tiled kernel's chain starts from the half norm)
+    check_label_mismatches(Xt, init, lab, co.assign(Xt, init, hn), 4)
+    cnt = np.bincount(lab, w, minlength=k)
+    # m values a cluster: each product and each addition rounds once
+    m = np.bincount(lab, minlength=k)
+    got = to_np(scp).astype(np.float64).sum(axis=0)
+    assert np.all(np.abs(got - cnt) <= (m + 4) * 2.0 ** -24 * cnt)
+    sums = to_np(cp).astype(np.float64).sum(axis=0)
+    for f in range(d):
+        v = Xt[f].astype(np.float64) * w
+        exp, mag = (np.bincount(lab, a, minlength=k) for a in (v, np.abs(v)))
+        assert np.all(np.abs(sums[f] - exp) <= (m + 4) * 2.0 ** -24 * mag)
