@@ -16,12 +16,15 @@
 //    kernel keeps the loop's state on the device (finished iterations, and
 //    whether the loop converged or found empty clusters) and publishes it in
 //    pinned host memory; the kernels of an iteration return at once when the
-//    loop has stopped, so a few iterations are enqueued ahead and cost next
-//    to nothing when they were not needed.  The host reads the state from
+//    loop has stopped, so the next iteration is enqueued ahead and costs next
+//    to nothing when it was not needed.  The host reads the state from
 //    memory between launches; it relocates empty clusters and enqueues the
 //    iterations after that again;
 //  * private copies are one per block of the persistent fused kernel and are
-//    written with plain stores, so the sums are deterministic;
+//    written with plain stores, so the sums are deterministic (not on the two
+//    paths that add the blocks' totals into eight copies with atomics: float32
+//    beyond the tiled kernels, d > 128 or k > 32768, and sums that do not fit
+//    LDS on the generic one; there the last bits depend on the blocks' order);
 //  * the relocation path reuses the labels of the fused step instead of
 //    recomputing them from the same centroids and half-norms
 //    (src/kmeans_lloyd_driver.hpp:226-250);

@@ -73,7 +73,8 @@ __device__ inline void wait_dma_and_sync() {
 // FP32 k-steps (2 features each), bucketed.  Every k-step of padding is a
 // product per tile and column block that nobody needs: with buckets of 16, 32
 // and 64 k-steps alone, d = 96 did a third more products than it has (n =
-// 500,000, k = 512: 0.449 ms per pass, 0.348 with 48).
+// 500,000, k = 512: 0.531 ms per pass, 0.407 with 48, where the products alone
+// need 0.321 at the rate of a large one).
 inline int ks_of(int64_t d) {
   const int64_t ks = (d + 1) / 2;
   return ks <= 16 ? 16 : (int)ceil_div<int64_t>(ks, 8) * 8;
@@ -381,7 +382,7 @@ __global__ void __launch_bounds__(256) cand_count_krn(CandArgs a) {
 }
 
 // One wave: the at most 32 tiles' counts by shuffles, the segments' by lane (one
-// thread's chain of dependent loads took 15 us; here 4.3).
+// thread's chain of dependent loads took 18 us; here 4.3).
 __global__ void __launch_bounds__(kWave) cand_scan_krn(CandArgs a) {
   if (skipped(a)) return;
   const int lane = threadIdx.x;
@@ -1390,8 +1391,8 @@ __global__ void __launch_bounds__(256)
 // to every cluster's counter once, and device atomics of one address serialise, so
 // a block takes at least 16K samples; its time is then the round trips of its
 // labels, so 1024 threads have 16 of them in flight each (256 threads with one at
-// a time, n = 500K, k = 512: 15.3 us counting and 24.2 scattering, 4.6 and
-// 12.0 here).
+// a time, n = 500K, k = 512: 17 us counting and 28 scattering, 4.6 and 14
+// here).
 constexpr int kLabelThreads = 1024;
 constexpr int kLabelRun = 16;
 

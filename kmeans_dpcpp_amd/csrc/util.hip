@@ -229,10 +229,10 @@ __global__ void __launch_bounds__(kBlock)
 // Column tiles are staged in LDS by the whole block (all loads in flight)
 // before the serial chains over the features; a thread per column reading
 // global memory, and a launch for the list, took 38 + 5 us at d = 300, k =
-// 100 and 5.4 + 2.7 us at d = 14, k = 127, where this takes 16 and 4.3 us.
+// 100 and 5.4 + 2.7 us at d = 14, k = 127, where this takes 16 and 4.7 us.
 // Shapes that fit one tile (d = 32, k = 256 does) run on one block and keep
 // the shifts in registers (65 us for one block over six tiles, d = 96, k =
-// 512: 15 us with the others); the others run a block per tile, at most
+// 512: 17 us with the others); the others run a block per tile, at most
 // kTailBlocks (the ticket's atomics serialise), and the last one to finish
 // adds up the shifts.
 constexpr int kTailThreads = 1024;
