@@ -243,73 +243,145 @@ WideFn pick_wide(int nt, bool two) {
 // pass over X for scales, any input (values outside a window go to the copy
 // one by one).  FP32 sums in LDS were measured first: ds_add_f32 took 0.42 ms
 // at n = 200,003, d = 300, k = 100; the integer form takes
-// 0.071 ms (the read of X alone: 0.051 ms).
+// 0.072 ms (the read of X alone: 0.051 ms).
 constexpr int kSNT = 1024;
 constexpr int kSWaves = kSNT / kWave;
 constexpr size_t kSumLds = 152 * 1024;   // one block per CU: the fewest totals
+constexpr int kSumStep = 8;              // row loads in flight per thread
 
-template <typename I>
+// exponent of a finite value, 0 of an infinity or NaN
+__device__ inline int finite_binade(float v) {
+  const int e = (int)((__float_as_uint(v) >> 23) & 0xffu);
+  return e != 0xff ? e : 0;
+}
+
+template <bool COPIES, typename I>
 __global__ void __launch_bounds__(kSNT)
-    label_sums_krn(int64_t n, int d, int k, int rows, int64_t chunk, int W,
+    label_sums_krn(int64_t n, int d, int k, int rows, int rshift, int64_t chunk, int W,
                    const float *__restrict__ X, const float *__restrict__ w,
                    const float *__restrict__ C, const I *__restrict__ labels,
                    float *copies, float *sizes_copies, int n_copies, const int *skip) {
   if (skip != nullptr && *skip != 0) return;
-  extern __shared__ u64 acc[];   // [rows][k], then the rows' windows
-  int *low = reinterpret_cast<int *>(acc + (int64_t)rows * k);
+  // [rows][k][1 << rshift] sums, then the rows' windows (whole steps)
+  extern __shared__ u64 acc[];
+  int *low = reinterpret_cast<int *>(acc + (((int64_t)rows * k) << rshift));
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int f0 = blockIdx.y * rows;
   const int nf = min(rows, d + 1 - f0);   // rows of this group
   const int nx = min(nf, d - f0);         // those of them that are features
-  for (int i = threadIdx.x; i < nf * k; i += kSNT) acc[i] = 0ull;
-  // the window of feature f ends kWinMargin binades above the largest finite
-  // centroid coordinate of f, that of the weights at 2^kWinTopW
-  for (int f = wave; f < nx; f += kSWaves) {
-    int e = 0;
-    for (int c = lane; c < k; c += kWave) {
-      const int ec = (int)((__float_as_uint(C[(int64_t)(f0 + f) * k + c]) >> 23) & 0xffu);
-      e = ec != 0xff ? max(e, ec) : e;
+  const int64_t beg = blockIdx.x * chunk, s1 = min(n, beg + chunk);
+  // The window of feature f ends kWinMargin binades above the largest finite
+  // of its centroid coordinates and of the block's first 64 products w x (1 where
+  // all of them are 0): of centred data with few clusters the coordinates alone can
+  // be far smaller, and then every value went to the copy by itself (n = 200,000,
+  // d = 129, k = 2: 2.2 ms instead of 0.04).  That of the weights likewise.
+  const int64_t sl = beg + lane;
+  const float w0 = sl < s1 ? w[sl] : 0.f;
+  constexpr int kRound = 10;   // rows a wave reads side by side (one after another: 2 us each)
+  float x[kRound], c[kRound];
+  auto load = [&](int fb) {
+#pragma unroll
+    for (int u = 0; u < kRound; ++u) {
+      const int f = fb + u * kSWaves;
+      x[u] = f < nx && sl < s1 ? X[(int64_t)(f0 + f) * n + sl] : 1.f;
+      c[u] = f < nx && lane < k ? C[(int64_t)(f0 + f) * k + lane] : 0.f;
     }
-    for (int o = kWave / 2; o > 0; o >>= 1) e = max(e, __shfl_xor(e, o, kWave));
-    if (lane == 0) low[f] = window_low(e, kWinMargin, W);
+  };
+  load(wave);
+  for (int i = threadIdx.x; i < (nf * k) << rshift; i += kSNT) acc[i] = 0ull;
+  for (int fb = wave; fb < nf + kSumStep; fb += kRound * kSWaves) {
+    if (fb != wave) load(fb);
+#pragma unroll
+    for (int u = 0; u < kRound; ++u) {
+      const int f = fb + u * kSWaves;
+      int e = max(finite_binade(x[u] * w0), finite_binade(c[u]));
+      if (f < nx)
+        for (int cc = kWave + lane; cc < k; cc += kWave)
+          e = max(e, finite_binade(C[(int64_t)(f0 + f) * k + cc]));
+      for (int o = kWave / 2; o > 0; o >>= 1) e = max(e, __shfl_xor(e, o, kWave));
+      if (lane == 0 && f < nf + kSumStep && f < ((rows + kSumStep - 1) & -kSumStep))
+        low[f] = window_low(e != 0 ? e : 127, kWinMargin, W);
+    }
   }
-  if (nx < nf && threadIdx.x == 0) low[nx] = window_low(127, kWinTopW, W);
   __syncthreads();
   const int64_t copy = blockIdx.x % (unsigned)n_copies;
   float *out = copies + (copy * d + f0) * k;
   float *out_w = sizes_copies + copy * k;
-  const int64_t s1 = min(n, (int64_t)(blockIdx.x + 1) * chunk);
-  constexpr int kU = 8;   // row loads in flight per thread
-  for (int64_t s = blockIdx.x * chunk + threadIdx.x; s < s1; s += kSNT) {
+  const int own = lane & ((1 << rshift) - 1);
+  for (int64_t s = beg + threadIdx.x; s < s1; s += kSNT) {
     const int l = (int)labels[s];
     const float ws = w[s];
     const float *col = X + (int64_t)f0 * n + s;
+    auto add = [&](int f, float v) {
+      const int off = f * k + l;
+      window_add(acc + (COPIES ? (off << rshift) + own : off), out + off, 0, v, low[f], W);
+    };
     int f = 0;
-    for (; f + kU <= nx; f += kU) {
-      float x[kU];
+    for (; f + kSumStep <= nx; f += kSumStep) {
+      float x[kSumStep];
 #pragma unroll
-      for (int j = 0; j < kU; ++j) x[j] = col[(int64_t)(f + j) * n];
+      for (int j = 0; j < kSumStep; ++j) x[j] = col[(int64_t)(f + j) * n];
 #pragma unroll
-      for (int j = 0; j < kU; ++j)
-        window_add(acc, out, (int64_t)(f + j) * k + l, x[j] * ws, low[f + j], W);
+      for (int j = 0; j < kSumStep; ++j) add(f + j, x[j] * ws);
     }
-    for (; f < nx; ++f)
-      window_add(acc, out, (int64_t)f * k + l, col[(int64_t)f * n] * ws, low[f], W);
-    if (nx < nf) window_add(acc + (int64_t)nx * k, out_w, l, ws, low[nx], W);
+    if (f < nx) {   // (a product of 0 is added nowhere)
+      float x[kSumStep];
+#pragma unroll
+      for (int j = 0; j < kSumStep; ++j) x[j] = f + j < nx ? col[(int64_t)(f + j) * n] : 0.f;
+#pragma unroll
+      for (int j = 0; j < kSumStep; ++j) add(f + j, f + j < nx ? x[j] * ws : 0.f);
+    }
+    if (nx < nf) {
+      const int off = nx * k + l;
+      window_add(acc + (COPIES ? (off << rshift) + own : off), out_w + l, 0, ws, low[nx], W);
+    }
   }
   __syncthreads();
   for (int i = threadIdx.x; i < nf * k; i += kSNT) {
     const int f = i / k;
-    const float v = (float)ldexp((double)(long long)acc[i], low[f] - 150);
+    u64 t = 0;
+    for (int r = 0; r < 1 << rshift; ++r) t += acc[(i << rshift) + ((r + lane) & ((1 << rshift) - 1))];
+    const float v = (float)ldexp((double)(long long)t, low[f] - 150);
     if (v != 0.f) atomic_add(f < nx ? out + i : out_w + (i - nx * k), v);
   }
 }
 
-// Rows of one group: as many as fit kSumLds, the groups of about equal size.
-inline int sum_rows(int64_t d, int64_t k) {
-  const int64_t most = std::max<int64_t>(
-      1, (int64_t)kSumLds / (int64_t)(sizeof(u64) * k + sizeof(int)));
-  return (int)ceil_div<int64_t>(d + 1, ceil_div<int64_t>(d + 1, most));
+struct SumPlan {
+  int rows, rshift;
+  int64_t groups, blocks;   // of rows; of samples
+};
+
+inline size_t sum_lds(int64_t rows, int64_t k, int rshift) {
+  return (sizeof(u64) * (size_t)k << rshift) * rows +
+         sizeof(int) * (ceil_div<int64_t>(rows, kSumStep) * kSumStep);
+}
+
+// Groups of rows: as few as LDS allows, of about equal size, for labels and weights
+// are read once per group; with few samples more of them, so that the blocks are
+// near one per CU (never more: four blocks past that are a second round of all),
+// a block taking at least 2048 samples.
+//
+// Copies of a sum: lanes of one label add to one address, one after the other, so
+// the lanes of a wave have 64 sums of a row or more between them.
+//
+// A fused step with one sum each and groups as few as LDS allows, whatever n, against
+// this: n = 3000, d = 800, k = 8: 907 -> 85 us; n = 40,000, d = 128, k = 2: 257 -> 105;
+// n = 10,000, d = 400, k = 20: 338 -> 84.
+SumPlan plan_sums(int64_t n, int64_t d, int64_t k) {
+  SumPlan p{};
+  while ((k << p.rshift) < kWave && p.rshift < 5) ++p.rshift;
+  int64_t most = std::max<int64_t>(1, (int64_t)kSumLds / (int64_t)(sizeof(u64) * k << p.rshift));
+  while (most > 1 && sum_lds(most, k, p.rshift) > kSumLds) --most;
+  const int64_t cus = device_cu_count();
+  p.groups = ceil_div<int64_t>(d + 1, most);
+  p.blocks = std::max<int64_t>(1, std::min<int64_t>(cus / p.groups, ceil_div<int64_t>(n, 2048)));
+  p.rows = (int)ceil_div<int64_t>(d + 1, p.groups);
+  if (cus / p.blocks > p.groups) {
+    const int64_t r = ceil_div<int64_t>(d + 1, cus / p.blocks);
+    p.rows = (int)std::min<int64_t>(p.rows, ceil_div<int64_t>(r, kSumStep) * kSumStep);
+    p.groups = ceil_div<int64_t>(d + 1, p.rows);
+  }
+  return p;
 }
 
 }  // namespace
@@ -347,7 +419,7 @@ void launch_wide_assign(int64_t n, int64_t d, int64_t k, const float *X_t,
 
 // one row of sums fits kSumLds
 bool label_sums_supported(int64_t k) {
-  return k >= 1 && (size_t)k * sizeof(u64) + sizeof(int) <= kSumLds;
+  return k >= 1 && (size_t)k * sizeof(u64) + sizeof(int) <= kSumLds;   // (and a few windows)
 }
 
 // label_update_krn's sums are 4 bytes, so it holds twice the rows; the 8 bytes a
@@ -357,7 +429,7 @@ bool label_sums_supported(int64_t k) {
 // 1.04 x; one row at a time (n = 1M, d = 128, k = 10,000) 1497 us against 829.
 bool label_sums_first(int64_t n, int64_t k) {
   return label_sums_supported(k) &&
-         2 * ((size_t)k * sizeof(u64) + sizeof(int)) <= kSumLds && (k <= 1024 || n >= 8 * k);
+         sum_lds(2, k, 0) <= kSumLds && (k <= 1024 || n >= 8 * k);
 }
 
 template <typename I>
@@ -367,17 +439,13 @@ void launch_label_sums(int64_t n, int64_t d, int64_t k, int64_t n_copies,
                        hipStream_t s, const int *skip) {
   if (n <= 0) return;
   require(label_sums_supported(k), "label sums: too many clusters for one LDS row");
-  const int rows = sum_rows(d, k);
-  const int64_t groups = ceil_div<int64_t>(d + 1, rows);
-  // at most one block per CU over all groups (four blocks more are a second round
-  // of all), at least 2048 samples each
-  const int64_t b = std::max<int64_t>(
-      1, std::min<int64_t>(device_cu_count() / groups, ceil_div<int64_t>(n, 2048)));
-  const int64_t chunk = ceil_div<int64_t>(n, b);
-  allow_full_lds(reinterpret_cast<const void *>(&label_sums_krn<I>));
-  hipLaunchKernelGGL(label_sums_krn<I>, dim3((unsigned)b, (unsigned)groups), dim3(kSNT),
-                     (sizeof(u64) * k + sizeof(int)) * (size_t)rows, s, n, (int)d, (int)k,
-                     rows, chunk, window_width(chunk), X_t, w, C, labels, copies,
+  const SumPlan p = plan_sums(n, d, k);
+  const int64_t chunk = ceil_div<int64_t>(n, p.blocks);
+  auto fn = p.rshift > 0 ? &label_sums_krn<true, I> : &label_sums_krn<false, I>;
+  allow_full_lds(reinterpret_cast<const void *>(fn));
+  hipLaunchKernelGGL(fn, dim3((unsigned)p.blocks, (unsigned)p.groups),
+                     dim3(kSNT), sum_lds(p.rows, k, p.rshift), s, n, (int)d, (int)k, p.rows,
+                     p.rshift, chunk, window_width(chunk), X_t, w, C, labels, copies,
                      sizes_copies, (int)n_copies, skip);
   KMD_LAUNCH_CHECK();
 }

@@ -99,9 +99,9 @@ def test_fused_step_follows_its_labels(kd, torch_dev):
 
 
 # both sides of the rule between the two updates from labels: k = 1024, n = 8 k,
-# and the largest k of which two rows of sums fit LDS (9727)
+# and the largest k of which two rows of sums fit LDS (9726)
 @pytest.mark.parametrize("n,d,k", [(2050, 96, 1024), (2050, 96, 1025), (8200, 96, 1025),
-                                   (77_815, 5, 9727), (77_816, 5, 9727), (77_824, 5, 9728)])
+                                   (77_807, 5, 9726), (77_808, 5, 9726), (77_816, 5, 9727)])
 def test_both_updates_of_the_fused_step(kd, torch_dev, n, d, k):
     rng = np.random.default_rng(n + k)
     Xt = rng.standard_normal((d, n)).astype(np.float32)
@@ -126,3 +126,43 @@ def test_both_updates_of_the_fused_step(kd, torch_dev, n, d, k):
         v = Xt[f].astype(np.float64) * w
         exp, mag = (np.bincount(lab, a, minlength=k) for a in (v, np.abs(v)))
         assert np.all(np.abs(sums[f] - exp) <= (m + 4) * 2.0 ** -24 * mag)
+
+
+# few clusters (copies of the sums by lane), few samples (more groups of rows),
+# rows that are no whole step of eight, one sample
+@pytest.mark.parametrize("n,d,k", [(1, 131, 1), (65, 130, 2), (700, 513, 3), (3000, 800, 8),
+                                   (2049, 136, 31), (10_000, 129, 33), (4097, 305, 63),
+                                   (5000, 143, 64), (40_000, 128, 2), (2048, 97, 5)])
+@pytest.mark.parametrize("kind", ["plain", "spread", "zero start", "small weights"])
+def test_sums_of_few_clusters(kd, torch_dev, n, d, k, kind):
+    """The fused step's sums against FP64 ones of its labels, also where values lie
+    outside the window that the first samples of a block set (spread), where those
+    have no weight, and where the weights are far from 1."""
+    rng = np.random.default_rng(n + d + k)
+    Xt = rng.standard_normal((d, n)).astype(np.float32)
+    w = rng.uniform(0.5, 2.0, n).astype(np.float32)
+    if kind == "spread":
+        Xt *= (10.0 ** rng.uniform(-15, 9, n)).astype(np.float32)
+    elif kind == "zero start":
+        w[:64] = 0.0
+    elif kind == "small weights":
+        w *= np.float32(1e-9)
+    # coordinates far below the samples', as of centred data
+    init = (1e-3 * rng.standard_normal((d, k))).astype(np.float32)
+    hn = co.half_norm(init)
+    ids = torch.empty(n, dtype=torch.int32, device=torch_dev)
+    cp = torch.zeros((2, d, k), device=torch_dev)
+    scp = torch.zeros((2, k), device=torch_dev)
+    kd.fused_lloyd_single_step(to_dev(Xt), to_dev(w), to_dev(init), to_dev(hn), ids, cp, scp,
+                               8, 256, q())[0].wait()
+    lab = to_np(ids)
+    m = np.bincount(lab, minlength=k)
+    # m values a cluster, each rounded in its product, at most each in its addition
+    cnt = np.bincount(lab, w, minlength=k)
+    assert np.all(np.abs(to_np(scp).astype(np.float64).sum(axis=0) - cnt)
+                  <= (m + 4) * 2.0 ** -24 * cnt)
+    sums = to_np(cp).astype(np.float64).sum(axis=0)
+    for f in range(d):
+        v = Xt[f].astype(np.float64) * w
+        exp, mag = (np.bincount(lab, a, minlength=k) for a in (v, np.abs(v)))
+        assert np.all(np.abs(sums[f] - exp) <= (m + 4) * 2.0 ** -24 * mag + 1e-40)
