@@ -41,7 +41,7 @@ __global__ void __launch_bounds__(kRNT)
 // 0.106 + 0.186 + 0.129 ms.
 template <typename T, int DB>
 __global__ void __launch_bounds__(kRNT)
-    row_distances_krn(int64_t n, int d, int k, const T *__restrict__ X,
+    row_distances_krn(int64_t n, int d, int k, int span, const T *__restrict__ X,
                       const T *__restrict__ C, T *__restrict__ D) {
   constexpr int kRF = 128 / sizeof(T);   // features (and centres) per LDS tile
   __shared__ T tiles[kRWaves][kWave][kRF + 1];
@@ -67,8 +67,10 @@ __global__ void __launch_bounds__(kRNT)
     for (int f = 0; f < kW; ++f) x[f0 + f] = tile[lane][f];
     wave_lds_order();
   }
-  for (int c0 = 0; c0 < k; c0 += kRF) {
-    const int m = min(kRF, k - c0);
+  // this block's centres (span: a multiple of kRF)
+  const int c1 = (int)min<int64_t>(k, (int64_t)(blockIdx.y + 1) * span);
+  for (int c0 = blockIdx.y * span; c0 < c1; c0 += kRF) {
+    const int m = min(kRF, c1 - c0);
     for (int c = 0; c < m; c += kRC) {
       const T *row = C + (int64_t)(c0 + c) * DB;
       T acc[kRC];
@@ -121,10 +123,20 @@ void launch_row_distances(int64_t n, int64_t d, int64_t k, const T *X, const T *
   hipLaunchKernelGGL(pad_centres_krn<T>, dim3((unsigned)ceil_div<int64_t>(total, kRNT)),
                      dim3(kRNT), 0, s, k, d, __builtin_ctz(DB), total, C, scratch);
   KMD_LAUNCH_CHECK();
+  // Few rows leave most of the chip idle while a lane goes through all centres: then
+  // the centres are split over blocks too, up to two blocks per CU in all (float64,
+  // d = 17, k = 200: n = 2000 193 -> 81 us, n = 30,000 200 -> 116; the two transposes
+  // and the feature-major kernel 168 and 180).
+  constexpr int64_t kRF = 128 / sizeof(T);
+  const int64_t tiles = ceil_div<int64_t>(k, kRF);
+  const int64_t want = std::max<int64_t>(
+      1, std::min<int64_t>(std::min<int64_t>(tiles, 65535), 2 * device_cu_count() / blocks));
+  const int64_t span = ceil_div<int64_t>(tiles, want) * kRF;
+  const dim3 grid((unsigned)blocks, (unsigned)ceil_div<int64_t>(k, span));
   auto run = [&](auto bucket) {
     if constexpr (sizeof(T) == 4 || bucket() <= 64)
-      hipLaunchKernelGGL((row_distances_krn<T, bucket()>), dim3((unsigned)blocks),
-                         dim3(kRNT), 0, s, n, (int)d, (int)k, X, (const T *)scratch, D);
+      hipLaunchKernelGGL((row_distances_krn<T, bucket()>), grid, dim3(kRNT), 0, s, n, (int)d,
+                         (int)k, (int)span, X, (const T *)scratch, D);
   };
   switch (DB) {
     case 8: run(std::integral_constant<int, 8>{}); break;

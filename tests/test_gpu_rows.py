@@ -68,3 +68,16 @@ def test_predict_equals_assignment(kd, torch_dev, n, d, k):
     kd.half_l2_norm_squared(to_dev(C.T), hn, 128, q())
     kd.assignment(to_dev(X.T), to_dev(C.T), hn, lab, 8, 128, q())[0].wait()
     assert_array_equal(to_np(got), to_np(lab))
+
+
+# several blocks of centres: one tile each, two each and a ragged last one
+@pytest.mark.parametrize("n,d,k,dt", [(100, 5, 1000, np.float32), (25_600, 9, 200, np.float32),
+                                      (30_001, 17, 201, np.float64), (65, 64, 17, np.float64)])
+def test_transform_with_centres_over_blocks(kd, torch_dev, n, d, k, dt):
+    rng = np.random.default_rng(n + k)
+    X = rng.standard_normal((n, d)).astype(dt)
+    C = rng.standard_normal((k, d)).astype(dt)
+    got = model_of(kd, C).transform(to_dev(X))
+    D = torch.empty((k, n), dtype=got.dtype, device=torch_dev)
+    kd.compute_centroid_to_sample_distances(to_dev(X.T), to_dev(C.T), D, 128, 32, q())[0].wait()
+    assert_array_equal(to_np(got), to_np(D).T)
