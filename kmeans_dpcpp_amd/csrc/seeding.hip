@@ -842,8 +842,7 @@ void launch_kmeans_plusplus(int64_t n, int64_t d, int64_t k, int trials,
   require(nb <= INT32_MAX, "too many samples");
   TempBuffer dbuf(2 * (size_t)n * sizeof(double), s);
   TempBuffer part((size_t)trials * (size_t)(nb + nsub) * sizeof(double), s);
-  TempBuffer small(512, s);
-  TempBuffer crow((size_t)(trials + 1) * (size_t)d * sizeof(double), s);
+  TempBuffer small(512 + (size_t)(trials + 1) * (size_t)d * sizeof(double), s);
   KppArgs a{};
   a.n = n; a.d = d; a.k = k; a.nb = nb; a.nsub = nsub; a.trials = trials;
   a.X_t = X_t; a.w = w; a.u = u_dev; a.centers_t = centers_t;
@@ -855,7 +854,7 @@ void launch_kmeans_plusplus(int64_t n, int64_t d, int64_t k, int trials,
   char *sm = small.as<char>();
   a.cand = reinterpret_cast<int64_t *>(sm);              // 16 x 8 bytes
   a.csq = reinterpret_cast<double *>(sm + 128);          // 17 x 8 bytes
-  a.crow = crow.as<double>();
+  a.crow = reinterpret_cast<double *>(sm + 512);
   KMD_HIP_CHECK(hipMemsetAsync(sm, 0, 512, s));
   hipLaunchKernelGGL(kpp_wsum_krn<T>, dim3((unsigned)nb), dim3(kSNT), 0, s, a);
   KMD_LAUNCH_CHECK();
