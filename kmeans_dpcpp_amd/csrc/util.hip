@@ -968,10 +968,10 @@ __global__ void __launch_bounds__(kBlock)
   if (f >= d) return;
   for (int64_t j = 0; j < m; ++j) {
     int64_t s = order[j];
-    if (s < 0 || s >= n) continue;
-    int64_t p = (int64_t)labels[s];
     int64_t e = (int64_t)empty_list[j];
-    if (p < 0 || p >= k || e < 0 || e >= k) continue;
+    const bool none = s < 0 || s >= n;
+    int64_t p = (int64_t)labels[none ? 0 : s];
+    if (none || p < 0 || p >= k || e < 0 || e >= k) continue;
     T ws = w[s];
     T add = X[f * n + s] * ws;
     C[f * k + p] -= add;
@@ -1204,13 +1204,16 @@ void launch_relocate(int64_t n, int64_t d, int64_t k, int64_t n_empty,
   const int64_t m = n_empty < n ? n_empty : n;
   if (m <= 0 || d <= 0) return;
   TempBuffer order(sizeof(int64_t) * m, s);
+  // (released behind the last launch: a release in front of it is a marker in the
+  // stream that the launch waits behind, 10 us)
+  TempBuffer thr(0, s), sel(0, s);
   if (n <= kFarN && m <= kFarM) {
     hipLaunchKernelGGL(far_order_krn<T>, dim3(1), dim3(kFarThreads), 0, s, (int)n, (int)m,
                        sq_dist, order.as<int64_t>());
     KMD_LAUNCH_CHECK();
   } else {
-    TempBuffer thr(sizeof(T), s);
-    TempBuffer sel(sizeof(I) * (n + 2), s);
+    thr = TempBuffer(sizeof(T), s);
+    sel = TempBuffer(sizeof(I) * (n + 2), s);
     I *n_gt = sel.as<I>() + n;
     I *n_eq = n_gt + 1;
     launch_far_threshold<T>(n, sq_dist, m, thr.as<T>(), s);
