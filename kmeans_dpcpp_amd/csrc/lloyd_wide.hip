@@ -426,7 +426,7 @@ bool label_sums_supported(int64_t k) {
 // sum here have to be cleared and flushed for the samples to pay for.  Steps of d
 // = 16 to 128, this against that one: k <= 1024 0.81 - 1.02 x at any n; n >= 8 k up
 // to the k whose rows stand two at a time in LDS 0.83 - 1.02 x; n = 2 k there 1.00 -
-// 1.04 x; one row at a time (n = 1M, d = 128, k = 10,000) 1497 us against 829.
+// 1.05 x; one row at a time (n = 1M, d = 128, k = 10,000) 1272 us against 780.
 bool label_sums_first(int64_t n, int64_t k) {
   return label_sums_supported(k) &&
          sum_lds(2, k, 0) <= kSumLds && (k <= 1024 || n >= 8 * k);
